@@ -1671,8 +1671,9 @@ extern "C" int lsh_lif_scan_bwd(const float* I, const float* u0, const float* U,
 }
 
 extern "C" int64_t lsh_lif_param_partials(int64_t T, int64_t N, int mode, int C) {
-  if (T < 0 || N < 0 || mode < 0 || mode > 3) return -1;
+  if (T < 0 || N < 0 || mode < 0 || mode > 4) return -1;
   const int64_t NB = (N + WAVE - 1) / WAVE;
+  if (mode == 4) return (T + 255) / 256 * NB;  // look-back of any T: one row per tile
   if (mode == 3) return T % 256 == 0 ? (T / 256) * NB : -1;  // look-back: one row per tile
   if (mode != 1) return NB;
   if (C < 1 || T % C != 0) return -1;
@@ -1690,10 +1691,11 @@ static int param_bwd(const float* I, const float* u0, const float* U, const floa
       bad_ptr(partials))
     return LSH_ERR_ARG;
   if (T < 0 || N < 0 || N > (int64_t)1 << 31) return LSH_ERR_SHAPE;
-  if (mode < 0 || mode > 3) return LSH_ERR_ARG;
+  if (mode < 0 || mode > 4) return LSH_ERR_ARG;
   hipStream_t st = (hipStream_t)stream;
   const float g = ur_or_gamma;
-  if (mode == 3)
+  if (mode == 3 && T % 256 != 0) return bad_ptr(ws) ? LSH_ERR_ARG : LSH_ERR_DIVISIBILITY;
+  if (mode >= 3)
     return lif_param_bwd_lookback(I, u0, U, S, GS, Lam, partials, ws, ws_bytes, T, N, beta, theta, g,
                                   alpha, PS, st);
   if (mode == 0) {

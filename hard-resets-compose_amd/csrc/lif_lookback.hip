@@ -41,13 +41,17 @@ void fill_i32_launch(int* p, int64_t n, int v, hipStream_t st) {
 // PS (detached, no GU): parameter sums in fp64, one partials row per workgroup (tile), as
 // k_lif_bwd_fused: PS == 1 the hard reset's (fit.py:43-47), PS == 2 the affine reset's
 // (triton_affine.py:229-242) with `u_r` carrying gamma.
-template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0>
+// RAG: T is no multiple of the segment W*C.  A step past T has a = b = 0: it leaves lam = 0 at the
+// end of time and adds nothing to the sums; its loads read the chunk's last row, its store is
+// left out.  Its own instantiation, since the tests cost the whole-segment kernel 2 % (N 1024,
+// T 2^18: 0.94 ms).
+template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0, bool RAG = false>
 __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
     const float* __restrict__ I, const float* __restrict__ u0, const float* __restrict__ U,
     const float* __restrict__ S, const float* __restrict__ GS, const float* __restrict__ GU,
     float* __restrict__ Lam, float* __restrict__ aggP, float* __restrict__ aggQ,
     float* __restrict__ incl, int* __restrict__ flags, WsHeader* hdr, double* __restrict__ partials,
-    int64_t N, int NB, int NSEG, float beta, float theta, float u_r, float alpha) {
+    int64_t T, int64_t N, int NB, int NSEG, float beta, float theta, float u_r, float alpha) {
   static_assert(!PS || (DETACH && !HAS_GU && C <= 64), "parameter sums: detached, no GU");
   constexpr bool AFF = PS == 2;
   __shared__ float sP[W][WAVE], sQ[W][WAVE];
@@ -68,6 +72,8 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
   const unsigned lb = ln * 4u, sb = lane * 4u;
   const unsigned rstride = (unsigned)(N * 4);
   const size_t row0 = ((size_t)seg * W + (W - 1 - w)) * C;  // wave 0 holds the latest chunk
+  // RAG: rows of this chunk (wave-uniform; <= 0 for a chunk past the end of the last segment)
+  const int rows = !RAG || (int64_t)row0 + C <= T ? C : (int)(T - (int64_t)row0);
   const float u0n = u0[nb0 + ln];
 
   // 1. coefficients of the chunk and its map
@@ -77,29 +83,39 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
   unsigned long long sbits = 0;
   const float gbeta = beta * u_r;  // AFF: beta*gamma
   double acc_b = 0.0, acc_t = 0.0, acc_r = 0.0;
-  {
+  if (!RAG || rows > 0) {
     const Buf bi(I + nb0 + row0 * N), bs(S + nb0 + row0 * N), bg(GS + nb0 + row0 * N);
     const Buf bp(U + nb0 + row0 * N);
     const float up0 = row0 > 0 ? ld_row(U + nb0 + (row0 - 1) * N, lb) : u0n;
 #pragma unroll
     for (int j = 0; j < C; ++j) {
-      const unsigned so = j * rstride;
+      const bool in = !RAG || j < rows;
+      const unsigned so = (in ? j : rows - 1) * rstride;  // steps past T read the last row
       const float x = bi.ld(lb, so);
       const float s = bs.ld(lb, so);
       const float gs = bg.ld(lb, so);
-      const float up = j == 0 ? up0 : bp.ld(lb, so - rstride);
+      const float up = j == 0 ? up0 : bp.ld(lb, in ? so - rstride : so);
       const float v = lif_v(up, x, beta);
       const float sg = surrogate(v, theta, alpha);
       float J = 1.0f - s;
       if (!DETACH) J = J + (u_r - v) * sg;
-      if constexpr (!AFF) a[j] = beta * J;
+      if constexpr (!AFF) a[j] = in ? beta * J : 0.0f;
       b[j] = HAS_GU ? gs * sg + J * Buf(GU + nb0 + row0 * N).ld(lb, so) : gs * sg;
+      if (!in) b[j] = 0.0f;
       if (PS) {
         upk[j] = up;
-        if (s != 0.0f) sbits |= 1ull << j;
+        if (s != 0.0f && in) sbits |= 1ull << j;
         if (PS == 1 && valid) acc_t += (double)b[j];
         if constexpr (AFF) vpk[j] = v;
       }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      if constexpr (!AFF) a[j] = 0.0f;
+      b[j] = 0.0f;
+      if (PS) upk[j] = 0.0f;
+      if constexpr (AFF) vpk[j] = 0.0f;
     }
   }
   float P = 1.0f, Q = 0.0f;
@@ -162,7 +178,7 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
       lam = b[j] + (((sbits >> j) & 1ull) ? gbeta : beta) * lam;
     else
       lam = b[j] + a[j] * lam;
-    if (valid) {
+    if (valid && (!RAG || j < rows)) {
       bl.st_nt(sb, j * rstride, lam);
       if (PS) {
         acc_b += (double)lam * (double)upk[j];
@@ -201,12 +217,23 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
   }
 }
 
+// Segment = 256 steps: 16 waves of 16 steps (C = 16) or 8 waves of 32 steps (C = 32).  The last
+// segment of a T that is no multiple of it is short: its steps past T are neutral.
+constexpr int kLookbackSeg = 256;
+static int64_t lookback_segments(int64_t T) { return (T + kLookbackSeg - 1) / kLookbackSeg; }
+
+static size_t lookback_ws(int64_t T, int64_t N) {
+  const size_t NSEG = (size_t)lookback_segments(T), NB = (size_t)((N + WAVE - 1) / WAVE);
+  return kWsHeaderBytes + 3 * align_up(NSEG * (size_t)N * 4, 256) + align_up(NSEG * NB * 4, 256);
+}
+
 template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0>
 static void launch_lookback(const float* I, const float* u0, const float* U, const float* S,
-                            const float* GS, const float* GU, float* Lam, char* ws, int64_t N,
-                            int NSEG, float beta, float theta, float u_r, float alpha,
+                            const float* GS, const float* GU, float* Lam, char* ws, int64_t T,
+                            int64_t N, float beta, float theta, float u_r, float alpha,
                             hipStream_t st, double* partials = nullptr) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
+  const int NSEG = (int)lookback_segments(T);
   const size_t sn = align_up((size_t)NSEG * (size_t)N * 4, 256);
   float* aggP = reinterpret_cast<float*>(ws + kWsHeaderBytes);
   float* aggQ = reinterpret_cast<float*>(ws + kWsHeaderBytes + sn);
@@ -216,47 +243,68 @@ static void launch_lookback(const float* I, const float* u0, const float* U, con
   hipLaunchKernelGGL(k_ws_header_reset, dim3(1), dim3(64), 0, st, reinterpret_cast<WsHeader*>(ws));
   hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)((nflags + WAVE - 1) / WAVE)), dim3(WAVE), 0, st,
                      flags, nflags, 0);
-  hipLaunchKernelGGL((k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS>), dim3((unsigned)nflags),
-                     dim3(WAVE * W), 0, st, I, u0, U, S, GS, GU, Lam, aggP, aggQ, incl, flags,
-                     reinterpret_cast<WsHeader*>(ws), partials, N, NB, NSEG, beta, theta, u_r,
-                     alpha);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nflags), dim3(WAVE * W), 0, st, I, u0, U, S, GS, GU, Lam,
+                       aggP, aggQ, incl, flags, reinterpret_cast<WsHeader*>(ws), partials, T, N, NB,
+                       NSEG, beta, theta, u_r, alpha);
+  };
+  if (T % kLookbackSeg == 0)
+    launch(k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS, false>);
+  else
+    launch(k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS, true>);
 }
 
 template <int C, int W>
 static void lookback_cw(const float* I, const float* u0, const float* U, const float* S,
-                        const float* GS, const float* GU, float* Lam, char* ws, int64_t N, int NSEG,
+                        const float* GS, const float* GU, float* Lam, char* ws, int64_t T, int64_t N,
                         float beta, float theta, float u_r, float alpha, bool detach,
                         hipStream_t st) {
   if (detach) {
     if (GU)
-      launch_lookback<C, W, true, true>(I, u0, U, S, GS, GU, Lam, ws, N, NSEG, beta, theta, u_r,
+      launch_lookback<C, W, true, true>(I, u0, U, S, GS, GU, Lam, ws, T, N, beta, theta, u_r,
                                         alpha, st);
     else
-      launch_lookback<C, W, true, false>(I, u0, U, S, GS, GU, Lam, ws, N, NSEG, beta, theta, u_r,
+      launch_lookback<C, W, true, false>(I, u0, U, S, GS, GU, Lam, ws, T, N, beta, theta, u_r,
                                          alpha, st);
   } else {
     if (GU)
-      launch_lookback<C, W, false, true>(I, u0, U, S, GS, GU, Lam, ws, N, NSEG, beta, theta, u_r,
+      launch_lookback<C, W, false, true>(I, u0, U, S, GS, GU, Lam, ws, T, N, beta, theta, u_r,
                                          alpha, st);
     else
-      launch_lookback<C, W, false, false>(I, u0, U, S, GS, GU, Lam, ws, N, NSEG, beta, theta, u_r,
+      launch_lookback<C, W, false, false>(I, u0, U, S, GS, GU, Lam, ws, T, N, beta, theta, u_r,
                                           alpha, st);
   }
+}
+
+// The look-back adjoint for any T (arguments already known not to be NULL).
+static int lookback_run(const float* I, const float* u0, const float* U, const float* S,
+                        const float* GS, const float* GU, float* Lam, int64_t T, int64_t N,
+                        float beta, float theta, float u_r, float alpha, int detach, int C, void* ws,
+                        size_t ws_bytes, void* stream) {
+  if (T < 0 || N < 0 || N > (int64_t)1 << 31) return LSH_ERR_SHAPE;
+  if (C != 16 && C != 32) return LSH_ERR_SHAPE;
+  if ((uint64_t)N * (uint64_t)C * 4u >= ((uint64_t)1 << 32)) return LSH_ERR_SHAPE;
+  if (ws_bytes < lookback_ws(T, N) || (reinterpret_cast<uintptr_t>(ws) & 255u) != 0)
+    return LSH_ERR_WORKSPACE;
+  if (lookback_segments(T) * ((N + WAVE - 1) / WAVE) > ((int64_t)1 << 31) - 1) return LSH_ERR_SHAPE;
+  if (T == 0 || N == 0) return LSH_OK;
+  hipStream_t st = (hipStream_t)stream;
+  char* w = static_cast<char*>(ws);
+  if (C == 16)
+    lookback_cw<16, 16>(I, u0, U, S, GS, GU, Lam, w, T, N, beta, theta, u_r, alpha, detach != 0, st);
+  else
+    lookback_cw<32, 8>(I, u0, U, S, GS, GU, Lam, w, T, N, beta, theta, u_r, alpha, detach != 0, st);
+  LSH_CHECK_LAUNCH();
+  return LSH_OK;
 }
 
 }  // namespace lsh
 
 using namespace lsh;
 
-// Segment = 256 steps: 16 waves of 16 steps (C = 16) or 8 waves of 32 steps (C = 32).
-static constexpr int kLookbackSeg = 256;
-
 extern "C" size_t lsh_lif_scan_lookback_bwd_workspace(int64_t T, int64_t N) {
   if (T < 0 || N < 0 || T % kLookbackSeg != 0) return 0;
-  const int64_t NSEG = T / kLookbackSeg;
-  const int64_t NB = (N + WAVE - 1) / WAVE;
-  const size_t sn = align_up((size_t)NSEG * (size_t)N * 4, 256);
-  return kWsHeaderBytes + 3 * sn + align_up((size_t)NSEG * (size_t)NB * 4, 256);
+  return lookback_ws(T, N);
 }
 
 extern "C" int lsh_lif_scan_lookback_bwd(const float* I, const float* u0, const float* U,
@@ -270,24 +318,24 @@ extern "C" int lsh_lif_scan_lookback_bwd(const float* I, const float* u0, const 
   if (T < 0 || N < 0 || N > (int64_t)1 << 31) return LSH_ERR_SHAPE;
   if (C != 16 && C != 32) return LSH_ERR_SHAPE;
   if (T % kLookbackSeg != 0) return LSH_ERR_DIVISIBILITY;
-  if ((uint64_t)N * (uint64_t)C * 4u >= ((uint64_t)1 << 32)) return LSH_ERR_SHAPE;
-  if (ws_bytes < lsh_lif_scan_lookback_bwd_workspace(T, N) ||
-      (reinterpret_cast<uintptr_t>(ws) & 255u) != 0)
-    return LSH_ERR_WORKSPACE;
-  const int64_t NSEG = T / kLookbackSeg;
-  const int64_t NB = (N + WAVE - 1) / WAVE;
-  if (NSEG * NB > ((int64_t)1 << 31) - 1) return LSH_ERR_SHAPE;
-  if (T == 0 || N == 0) return LSH_OK;
-  hipStream_t st = (hipStream_t)stream;
-  char* w = static_cast<char*>(ws);
-  if (C == 16)
-    lookback_cw<16, 16>(I, u0, U, S, GS, GU, Lam, w, N, (int)NSEG, beta, theta, u_r, alpha,
-                        detach != 0, st);
-  else
-    lookback_cw<32, 8>(I, u0, U, S, GS, GU, Lam, w, N, (int)NSEG, beta, theta, u_r, alpha,
-                       detach != 0, st);
-  LSH_CHECK_LAUNCH();
-  return LSH_OK;
+  return lookback_run(I, u0, U, S, GS, GU, Lam, T, N, beta, theta, u_r, alpha, detach, C, ws,
+                      ws_bytes, stream);
+}
+
+extern "C" size_t lsh_lif_scan_lookback_any_bwd_workspace(int64_t T, int64_t N) {
+  return T < 0 || N < 0 ? 0 : lookback_ws(T, N);
+}
+
+extern "C" int lsh_lif_scan_lookback_any_bwd(const float* I, const float* u0, const float* U,
+                                             const float* S, const float* GS, const float* GU,
+                                             float* Lam, int64_t T, int64_t N, float beta,
+                                             float theta, float u_r, float alpha, int detach, int C,
+                                             void* ws, size_t ws_bytes, void* stream) {
+  if (bad_ptr(I) || bad_ptr(u0) || bad_ptr(U) || bad_ptr(S) || bad_ptr(GS) || bad_ptr(Lam) ||
+      bad_ptr(ws))
+    return LSH_ERR_ARG;
+  return lookback_run(I, u0, U, S, GS, GU, Lam, T, N, beta, theta, u_r, alpha, detach, C, ws,
+                      ws_bytes, stream);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -339,19 +387,17 @@ int lsh::lif_param_bwd_lookback(const float* I, const float* u0, const float* U,
                                 float u_r, float alpha, int ps, hipStream_t st) {
   if (bad_ptr(ws)) return LSH_ERR_ARG;
   if (T < 0 || N < 0 || N > (int64_t)1 << 31) return LSH_ERR_SHAPE;
-  if (T % kLookbackSeg != 0) return LSH_ERR_DIVISIBILITY;
-  if (ws_bytes < lsh_lif_scan_lookback_bwd_workspace(T, N) ||
-      (reinterpret_cast<uintptr_t>(ws) & 255u) != 0)
+  if ((uint64_t)N * 16u * 4u >= ((uint64_t)1 << 32)) return LSH_ERR_SHAPE;
+  if (ws_bytes < lookback_ws(T, N) || (reinterpret_cast<uintptr_t>(ws) & 255u) != 0)
     return LSH_ERR_WORKSPACE;
-  const int64_t NSEG = T / kLookbackSeg;
-  if (NSEG * ((N + WAVE - 1) / WAVE) > ((int64_t)1 << 31) - 1) return LSH_ERR_SHAPE;
+  if (lookback_segments(T) * ((N + WAVE - 1) / WAVE) > ((int64_t)1 << 31) - 1) return LSH_ERR_SHAPE;
   if (T == 0 || N == 0) return LSH_OK;
   if (ps == 2)
-    launch_lookback<16, 16, true, false, 2>(I, u0, U, S, GS, nullptr, Lam, static_cast<char*>(ws), N,
-                                            (int)NSEG, beta, theta, u_r, alpha, st, partials);
+    launch_lookback<16, 16, true, false, 2>(I, u0, U, S, GS, nullptr, Lam, static_cast<char*>(ws), T, N,
+                                            beta, theta, u_r, alpha, st, partials);
   else
-    launch_lookback<16, 16, true, false, 1>(I, u0, U, S, GS, nullptr, Lam, static_cast<char*>(ws), N,
-                                            (int)NSEG, beta, theta, u_r, alpha, st, partials);
+    launch_lookback<16, 16, true, false, 1>(I, u0, U, S, GS, nullptr, Lam, static_cast<char*>(ws), T, N,
+                                            beta, theta, u_r, alpha, st, partials);
   LSH_CHECK_LAUNCH();
   return LSH_OK;
 }

@@ -129,6 +129,9 @@ SIGNATURES = {
     "lsh_lif_scan_lookback_bwd_workspace": (c_sz, [c_i64, c_i64]),
     "lsh_lif_scan_lookback_bwd": (c_i, [c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_i64, c_i64, c_f, c_f, c_f,
                                         c_f, c_i, c_i, c_p, c_sz, c_p]),
+    "lsh_lif_scan_lookback_any_bwd_workspace": (c_sz, [c_i64, c_i64]),
+    "lsh_lif_scan_lookback_any_bwd": (c_i, [c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_i64, c_i64, c_f, c_f,
+                                            c_f, c_f, c_i, c_i, c_p, c_sz, c_p]),
     "lsh_lif_scan_lookback_bwd_noalloc": (c_i, [c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_i64, c_i64, c_f,
                                                 c_f, c_f, c_f, c_i, c_i, c_p]),
     "lsh_lif_param_bwd": (c_i, [c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_i64, c_i64, c_f, c_f, c_f, c_f,

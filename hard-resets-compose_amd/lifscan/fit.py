@@ -33,6 +33,10 @@ def _param_backward(I, u0, U, S, GS, beta, theta, u_r, alpha, mode):
             code, C = 3, 16
         else:
             code, C = 1, L.chunked_bwd_C(T, N, min(128, L._pick_C(T, D=2)))
+            if L.lookback_any(N):
+                code, C = 4, 16
+    elif mode == "lookback":
+        code, C = 4, 16
     else:
         code, C = 0, 1
     P = lib.lsh_lif_param_partials(T, N, code, C)
@@ -44,8 +48,8 @@ def _param_backward(I, u0, U, S, GS, beta, theta, u_r, alpha, mode):
     if code == 1:
         nbytes = lib.lsh_lif_scan_bwd_workspace(T, N, C)
         ws = _n.workspace(nbytes, I.device)
-    elif code == 3:
-        nbytes = lib.lsh_lif_scan_lookback_bwd_workspace(T, N)
+    elif code >= 3:
+        nbytes = lib.lsh_lif_scan_lookback_any_bwd_workspace(T, N)
         ws = _n.workspace(nbytes, I.device)
     with _n.on_device(I):
         _n.check(lib.lsh_lif_param_bwd(
@@ -103,6 +107,7 @@ def lif_param(I, u0, beta, theta, u_r, alpha=4.0, mode="auto", K=16):
     T, N = I.shape
     if mode == "auto":
         fwd, bwd = L.auto_modes(N, T)
+        bwd = L._auto_bwd(bwd, N, T)
     else:
         fwd = bwd = mode
     return LIFParamFn.apply(I, u0, beta, theta, u_r, alpha, fwd, bwd, K)

@@ -129,14 +129,17 @@ def _aff_backward(I, u0, U, S, GS, beta, theta, gamma, alpha, mode="auto", C=Non
             mode = "fused"
         elif L.LOOKBACK_BWD and T % L.LOOKBACK_SEG == 0:
             mode = "lookback"
-        elif T >= L.AUTO_BWD_MIN_T:
-            mode = "chunked"
         else:
-            mode = "serial"
+            if T >= L.AUTO_BWD_MIN_T:
+                L._pick_C(T, D=2)  # a long T without a chunk is refused, as ever
+            mode = "lookback_any" if L.lookback_any(N) else (
+                "chunked" if T >= L.AUTO_BWD_MIN_T else "serial")
     if mode == "fused":
         code, C = 2, int(C or L.FUSED_BWD_C)
     elif mode == "lookback":
         code, C = 3, 16
+    elif mode == "lookback_any":
+        code, C = 4, 16
     elif mode == "chunked":
         code, C = 1, int(C or L.chunked_bwd_C(T, N, min(128, L._pick_C(T, D=2))))
     elif mode == "serial":
@@ -153,8 +156,8 @@ def _aff_backward(I, u0, U, S, GS, beta, theta, gamma, alpha, mode="auto", C=Non
     if code == 1:
         nbytes = lib.lsh_lif_scan_bwd_workspace(T, N, C)
         ws = _n.workspace(nbytes, I.device)
-    elif code == 3:
-        nbytes = lib.lsh_lif_scan_lookback_bwd_workspace(T, N)
+    elif code >= 3:
+        nbytes = lib.lsh_lif_scan_lookback_any_bwd_workspace(T, N)
         ws = _n.workspace(nbytes, I.device)
     with _n.on_device(I):
         _n.check(lib.lsh_aff_bwd(

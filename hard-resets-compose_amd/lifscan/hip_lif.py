@@ -910,23 +910,31 @@ _LAST_LOOKBACK = None
 def scan_backward_lookback(I, u0, U, S, GS, GU, beta, theta, u_r, alpha=4.0, detach=True, C=16):
     """Single-pass affine-scan adjoint with a decoupled look-back across workgroups -> Lam
     (for few neurons; T % 256 == 0; C in {16, 32} steps per wave)."""
+    I = _input(I)
+    if I.shape[0] % LOOKBACK_SEG:
+        raise ValueError(f"look-back adjoint needs T % {LOOKBACK_SEG} == 0 (T={I.shape[0]})")
+    return _lookback(I, u0, U, S, GS, GU, beta, theta, u_r, alpha, detach, C)
+
+
+def _lookback(I, u0, U, S, GS, GU, beta, theta, u_r, alpha, detach, C=16):
+    """The look-back adjoint for every T (its last segment may be short) -> Lam."""
     global _LAST_LOOKBACK
     I = _input(I)
     T, N = I.shape
     u0 = _vec(u0, N, I)
     U, S, GS = _same(U, I, "U"), _same(S, I, "S"), _same(GS, I, "GS")
     GU = _same(GU, I, "GU")
-    L = _n.lib()
-    nbytes = L.lsh_lif_scan_lookback_bwd_workspace(T, N)
-    if nbytes == 0:
-        raise ValueError(f"look-back adjoint needs T % {LOOKBACK_SEG} == 0 (T={T})")
-    ws = _n.workspace(nbytes, I.device)
     Lam = torch.empty_like(I)
+    if T == 0 or N == 0:
+        return Lam
+    L = _n.lib()
+    nbytes = L.lsh_lif_scan_lookback_any_bwd_workspace(T, N)
+    ws = _n.workspace(nbytes, I.device)
     with _n.on_device(I):
-        _n.check(L.lsh_lif_scan_lookback_bwd(
+        _n.check(L.lsh_lif_scan_lookback_any_bwd(
             _n.ptr(I), _n.ptr(u0), _n.ptr(U), _n.ptr(S), _n.ptr(GS), _n.ptr(GU), _n.ptr(Lam), T, N,
             _f32(beta), _f32(theta), _f32(u_r), _f32(alpha), int(bool(detach)), int(C), _n.ptr(ws),
-            nbytes, _n.stream_of(I)), "lsh_lif_scan_lookback_bwd")
+            nbytes, _n.stream_of(I)), "lsh_lif_scan_lookback_any_bwd")
     _LAST_LOOKBACK = ws
     return Lam
 
@@ -942,19 +950,29 @@ def scan_backward_tiled(I, u0, U, S, GS, GU, beta, theta, u_r, alpha=4.0, detach
                         BNr=32, D=4, nwr=1):
     """Affine-scan adjoint (triton_lif.py:512-526) -> Lam.  GU may be None (zeros).
     Runs the single-pass kernel when there are enough neurons to fill the chip and T is a
-    multiple of its internal chunk, else the three-kernel chunk scan (chunk from
-    chunked_bwd_C; the given C when none fits)."""
+    multiple of its internal chunk, else the look-back pass.  T must have a chunk either way
+    (chunked_bwd_C, or the given C: ValueError)."""
     I = _input(I)
     T, N = I.shape
     if N >= FUSED_BWD_MIN_N and T % FUSED_BWD_C == 0:
         return scan_backward_fused(I, u0, U, S, GS, GU, beta, theta, u_r, alpha, detach)
-    if LOOKBACK_BWD and T % LOOKBACK_SEG == 0:
-        return scan_backward_lookback(I, u0, U, S, GS, GU, beta, theta, u_r, alpha, detach)
-    return scan_backward_chunked(I, u0, U, S, GS, GU, beta, theta, u_r, alpha, detach,
-                                 chunked_bwd_C(T, N, C))
+    C = chunked_bwd_C(T, N, C)
+    if lookback_any(N) and C >= 1 and T % C == 0:
+        return _lookback(I, u0, U, S, GS, GU, beta, theta, u_r, alpha, detach)
+    return scan_backward_chunked(I, u0, U, S, GS, GU, beta, theta, u_r, alpha, detach, C)
 
 
 LOOKBACK_BWD = True
+
+
+# The look-back adjoint takes every T (a short last segment), so the three-kernel chunk scan,
+# which reads its inputs twice and walks T/C chunks one after another, is left only for more
+# neurons than the look-back kernel's 32-bit row offsets reach.  Measured on MI355X, chunked ->
+# look-back: N = 64, T = 50000 (chunk 16; with parameter sums) 0.85 -> 0.04 ms; N = 160, T =
+# 235584 1.49 -> 0.15 ms; N = 1488, T = 41088 0.56 -> 0.26 ms.
+def lookback_any(N):
+    """True when the adjoint of a T that is no multiple of the segment takes the look-back pass."""
+    return LOOKBACK_BWD and N * 16 * 4 < 1 << 32
 
 
 def scan_backward_chunked(I, u0, U, S, GS, GU, beta, theta, u_r, alpha=4.0, detach=True, C=64):
@@ -1029,6 +1047,21 @@ def auto_modes(N, T):
     if bwd == "scan" and _chunk_or_none(T, 2) is None:
         bwd = "serial"
     return fwd, bwd
+
+
+# Up to this many neurons lif_auto's adjoint of a long T that has no chunk (auto_modes: serial) is
+# the look-back pass, serial -> look-back: N = 64, T = 4001 94 -> 19 us; N = 1024, T = 2001 50 -> 19
+# us; N = 8192, T = 4001 166 -> 119 us.  Above, the serial sweep fills the chip as well (N = 14083,
+# T = 2001: 130 against 151 us; rows of odd N are not aligned, which costs both).
+AUTO_LOOKBACK_MAX_N = 8192
+
+
+def _auto_bwd(bwd, N, T):
+    """auto_modes' adjoint mode, or "lookback" for few neurons where only the chunk policy kept a
+    long T serial: the look-back pass needs no chunk."""
+    if bwd == "serial" and LOOKBACK_BWD and N <= AUTO_LOOKBACK_MAX_N and T >= AUTO_BWD_MIN_T:
+        return "lookback"
+    return bwd
 
 
 # ----------------------------------------------------------------------------- autograd layers
@@ -1197,6 +1230,8 @@ class LIFAuto(torch.autograd.Function):
         I, u0, U, S = ctx.saved_tensors
         if bwd_mode == "scan":
             Lam = scan_backward_auto(I, u0, U, S, gS, None, b, theta, u_r, alpha)
+        elif bwd_mode == "lookback":
+            Lam = _lookback(I, u0, U, S, gS, None, b, theta, u_r, alpha, True)
         else:
             Lam = serial_backward_auto(I, u0, U, S, gS, None, b, theta, u_r, alpha)
         du0 = b * Lam[0] if ctx.needs_input_grad[1] else None
@@ -1206,6 +1241,7 @@ class LIFAuto(torch.autograd.Function):
 
 def lif_auto(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, K=16, repair=0):
     fwd, bwd = auto_modes(I.shape[1], I.shape[0])
+    bwd = _auto_bwd(bwd, I.shape[1], I.shape[0])
     if fwd == bwd:  # one mode for both passes: lif_tuned's path (the same kernels and bits)
         return lif_tuned(I, u0, beta, theta, u_r, alpha, mode=fwd, K=K, repair=repair)
     return LIFAuto.apply(I, u0, beta, theta, u_r, alpha, K, repair, fwd, bwd)

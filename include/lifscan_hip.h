@@ -329,6 +329,14 @@ int lsh_lif_scan_lookback_bwd(const float* I, const float* u0, const float* U, c
                               float beta, float theta, float u_r, float alpha, int detach, int C,
                               void* ws, size_t ws_bytes, void* stream);
 
+/* lsh_lif_scan_lookback_bwd for every T: the last segment may be short (its steps past T are
+ * neutral).  Where T % 256 == 0 the same launch and the same bits; its own workspace query. */
+size_t lsh_lif_scan_lookback_any_bwd_workspace(int64_t T, int64_t N);
+int lsh_lif_scan_lookback_any_bwd(const float* I, const float* u0, const float* U, const float* S,
+                                  const float* GS, const float* GU, float* Lam, int64_t T,
+                                  int64_t N, float beta, float theta, float u_r, float alpha,
+                                  int detach, int C, void* ws, size_t ws_bytes, void* stream);
+
 /* lsh_lif_scan_lookback_bwd with no workspace argument, for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * No counterpart in the reference.  Its workspace is a static device array of
@@ -354,7 +362,8 @@ int lsh_lif_scan_lookback_bwd_noalloc(const float* I, const float* u0, const flo
  * partials[P][3] (fp64) = (sum lam_t*u_{t-1}, sum gs_t*sg_t, sum s_t*lam_{t+1}), whose column
  * sums give dbeta, -dtheta and dL/du_r / beta.  mode 0: serial; 1: chunked scan of chunk C
  * (workspace lsh_lif_scan_bwd_workspace(T, N, C)); 2: single pass, C in {16, 32, 64};
- * 3: look-back (T % 256 == 0, workspace lsh_lif_scan_lookback_bwd_workspace(T, N)).
+ * 3: look-back (T % 256 == 0, workspace lsh_lif_scan_lookback_bwd_workspace(T, N)); 4: look-back
+ * for every T (workspace lsh_lif_scan_lookback_any_bwd_workspace(T, N)).
  * P = lsh_lif_param_partials(T, N, mode, C). */
 int64_t lsh_lif_param_partials(int64_t T, int64_t N, int mode, int C);
 int lsh_lif_param_bwd(const float* I, const float* u0, const float* U, const float* S,

@@ -1,0 +1,73 @@
+"""GPU: lengths that are no multiple of a kernel's tile, against the fp64 adjoint of the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import lif_oracle as O
+from tests._inputs import gpu, host, normal, uniform
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+    return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30))
+
+
+# one short segment; one step past a segment; a chunk and a wave past one; one step short of two
+@pytest.mark.parametrize("T", [1, 17, 255, 257, 290, 511, 2081])
+@pytest.mark.parametrize("N,detach,with_gu", [(1, True, False), (70, True, True), (130, False, True)])
+def test_lookback_any_length(dev, T, N, detach, with_gu):
+    """_lookback at every kind of last segment; the rows behind the inputs' last one are NaN, so a
+    step past T that was read and used would show."""
+    from lifscan import hip_lif as L
+    I, GS = normal(T, N, 0.15, 0.4, T), normal(T, N, 0.0, 1.0, T + 1)
+    GU = normal(T, N, 0.0, 0.3, T + 2) if with_gu else None
+    u0 = uniform(N, 0.0, 1.0, 3)
+    U, S = O.serial_forward(I, 0.95, 1.0, -0.1, u0)
+    want = O.serial_backward(I, u0, U, S, GS, GU, 0.95, 1.0, -0.1, 4.0, detach, dtype=np.float64)
+    pad = lambda a: torch.cat([gpu(a, dev), torch.full((300, N), float("nan"), device=dev)])[:T]
+    args = [pad(I), gpu(u0, dev), pad(U), pad(S), pad(GS)]
+    print(f"lookback any T={T} N={N}", flush=True)
+    for C in (16, 32):
+        Lam = L._lookback(*args, None if GU is None else pad(GU), 0.95, 1.0, -0.1, 4.0, detach, C=C)
+        assert L.last_lookback_timeouts() == 0
+        assert rel(host(Lam), want) < 1e-6  # fp32 recurrence: about 1e-7 of the fp64 one
+
+
+@pytest.mark.parametrize("T,N", [(300, 65), (1001, 40), (2050, 130)])
+def test_lookback_any_parameter_sums(dev, T, N):
+    """lsh_lif_param_bwd and lsh_aff_bwd mode 4: Lam and the fp64 sums at ragged T."""
+    from lifscan import fit
+    from lifscan import hip_affine as AF
+    beta, theta, u_r, gamma, delta = 0.93, 1.0, -0.1, 0.5, -0.25
+    I, GS = normal(T, N, 0.08, 0.5, 7), normal(T, N, 0.0, 1.0, 8)
+    u0 = uniform(N, 0.0, 1.0, 9)
+    U, S = O.serial_forward(I, beta, theta, u_r, u0)
+    Lam = O.serial_backward(I, u0, U, S, GS, None, beta, theta, u_r, 4.0, True, dtype=np.float64)
+    want = O.param_grads(I, u0, U, S, GS, Lam, beta, theta, u_r, 4.0)
+    print(f"param lookback any T={T} N={N}", flush=True)
+    got, sums = fit._param_backward(*[gpu(a, dev) for a in (I, u0, U, S, GS)], beta, theta, u_r, 4.0,
+                                    "lookback")
+    assert rel(host(got), Lam) < 1e-6
+    for k, g in enumerate((sums[0], -sums[1], beta * sums[2])):
+        assert rel(g.item(), want[2 + k]) < 1e-4, k
+    U, S = AF.aff_serial_forward(gpu(I, dev), beta, theta, gamma, delta, gpu(u0, dev))
+    a = [gpu(I, dev), gpu(u0, dev), U, S, gpu(GS, dev), beta, theta, gamma, 4.0]
+    l1, s1 = AF._aff_backward(*a, mode="lookback_any")
+    l2, s2 = AF._aff_backward(*a, mode="serial")
+    assert rel(host(l1), host(l2)) < 1e-6
+    assert torch.allclose(s1, s2, rtol=1e-5, atol=1e-5 * float(s2.abs().max()))
+
+
+def test_long_lengths_without_a_chunk_are_still_refused(dev):
+    from lifscan import hip_affine as AF
+    from lifscan import hip_lif as L
+    z = lambda T, N=3: torch.zeros(T, N, device=dev)
+    u0 = torch.zeros(3, device=dev)
+    with pytest.raises(ValueError):
+        L.scan_backward_tiled(z(1000), u0, z(1000), z(1000), z(1000), None, 0.9, 1.0, 0.0, C=64)
+    with pytest.raises(ValueError):
+        L.scan_backward_lookback(z(1000), u0, z(1000), z(1000), z(1000), None, 0.9, 1.0, 0.0)
+    with pytest.raises(ValueError):
+        AF._aff_backward(z(2049), u0, z(2049), z(2049), z(2049), 0.9, 1.0, 0.5, 4.0)
