@@ -33,15 +33,16 @@
 namespace lsh {
 
 // Rows per register tile of the warm-up and of the replay (loads of the next tile in flight
-// while the current one is computed).
+// while the current one is computed).  32 and 64 rows measured the same from N = 64 to 8192.
 constexpr int WARM_D = 16;
 
+// T need not be a multiple of C: the last chunk is short.
 __global__ __launch_bounds__(64) void k_lif_fwd_warm(const float* __restrict__ I,
                                                      const float* __restrict__ u0,
                                                      float* __restrict__ U, float* __restrict__ S,
                                                      float* __restrict__ starts,
-                                                     float* __restrict__ ends, int64_t N, int C,
-                                                     int W, int NB, float beta, float theta,
+                                                     float* __restrict__ ends, int64_t T, int64_t N,
+                                                     int C, int W, int NB, float beta, float theta,
                                                      float u_r) {
   const int64_t m = blockIdx.x / NB;
   const int nb = (int)(blockIdx.x - m * NB);
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(64) void k_lif_fwd_warm(const float* __restrict__ I
   const float* __restrict__ Ip = I + base;
   float* __restrict__ Up = U + base;
   float* __restrict__ Sp = S + base;
-  stream_rows<WARM_D>(Ip, (size_t)N, C, [&](int64_t j, float x) {
+  stream_rows<WARM_D>(Ip, (size_t)N, min<int64_t>(C, T - t0), [&](int64_t j, float x) {
     bool s;
     u = lif_step(u, x, beta, theta, u_r, s);
     st_nt(Up + (size_t)j * N, u);
@@ -95,8 +96,9 @@ __global__ __launch_bounds__(64) void k_lif_repair_wide(const float* __restrict_
                                                         float* __restrict__ U,
                                                         float* __restrict__ S,
                                                         float* __restrict__ starts,
-                                                        float* ends, int64_t N, int C, int NB,
-                                                        float beta, float theta, float u_r) {
+                                                        float* ends, int64_t T, int64_t N, int C,
+                                                        int NB, float beta, float theta,
+                                                        float u_r) {
   const int64_t m = blockIdx.x / NB + 1;
   const int nb = (int)(blockIdx.x % NB);
   const int64_t n = (int64_t)nb * WAVE + threadIdx.x;
@@ -107,7 +109,8 @@ __global__ __launch_bounds__(64) void k_lif_repair_wide(const float* __restrict_
   float u = prev;
   const size_t base = (size_t)m * C * N + n;
   const bool met = stream_rows_until<16>(
-      I + base, U + base, (size_t)N, C, [&](int64_t j, float x, float u_old) {
+      I + base, U + base, (size_t)N, min<int64_t>(C, T - m * C),
+      [&](int64_t j, float x, float u_old) {
         bool s;
         u = lif_step(u, x, beta, theta, u_r, s);
         U[base + (size_t)j * N] = u;
@@ -119,9 +122,8 @@ __global__ __launch_bounds__(64) void k_lif_repair_wide(const float* __restrict_
 
 static int warm_check(int64_t T, int64_t N, int C, int W) {
   if (T < 0 || N < 0 || N > ((int64_t)1 << 31) || C < 1 || W < 0) return LSH_ERR_SHAPE;
-  if (T % C != 0) return LSH_ERR_DIVISIBILITY;
-  if ((T / C) * ((N + WAVE - 1) / WAVE) > ((int64_t)1 << 31) - 1) return LSH_ERR_SHAPE;
-  if ((T / C) * ((N + WAVE - 1) / WAVE) * WAVE > ((int64_t)1 << 31) - 1) return LSH_ERR_SHAPE;
+  const int64_t waves = (T + C - 1) / C * ((N + WAVE - 1) / WAVE);
+  if (waves * WAVE > ((int64_t)1 << 31) - 1) return LSH_ERR_SHAPE;
   return LSH_OK;
 }
 
@@ -130,7 +132,7 @@ struct WarmLayout {
 };
 
 static WarmLayout warm_layout(int64_t T, int64_t N, int C) {
-  const int64_t M = T / C;
+  const int64_t M = (T + C - 1) / C;
   const size_t mn = (size_t)M * (size_t)N * 4;
   const size_t nb = (size_t)((N + WAVE - 1) / WAVE);
   WarmLayout L;
@@ -143,19 +145,9 @@ static WarmLayout warm_layout(int64_t T, int64_t N, int C) {
   return L;
 }
 
-}  // namespace lsh
-
-using namespace lsh;
-
-extern "C" size_t lsh_lif_scan_warm_workspace(int64_t T, int64_t N, int C) {
-  if (warm_check(T, N, C, 0) != LSH_OK) return 0;
-  return warm_layout(T, N, C).total;
-}
-
-extern "C" int lsh_lif_scan_warm_fwd(const float* I, const float* u0, float* U, float* S,
-                                     int64_t T, int64_t N, float beta, float theta, float u_r,
-                                     int C, int W, void* ws, size_t ws_bytes, void* stream) {
-  if (bad_ptr(I) || bad_ptr(u0) || bad_ptr(U) || bad_ptr(S) || bad_ptr(ws)) return LSH_ERR_ARG;
+static int warm_run(const float* I, const float* u0, float* U, float* S, int64_t T, int64_t N,
+                    float beta, float theta, float u_r, int C, int W, bool count, void* ws,
+                    size_t ws_bytes, void* stream) {
   const int rc = warm_check(T, N, C, W);
   if (rc != LSH_OK) return rc;
   const WarmLayout L = warm_layout(T, N, C);
@@ -168,23 +160,54 @@ extern "C" int lsh_lif_scan_warm_fwd(const float* I, const float* u0, float* U, 
     LSH_CHECK_LAUNCH();
     return LSH_OK;
   }
-  const int M = (int)(T / C);
+  const int M = (int)((T + C - 1) / C);
   const int NB = (int)((N + WAVE - 1) / WAVE);
   float* starts = reinterpret_cast<float*>(w + L.STARTS);
   float* ends = reinterpret_cast<float*>(w + L.ENDS);
-  hipLaunchKernelGGL(k_lif_fwd_warm, dim3((unsigned)((int64_t)M * NB)), dim3(WAVE), 0, st, I, u0,
-                     U, S, starts, ends, N, C, W, NB, beta, theta, u_r);
+  hipLaunchKernelGGL(k_lif_fwd_warm, dim3((unsigned)((int64_t)M * NB)), dim3(WAVE), 0, st, I, u0, U, S,
+                     starts, ends, T, N, C, W, NB, beta, theta, u_r);
   // The per-block repair counts the missed predictions, so count them here first (the wide
   // round fixes most of them before that repair looks).
   if (M > 1) {
-    hipLaunchKernelGGL(k_lif_count_missed, dim3((unsigned)((int64_t)(M - 1) * NB)), dim3(WAVE), 0,
-                       st, starts, ends, h, N, NB);
-    hipLaunchKernelGGL(k_lif_repair_wide, dim3((unsigned)((int64_t)(M - 1) * NB)), dim3(WAVE), 0,
-                       st, I, U, S, starts, ends, N, C, NB, beta, theta, u_r);
+    const dim3 rest((unsigned)((int64_t)(M - 1) * NB));
+    if (count)
+      hipLaunchKernelGGL(k_lif_count_missed, rest, dim3(WAVE), 0, st, starts, ends, h, N, NB);
+    hipLaunchKernelGGL(k_lif_repair_wide, rest, dim3(WAVE), 0, st, I, U, S, starts, ends, T, N, C, NB,
+                       beta, theta, u_r);
   }
   lif_repair_launch(I, U, S, starts, ends, reinterpret_cast<int*>(w + L.LIST0),
-                    reinterpret_cast<int*>(w + L.LIST1), h, N, M, C, (int64_t)M, beta, theta, u_r,
+                    reinterpret_cast<int*>(w + L.LIST1), h, T, N, M, C, (int64_t)M, beta, theta, u_r,
                     st);
   LSH_CHECK_LAUNCH();
   return LSH_OK;
+}
+
+}  // namespace lsh
+
+using namespace lsh;
+
+extern "C" size_t lsh_lif_scan_warm_workspace(int64_t T, int64_t N, int C) {
+  if (warm_check(T, N, C, 0) != LSH_OK || T % C != 0) return 0;
+  return warm_layout(T, N, C).total;
+}
+
+extern "C" int lsh_lif_scan_warm_fwd(const float* I, const float* u0, float* U, float* S,
+                                     int64_t T, int64_t N, float beta, float theta, float u_r,
+                                     int C, int W, void* ws, size_t ws_bytes, void* stream) {
+  if (bad_ptr(I) || bad_ptr(u0) || bad_ptr(U) || bad_ptr(S) || bad_ptr(ws)) return LSH_ERR_ARG;
+  const int rc = warm_check(T, N, C, W);
+  if (rc != LSH_OK) return rc;
+  if (T % C != 0) return LSH_ERR_DIVISIBILITY;
+  return warm_run(I, u0, U, S, T, N, beta, theta, u_r, C, W, true, ws, ws_bytes, stream);
+}
+
+extern "C" size_t lsh_lif_scan_warm_any_workspace(int64_t T, int64_t N, int C) {
+  return warm_check(T, N, C, 0) != LSH_OK ? 0 : warm_layout(T, N, C).total;
+}
+
+extern "C" int lsh_lif_scan_warm_any_fwd(const float* I, const float* u0, float* U, float* S,
+                                         int64_t T, int64_t N, float beta, float theta, float u_r,
+                                         int C, int W, void* ws, size_t ws_bytes, void* stream) {
+  if (bad_ptr(I) || bad_ptr(u0) || bad_ptr(U) || bad_ptr(S) || bad_ptr(ws)) return LSH_ERR_ARG;
+  return warm_run(I, u0, U, S, T, N, beta, theta, u_r, C, W, false, ws, ws_bytes, stream);
 }

@@ -93,6 +93,9 @@ SIGNATURES = {
     "lsh_lif_scan_warm_workspace": (c_sz, [c_i64, c_i64, c_i]),
     "lsh_lif_scan_warm_fwd": (c_i, [c_p, c_p, c_p, c_p, c_i64, c_i64, c_f, c_f, c_f, c_i, c_i, c_p,
                                     c_sz, c_p]),
+    "lsh_lif_scan_warm_any_workspace": (c_sz, [c_i64, c_i64, c_i]),
+    "lsh_lif_scan_warm_any_fwd": (c_i, [c_p, c_p, c_p, c_p, c_i64, c_i64, c_f, c_f, c_f, c_i, c_i, c_p,
+                                        c_sz, c_p]),
     "lsh_lif_scan_lo_fwd": (c_i, [c_p, c_p, c_p, c_p, c_p, c_i64, c_i64, c_f, c_f, c_f, c_i, c_i,
                                   c_i64, c_p, c_sz, c_p]),
     "lsh_scan_stats_read": (c_i, [c_p, c_i64, c_i64, c_i, ctypes.POINTER(ScanStats), c_p]),

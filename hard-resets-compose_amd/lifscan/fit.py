@@ -61,7 +61,7 @@ def _param_backward(I, u0, U, S, GS, beta, theta, u_r, alpha, mode):
 
 class LIFParamFn(torch.autograd.Function):
     """S = LIF(I; u0, beta, theta, u_r) with gradients for I, u0 and the three parameters
-    (fit.py:15-48).  fwd_mode / bwd_mode: "serial" or "scan"."""
+    (fit.py:15-48).  fwd_mode / bwd_mode: "serial" or "scan", or lif_param's own choices."""
 
     @staticmethod
     def forward(ctx, I, u0, beta, theta, u_r, alpha, fwd_mode, bwd_mode, K):
@@ -78,6 +78,8 @@ class LIFParamFn(torch.autograd.Function):
             return S
         if fwd_mode == "scan":
             U, S = L.scan_forward_auto(I, b, th, ur, u0, K=K)
+        elif fwd_mode == "auto":
+            U, S = L._auto_forward(I, b, th, ur, u0, K, 0)
         else:
             U, S = L.serial_forward_auto(I, b, th, ur, u0)
         ctx.save_for_backward(I, u0, U, S)
@@ -107,7 +109,7 @@ def lif_param(I, u0, beta, theta, u_r, alpha=4.0, mode="auto", K=16):
     T, N = I.shape
     if mode == "auto":
         fwd, bwd = L.auto_modes(N, T)
-        bwd = L._auto_bwd(bwd, N, T)
+        fwd, bwd = L._auto_fwd(fwd, N, T), L._auto_bwd(bwd, N, T)
     else:
         fwd = bwd = mode
     return LIFParamFn.apply(I, u0, beta, theta, u_r, alpha, fwd, bwd, K)

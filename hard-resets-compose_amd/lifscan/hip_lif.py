@@ -304,6 +304,9 @@ def _converged_fast(I, beta, theta, u_r, u0, C, K, repair, stats):
         plan = warm_plan(T, N, beta)
         if plan is not None:
             return _scan_warm_run(I, beta, theta, u_r, u0, *plan)
+        plan = warm_any_plan(T, N, beta)
+        if plan is not None:
+            return _warm_any(I, beta, theta, u_r, u0, *plan)
     if _fused_fwd_ok(T, C, K, repair, stats):
         long_c = long_sequence_C(T, N)
         if long_c:  # few neurons, long T: the multi-kernel scan with long chunks is faster
@@ -453,6 +456,49 @@ def _scan_warm_run(I, beta, theta, u_r, u0, C, W):
     global _LAST_RUN
     U, S = scan_forward_warm(I, beta, theta, u_r, u0, C=C, W=W)
     _LAST_RUN = _WarmRun(C, W)
+    return U, S
+
+
+# Warm-started chunks where T has no power-of-two chunk, and for the layers that pick their own
+# forward (lif_auto, lif_param): chunks of T*nb/WARM_TARGET_WAVES steps, the last one short.  From
+# 4W steps up to 1024 neurons and 8W up to 4096 (there the repair of the missed chunks weighs
+# more), against the serial sweep's 18 ns a step.  Measured on MI355X, serial -> warm: beta 0.95
+# (W 512) N = 64, T = 60001 1076 -> 55 us; N = 1000, T = 2001 / 16001 41 -> 27 / 293 -> 70 us;
+# N = 4096, T = 4001 77 -> 49 us; beta 0.99 (W 2560) N = 64 / 1000, T = 16001 290 -> 95 / 293 ->
+# 174 us, but N = 4096, T = 16001 294 -> 420 and T = 60001 1214 -> 972 us.  From 8192 neurons the
+# sweep fills the chip: T = 2001 / 4001 42 / 79 us against 47 / 76.
+WARM_ANY_WIDE_N = 1024
+
+
+def warm_any_plan(T, N, beta):
+    """(C, W) of the warm-started forward for any T, or None where the serial sweep is as fast."""
+    if N > WARM_FEW_MAX_N or N < 1:
+        return None
+    b = abs(_f32(beta))
+    if not b < 1.0:
+        return None
+    W = int(min(8192, max(256, 256 * math.ceil(WARM_K / (1.0 - b) / 256.0))))
+    if T < (4 if N <= WARM_ANY_WIDE_N else 8) * W:
+        return None
+    target = WARM_TARGET_WAVES_LARGE if T * N >= WARM_LARGE_WORK else WARM_TARGET_WAVES
+    C = T * ((N + 63) // 64) // target
+    return max(WARM_MIN_C, (C + 15) // 16 * 16), W
+
+
+def _warm_any(I, beta, theta, u_r, u0, C, W):
+    """The warm-started forward for every T (its last chunk may be short) -> (U, S)."""
+    I = _input(I)
+    T, N = I.shape
+    u0 = _vec(u0, N, I)
+    L = _n.lib()
+    nbytes = L.lsh_lif_scan_warm_any_workspace(T, N, C)
+    ws = _n.workspace(nbytes, I.device)
+    U = torch.empty_like(I)
+    S = torch.empty_like(I)
+    with _n.on_device(I):
+        _n.check(L.lsh_lif_scan_warm_any_fwd(
+            _n.ptr(I), _n.ptr(u0), _n.ptr(U), _n.ptr(S), T, N, _f32(beta), _f32(theta), _f32(u_r),
+            C, W, _n.ptr(ws), nbytes, _n.stream_of(I)), "lsh_lif_scan_warm_any_fwd")
     return U, S
 
 
@@ -1049,6 +1095,25 @@ def auto_modes(N, T):
     return fwd, bwd
 
 
+def _auto_fwd(fwd, N, T):
+    """auto_modes' forward mode, or "auto" where warm-started chunks may apply: the layer's forward
+    then decides from beta (_auto_forward)."""
+    return "auto" if 1 <= N <= WARM_FEW_MAX_N and T >= 4 * 256 else fwd
+
+
+def _auto_forward(I, beta, theta, u_r, u0, K, repair):
+    """(U, S) of a layer's own choice: warm-started chunks (the serial recurrence's bits, faster than
+    the serial sweep and than the map scan: N = 64, T = 50000 0.91 ms of map scan -> 0.06 ms), else
+    auto_modes' forward."""
+    T, N = I.shape
+    plan = warm_any_plan(T, N, beta)
+    if plan is not None:
+        return _warm_any(I, beta, theta, u_r, u0, *plan)
+    if auto_modes(N, T)[0] == "scan":
+        return scan_forward_auto(I, beta, theta, u_r, u0, K=K, repair=repair)
+    return serial_forward_auto(I, beta, theta, u_r, u0)
+
+
 # Up to this many neurons lif_auto's adjoint of a long T that has no chunk (auto_modes: serial) is
 # the look-back pass, serial -> look-back: N = 64, T = 4001 94 -> 19 us; N = 1024, T = 2001 50 -> 19
 # us; N = 8192, T = 4001 166 -> 119 us.  Above, the serial sweep fills the chip as well (N = 14083,
@@ -1210,6 +1275,8 @@ class LIFAuto(torch.autograd.Function):
             return S
         if fwd_mode == "scan":
             U, S = scan_forward_auto(I, b, theta, u_r, u0, K=K, repair=repair)
+        elif fwd_mode == "auto":
+            U, S = _auto_forward(I, b, theta, u_r, u0, K, repair)
         else:
             U, S = serial_forward_auto(I, b, theta, u_r, u0)
         ctx.save_for_backward(I, u0, U, S)
@@ -1240,8 +1307,9 @@ class LIFAuto(torch.autograd.Function):
 
 
 def lif_auto(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, K=16, repair=0):
-    fwd, bwd = auto_modes(I.shape[1], I.shape[0])
-    bwd = _auto_bwd(bwd, I.shape[1], I.shape[0])
+    T, N = I.shape
+    fwd, bwd = auto_modes(N, T)
+    fwd, bwd = _auto_fwd(fwd, N, T), _auto_bwd(bwd, N, T)
     if fwd == bwd:  # one mode for both passes: lif_tuned's path (the same kernels and bits)
         return lif_tuned(I, u0, beta, theta, u_r, alpha, mode=fwd, K=K, repair=repair)
     return LIFAuto.apply(I, u0, beta, theta, u_r, alpha, K, repair, fwd, bwd)

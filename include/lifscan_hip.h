@@ -127,6 +127,13 @@ int lsh_lif_scan_warm_fwd(const float* I, const float* u0, float* U, float* S, i
                           int64_t N, float beta, float theta, float u_r, int C, int W, void* ws,
                           size_t ws_bytes, void* stream);
 
+/* lsh_lif_scan_warm_fwd for every T: ceil(T/C) chunks, the last one short.  Same result; the missed
+ * predictions are not counted (fused_fixups stays 0). */
+size_t lsh_lif_scan_warm_any_workspace(int64_t T, int64_t N, int C);
+int lsh_lif_scan_warm_any_fwd(const float* I, const float* u0, float* U, float* S, int64_t T,
+                              int64_t N, float beta, float theta, float u_r, int C, int W, void* ws,
+                              size_t ws_bytes, void* stream);
+
 /* Two-level scan pruned with one caller-given lower bound per neuron (lo[N], e.g. the loose
  * state_bounds of triton_lif.py:238-243) instead of the per-chunk envelope.  Replaces
  * triton_lif.py:262-295 (scan_forward), :479-509 (scan_forward_tiled) and :609-642

@@ -71,3 +71,43 @@ def test_long_lengths_without_a_chunk_are_still_refused(dev):
         L.scan_backward_lookback(z(1000), u0, z(1000), z(1000), z(1000), None, 0.9, 1.0, 0.0)
     with pytest.raises(ValueError):
         AF._aff_backward(z(2049), u0, z(2049), z(2049), z(2049), 0.9, 1.0, 0.5, 4.0)
+
+
+@pytest.mark.parametrize("T,N,C,W", [(1, 3, 256, 256), (257, 70, 256, 256), (4001, 65, 272, 0),
+                                     (4095, 130, 256, 512), (4097, 64, 1024, 64)])
+@pytest.mark.parametrize("beta,mu,sd", [(0.9, 0.12, 0.25), (0.99, 0.012, 0.08)])
+def test_warm_forward_any_length(dev, T, N, C, W, beta, mu, sd):
+    """The warm-started forward with a short last chunk is the serial recurrence bit for bit, also
+    with warm-ups too short to predict anything (the repair's short chunk)."""
+    from lifscan import hip_lif as L
+    I, u0 = normal(T, N, mu, sd, T), uniform(N, 0.0, 1.0, 5)
+    Uo, So = O.serial_forward(I, beta, 1.0, -0.1, u0)
+    pad = torch.cat([gpu(I, dev), torch.full((300, N), float("nan"), device=dev)])[:T]
+    print(f"warm any T={T} N={N} C={C} W={W}", flush=True)
+    U, S = L._warm_any(pad, beta, 1.0, -0.1, gpu(u0, dev), C, W)
+    assert np.array_equal(host(U), Uo) and np.array_equal(host(S), So)
+
+
+def test_warm_any_plan_and_auto_layer(dev):
+    """The layers' own forward at the bounds of the plan: the serial recurrence's spikes, and the
+    adjoint of the look-back pass."""
+    from lifscan import hip_lif as L
+    assert L.warm_any_plan(2047, 64, 0.95) is None and L.warm_any_plan(2048, 64, 0.95) == (256, 512)
+    assert L.warm_any_plan(60001, 64, 0.95) == (256, 512)
+    assert L.warm_any_plan(4095, 4096, 0.95) is None and L.warm_any_plan(4096, 4096, 0.95) == (512, 512)
+    assert L.warm_any_plan(10 ** 5, 4097, 0.9) is None and L.warm_any_plan(10 ** 5, 64, 1.0) is None
+    T, N = 2501, 70
+    I, GS = normal(T, N, 0.15, 0.4, 1), normal(T, N, 0.0, 1.0, 2)
+    u0 = uniform(N, 0.0, 1.0, 3)
+    Uo, So = O.serial_forward(I, 0.95, 1.0, 0.0, u0)
+    want = O.serial_backward(I, u0, Uo, So, GS, None, 0.95, 1.0, 0.0, 4.0, True, dtype=np.float64)
+    Ig, ug = gpu(I, dev).requires_grad_(True), gpu(u0, dev).requires_grad_(True)
+    b = torch.tensor(0.95, device=dev, requires_grad=True)
+    for beta in (0.95, b):
+        S = L.lif_auto(Ig, ug, beta)
+        dI, du0 = torch.autograd.grad(S, [Ig, ug], gpu(GS, dev), retain_graph=True)
+        assert np.array_equal(host(S), So)
+        assert rel(host(dI), want) < 1e-6 and rel(host(du0), 0.95 * want[0]) < 1e-6
+    db, = torch.autograd.grad(S, [b], gpu(GS, dev))
+    up = np.concatenate([u0[None], Uo[:-1]]).astype(np.float64)
+    assert rel(db.item(), (want * up).sum()) < 1e-4
