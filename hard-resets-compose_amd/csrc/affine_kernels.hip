@@ -80,6 +80,8 @@ __global__ __launch_bounds__(64) void k_aff_env(const float* __restrict__ I,
   HB[o] = hb;
 }
 
+constexpr int kAffAhead = 8;  // chunks whose envelope maps the carry reads ahead
+
 // Sequential envelope carries (triton_lif.py:723-733, triton_affine.py:39-48), margin 1e-5:
 // LO[m] = l - 1e-5(|l| + 1), HI[m] = h + 1e-5(|h| + 1) with l, h the bounds at chunk m's start.
 __global__ __launch_bounds__(64) void k_aff_env_carry(
@@ -90,123 +92,259 @@ __global__ __launch_bounds__(64) void k_aff_env_carry(
   if (n >= N) return;
   const float margin = 1e-5f;
   float l = u0[n], h = l;
-  for (int m = 0; m < M; ++m) {
-    const size_t o = (size_t)m * N + n;
-    LO[o] = l - margin * (fabsf(l) + 1.0f);
-    HI[o] = h + margin * (fabsf(h) + 1.0f);
-    l = fminf(EC[o], __fadd_rn(__fmul_rn(EA[o], l), EB[o]));
-    h = fmaxf(HC[o], __fadd_rn(__fmul_rn(HA[o], h), HB[o]));
+  // The maps of the next kAffAhead chunks are in flight while one is applied (index clamped, every
+  // load unconditional): one chunk at a time waited for six loads per chunk, 23 us for 64 chunks.
+  float ec[kAffAhead], ea[kAffAhead], eb[kAffAhead], hc[kAffAhead], ha[kAffAhead], hb[kAffAhead];
+  const auto load = [&](int k, int m) {
+    const size_t o = (size_t)min(m, M - 1) * N + n;
+    ec[k] = EC[o];
+    ea[k] = EA[o];
+    eb[k] = EB[o];
+    hc[k] = HC[o];
+    ha[k] = HA[o];
+    hb[k] = HB[o];
+    __builtin_amdgcn_sched_barrier(0);  // issued in the chunks' order
+  };
+#pragma unroll
+  for (int k = 0; k < kAffAhead; ++k) load(k, k);
+  for (int m0 = 0; m0 < M; m0 += kAffAhead) {
+#pragma unroll
+    for (int k = 0; k < kAffAhead; ++k) {
+      const int m = m0 + k;
+      if (m < M) {
+        const size_t o = (size_t)m * N + n;
+        LO[o] = l - margin * (fabsf(l) + 1.0f);
+        HI[o] = h + margin * (fabsf(h) + 1.0f);
+        l = fminf(ec[k], __fadd_rn(__fmul_rn(ea[k], l), eb[k]));
+        h = fmaxf(hc[k], __fadd_rn(__fmul_rn(ha[k], h), hb[k]));
+      }
+      load(k, m + kAffAhead);
+    }
   }
 }
 
 // ---------------------------------------------------------------------------------------
-// Chunk maps (triton_affine.py:51-111).  A workgroup owns 16 neurons of one chunk; 32 lanes
-// serve one neuron (two per wave), lane i holding piece slot i.  Inputs are staged through LDS
-// in tiles of 64 steps together with ct = (theta - x)/beta, computed once per (neuron, step).
+// Chunk maps (triton_affine.py:51-111).  A workgroup owns 16 neurons of one chunk; a 16-lane row
+// serves one neuron (4 neurons a wave), lane i holding piece slots i and 16 + i; the second is
+// touched only while some neuron of the wave has more than 16 pieces.  Inputs are staged through
+// LDS in tiles of 32 steps together with ct = (theta - x)/beta, computed once per (neuron, step);
+// the next tile's inputs are loaded while a tile runs.
 // Per step every piece [xl, xr) with value a*u + c meets the threshold cut z = (ct - c)/a
 // (u >= z spikes; a == 0: all or nothing); its left part [xl, min(xr, z)) and its spiking
-// right part [z, xr) are kept when they meet [lo, hi].  When every live piece keeps exactly
-// one part (the common case) the pieces stay in their slots; otherwise the list is compacted
-// in order, left before right: an inclusive prefix sum of the part counts over the neuron's
-// 32 lanes (DPP row shifts plus a row broadcast), then every part is written to its slot in
-// this wave's LDS row and read back by the slot's lane.  A count above K sets the overflow
-// flag and the parts beyond slot K are dropped, as the reference's compaction does.
-constexpr int kAffNPW = 16;  // neurons per build workgroup
-constexpr int kAffTS = 64;   // steps per staged tile
+// right part [z, xr) are kept when they meet [lo, hi].
+// Between steps the slots are in no order: a piece that keeps one part stays where it is, one that
+// dies leaves a free slot, and the right part of one that keeps both goes to a free slot (through
+// the neuron's LDS row).  The pieces are disjoint intervals, so the reference's list is the slots
+// sorted by xl; they are sorted at the end of the chunk, and in a step after which a neuron would
+// hold more than K (the overflow flag is set and the parts beyond slot K are dropped, as the
+// reference's compaction does).  Compacting on every birth and death ran on two steps of three.
+// The tests are kept as wave masks (a ballot of one compare is the compare's own result); free
+// slots drift with the others and the masks leave them out.
+// Bound by VALU issue (a correctly rounded division per piece and step): most maps hold 3 to 9
+// pieces, so 32 lanes a neuron left most lanes idle.  Measured, C 128, 32 lanes a neuron and
+// compaction -> this: T 8192, N 200 gamma 0.5 82 -> 51 us, N 333 soft reset 121 -> 101 us;
+// T 4096, N 4096 537 -> 284 and 543 -> 300 us (16 lanes with compaction 59, 111, 353, 367; 8 lanes
+// and four slots 98, 177, 416, 492).
+constexpr int kAffWaves = 4;                 // waves per workgroup
+constexpr int kAffNPW = kAffWaves * 4;       // neurons per workgroup
+constexpr int kAffTS = 32;                   // steps per staged tile
+constexpr int kAffLd = kAffNPW * kAffTS / (kAffWaves * WAVE);  // inputs a lane stages per tile
 
-__global__ __launch_bounds__(WAVE * kAffNPW / 2) void k_aff_build(
+// One piece slot's step: the cut, the masks of the kept left / right parts and the updated fields.
+struct AffStepSlot {
+  float z, xr, vns, c_sp, a_sp, a_ns;
+  unsigned long long left, right, full;
+};
+__device__ __forceinline__ AffStepSlot aff_slot_step(float pxl, float pxr, float pa, float pc,
+                                                     unsigned long long live, float x, float ct,
+                                                     float lo, float hi, float beta, float gb,
+                                                     float gamma, float delta) {
+  AffStepSlot r;
+  const float num = ct - pc;
+  r.z = num / pa;
+  if (wave_ballot(pa == 0.0f) != 0ull)
+    r.z = pa == 0.0f ? (num > 0.0f ? INFINITY : -INFINITY) : r.z;
+  const unsigned long long cut = live & wave_ballot(r.z > pxl) & wave_ballot(r.z < pxr);
+  r.full = wave_ballot(r.z <= pxl);
+  r.xr = __builtin_amdgcn_inverse_ballot_w64(cut) ? r.z : pxr;
+  r.left = live & wave_ballot(r.xr > lo) & wave_ballot(pxl <= hi);
+  r.right = cut & wave_ballot(pxr > lo) & wave_ballot(r.z <= hi);
+  r.vns = lif_v(pc, x, beta);
+  r.c_sp = __fadd_rn(__fmul_rn(gamma, r.vns), delta);
+  r.a_sp = gb * pa;
+  r.a_ns = beta * pa;
+  return r;
+}
+
+__global__ __launch_bounds__(WAVE * kAffWaves) void k_aff_build(
     const float* __restrict__ I, const float* __restrict__ LO, const float* __restrict__ HI,
     float4* __restrict__ PC, int* __restrict__ NP, int* __restrict__ OVF, int64_t N, int NBLK,
     int C, int K, float beta, float theta, float gamma, float delta) {
-  constexpr int NW = kAffNPW / 2;
-  __shared__ float sX[kAffNPW][kAffTS], sCt[kAffNPW][kAffTS];
-  __shared__ float4 sSlot[NW][WAVE];
+  __shared__ float sX[kAffNPW][kAffTS + 1], sCt[kAffNPW][kAffTS + 1];
+  __shared__ float4 sSlot[kAffNPW][33];  // a neuron's slots, off the banks of the next neuron's
+  __shared__ float sKey[kAffNPW][65];    // sort keys: at most 32 pieces, each with a new part
   const int64_t m = blockIdx.x / NBLK;
   const int blk = (int)(blockIdx.x - m * NBLK);
   const int tid = threadIdx.x;
-  const int wv = tid / WAVE;
   const int lane = tid % WAVE;
-  const int half = lane >> 5;
-  const int i = lane & 31;
-  const int ln = wv * 2 + half;
+  const int i = lane & 15;
+  const int ln = tid / 16;  // neuron of the workgroup
   const int64_t n0 = (int64_t)blk * kAffNPW;
   const int64_t n = n0 + ln;
   const bool valid_n = n < N;
   const size_t o = (size_t)m * N + (valid_n ? n : N - 1);
   const float lo = LO[o], hi = HI[o];
   const float gb = gamma * beta;
-  float pxl = i == 0 ? -INFINITY : INFINITY, pxr = INFINITY, pa = 1.0f, pc = 0.0f;
+  float pxl0 = i == 0 ? -INFINITY : INFINITY, pxr0 = INFINITY, pa0 = 1.0f, pc0 = 0.0f;
+  float pxl1 = INFINITY, pxr1 = INFINITY, pa1 = 1.0f, pc1 = 0.0f;
   int cnt = 1, ovf = 0;
-  float4* slot = sSlot[wv] + (half << 5);
+  unsigned long long live0 = wave_ballot(i < 1), live1 = 0ull;
+  float4* slot = sSlot[ln];
+  const unsigned below = (1u << i) - 1;  // the row's lanes before this one
+  // the row's bits of a wave mask
+  const auto row_of = [&](unsigned long long mask) {
+    const unsigned w = lane < 32 ? (unsigned)mask : (unsigned)(mask >> 32);
+    return (w >> (lane & 16)) & 0xffffu;
+  };
+  const auto lane_of = [](unsigned long long mask) {
+    return __builtin_amdgcn_inverse_ballot_w64(mask);
+  };
+  // The row's pieces (live0, live1) and, where the masks say so, the new parts n0, n1 of this
+  // lane's slots into slots 0, 1, ... by ascending xl, the first K of them.  Same-wave LDS accesses
+  // complete in order.
+  const auto sort_row = [&](unsigned long long new0, unsigned long long new1, const float4& n0,
+                            const float4& n1) {
+    const unsigned l0 = row_of(live0), l1 = row_of(live1), b0 = row_of(new0), b1 = row_of(new1);
+    const int o1 = __popc(l0), o2 = o1 + __popc(l1), o3 = o2 + __popc(b0), tot = o3 + __popc(b1);
+    float* key = sKey[ln];
+    const bool h0 = lane_of(live0), h1 = lane_of(live1), g0 = lane_of(new0), g1 = lane_of(new1);
+    if (h0) key[__popc(l0 & below)] = pxl0;
+    if (h1) key[o1 + __popc(l1 & below)] = pxl1;
+    if (g0) key[o2 + __popc(b0 & below)] = n0.x;
+    if (g1) key[o3 + __popc(b1 & below)] = n1.x;
+    __builtin_amdgcn_wave_barrier();
+    int k0 = 0, k1 = 0, m0 = 0, m1 = 0;  // ranks
+    for (int j = 0; j < tot; ++j) {
+      const float v = key[j];
+      k0 += v < pxl0 ? 1 : 0;
+      k1 += v < pxl1 ? 1 : 0;
+      m0 += v < n0.x ? 1 : 0;
+      m1 += v < n1.x ? 1 : 0;
+    }
+    if (h0 && k0 < K) slot[k0] = make_float4(pxl0, pxr0, pa0, pc0);
+    if (h1 && k1 < K) slot[k1] = make_float4(pxl1, pxr1, pa1, pc1);
+    if (g0 && m0 < K) slot[m0] = n0;
+    if (g1 && m1 < K) slot[m1] = n1;
+    if (tot > K) ovf = 1;
+    cnt = min(tot, K);
+    __builtin_amdgcn_wave_barrier();
+    const float4 q0 = slot[i], q1 = slot[16 + i];
+    pxl0 = q0.x, pxr0 = q0.y, pa0 = q0.z, pc0 = q0.w;
+    pxl1 = q1.x, pxr1 = q1.y, pa1 = q1.z, pc1 = q1.w;
+    live0 = wave_ballot(i < cnt);
+    live1 = wave_ballot(16 + i < cnt);
+    __builtin_amdgcn_wave_barrier();
+  };
   const float* __restrict__ Im = I + (size_t)m * C * N;
+  float xr[kAffLd];
+  const auto load = [&](int j0) {  // this lane's inputs of the tile at j0 (rows past C: the last)
+#pragma unroll
+    for (int q = 0; q < kAffLd; ++q) {
+      const int e = tid + q * kAffWaves * WAVE;
+      const int64_t ne = n0 + e % kAffNPW;
+      xr[q] = Im[(size_t)min(j0 + e / kAffNPW, C - 1) * N + (ne < N ? ne : N - 1)];
+    }
+  };
+  load(0);
   for (int j0 = 0; j0 < C; j0 += kAffTS) {
     const int ts = min(kAffTS, C - j0);
-    for (int e = tid; e < kAffNPW * ts; e += NW * WAVE) {
-      const int k = e / kAffNPW, nu = e - k * kAffNPW;
-      const int64_t ne = n0 + nu < N ? n0 + nu : N - 1;
-      const float x = Im[(size_t)(j0 + k) * N + ne];
-      sX[nu][k] = x;
-      sCt[nu][k] = (theta - x) / beta;
+    __syncthreads();  // the previous tile has been read
+#pragma unroll
+    for (int q = 0; q < kAffLd; ++q) {
+      const int e = tid + q * kAffWaves * WAVE;
+      sX[e % kAffNPW][e / kAffNPW] = xr[q];
+      sCt[e % kAffNPW][e / kAffNPW] = (theta - xr[q]) / beta;
     }
     __syncthreads();
+    load(j0 + kAffTS);
+    // second slots that are no longer needed: back to one slot a lane
+    if (live1 != 0ull &&
+        wave_ballot(__popc(row_of(live0)) + __popc(row_of(live1)) > 16) == 0ull)
+      sort_row(0ull, 0ull, make_float4(0, 0, 0, 0), make_float4(0, 0, 0, 0));
+    float xs = sX[ln][0], cts = sCt[ln][0];
     for (int k = 0; k < ts; ++k) {
-      const float x = sX[ln][k], ct = sCt[ln][k];
-      const bool valid = i < cnt;
-      const float num = ct - pc;
-      const float z = pa == 0.0f ? (num > 0.0f ? INFINITY : -INFINITY) : num / pa;
-      const bool full = z <= pxl;
-      const bool split = (z > pxl) && (z < pxr) && valid;
-      const float vns = lif_v(pc, x, beta);
-      const float c_sp = __fadd_rn(__fmul_rn(gamma, vns), delta);
-      const float a_sp = gb * pa;
-      const float cl = full ? c_sp : vns;
-      const float al = full ? a_sp : beta * pa;
-      const float xrl = split ? z : pxr;
-      const bool vl = valid && (xrl > lo) && (pxl <= hi);
-      const bool vr = split && (pxr > lo) && (z <= hi);
-      const int nl = vl ? 1 : 0;
-      const int nout = nl + (vr ? 1 : 0);
-      if (__ballot(valid && nout != 1) == 0ull) {
-        // every live piece keeps one part in its slot
-        if (valid) {
-          if (vl) {
-            pxr = xrl;
-            pa = al;
-            pc = cl;
-          } else {
-            pxl = z;
-            pa = a_sp;
-            pc = c_sp;
-          }
-        }
-      } else {
-        // inclusive prefix sum over the neuron's 32 slots: row shifts within 16-lane rows,
-        // then the last lane of rows 0 / 2 added to rows 1 / 3
-        int incl = nout;
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xF, 0xF, true);  // row_shr:1
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xF, 0xF, true);  // row_shr:2
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xF, 0xF, true);  // row_shr:4
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xF, 0xF, true);  // row_shr:8
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x142, 0xA, 0xF, false);  // row_bcast:15
-        const int p = incl - nout;
-        const int ntot = __shfl(incl, 31, 32);
-        if (ntot > K) ovf = 1;
-        // same-wave LDS accesses complete in order: the scatter lands before the read-back
-        if (vl && p < K) slot[p] = make_float4(pxl, xrl, al, cl);
-        if (vr && p + nl < K) slot[p + nl] = make_float4(z, pxr, a_sp, c_sp);
-        cnt = min(ntot, K);
-        const float4 q = slot[i];
-        const bool keep = i < cnt;
-        pxl = keep ? q.x : INFINITY;
-        pxr = keep ? q.y : INFINITY;
-        pa = keep ? q.z : 1.0f;
-        pc = keep ? q.w : 0.0f;
+      const float x = xs, ct = cts;
+      xs = sX[ln][k + 1];  // the next step's (behind the tile's last step: the padding)
+      cts = sCt[ln][k + 1];
+      const AffStepSlot r0 = aff_slot_step(pxl0, pxr0, pa0, pc0, live0, x, ct, lo, hi, beta, gb,
+                                           gamma, delta);
+      const unsigned long long new0 = r0.left & r0.right;
+      const float4 n0 = make_float4(r0.z, pxr0, r0.a_sp, r0.c_sp);
+      {
+        const unsigned long long ro = r0.right & ~r0.left;
+        const bool right = lane_of(ro), sp = lane_of(ro | r0.full);
+        pxr0 = right ? pxr0 : r0.xr;
+        pxl0 = right ? r0.z : pxl0;
+        pa0 = sp ? r0.a_sp : r0.a_ns;
+        pc0 = sp ? r0.c_sp : r0.vns;
+        live0 = r0.left | r0.right;
       }
+      unsigned long long new1 = 0ull;
+      float4 n1 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (live1 != 0ull) {
+        const AffStepSlot r1 = aff_slot_step(pxl1, pxr1, pa1, pc1, live1, x, ct, lo, hi, beta, gb,
+                                             gamma, delta);
+        new1 = r1.left & r1.right;
+        n1 = make_float4(r1.z, pxr1, r1.a_sp, r1.c_sp);
+        const unsigned long long ro = r1.right & ~r1.left;
+        const bool right = lane_of(ro), sp = lane_of(ro | r1.full);
+        pxr1 = right ? pxr1 : r1.xr;
+        pxl1 = right ? r1.z : pxl1;
+        pa1 = sp ? r1.a_sp : r1.a_ns;
+        pc1 = sp ? r1.c_sp : r1.vns;
+        live1 = r1.left | r1.right;
+      }
+      if ((new0 | new1) == 0ull) continue;
+      const unsigned b0 = row_of(new0), b1 = row_of(new1);
+      const unsigned f0 = ~row_of(live0) & 0xffffu, f1 = ~row_of(live1) & 0xffffu;
+      const int nb0 = __popc(b0), nb = nb0 + __popc(b1), nf0 = __popc(f0);
+      if (wave_ballot(32 - nf0 - __popc(f1) + nb > K) != 0ull) {
+        sort_row(new0, new1, n0, n1);
+        continue;
+      }
+      // the j-th new part of the row to its j-th free slot
+      if (lane_of(new0)) slot[__popc(b0 & below)] = n0;
+      if (lane_of(new1)) slot[nb0 + __popc(b1 & below)] = n1;
+      __builtin_amdgcn_wave_barrier();
+      const int j = __popc(f0 & below);
+      const bool take = ((f0 >> i) & 1u) != 0u && j < nb;
+      const float4 q = slot[j];
+      pxl0 = take ? q.x : pxl0;
+      pxr0 = take ? q.y : pxr0;
+      pa0 = take ? q.z : pa0;
+      pc0 = take ? q.w : pc0;
+      live0 |= wave_ballot(take);
+      if (wave_ballot(nb > nf0) != 0ull) {
+        const int j1 = nf0 + __popc(f1 & below);
+        const bool take1 = ((f1 >> i) & 1u) != 0u && j1 < nb;
+        const float4 q1 = slot[j1];
+        pxl1 = take1 ? q1.x : pxl1;
+        pxr1 = take1 ? q1.y : pxr1;
+        pa1 = take1 ? q1.z : pa1;
+        pc1 = take1 ? q1.w : pc1;
+        live1 |= wave_ballot(take1);
+      }
+      __builtin_amdgcn_wave_barrier();
     }
-    __syncthreads();  // the tile's LDS rows are rewritten next
   }
+  sort_row(0ull, 0ull, make_float4(0, 0, 0, 0), make_float4(0, 0, 0, 0));
   if (!valid_n) return;
-  if (i < K) PC[o * K + i] = make_float4(pxl, pxr, pa, pc);
+  if (i < K)
+    PC[o * K + i] = i < cnt ? make_float4(pxl0, pxr0, pa0, pc0)
+                            : make_float4(INFINITY, INFINITY, 1.0f, 0.0f);
+  if (16 + i < K)
+    PC[o * K + 16 + i] = 16 + i < cnt ? make_float4(pxl1, pxr1, pa1, pc1)
+                                      : make_float4(INFINITY, INFINITY, 1.0f, 0.0f);
   if (i == 0) {
     NP[o] = cnt;
     OVF[o] = ovf;
@@ -216,18 +354,20 @@ __global__ __launch_bounds__(WAVE * kAffNPW / 2) void k_aff_build(
 // Verified carry (triton_affine.py:114-140), two neurons per wave, lane i = piece slot i: the
 // start u must lie in exactly one piece of a map that did not overflow, and the chunk's end
 // state is that piece's a*u + c (plus 0.0: the reference sums the hit lanes, so a -0.0 reads
-// as +0.0); otherwise the chunk runs serially.  The next chunk's map is loaded before the
-// current one is evaluated.
-__global__ __launch_bounds__(64) void k_aff_carry(
+// as +0.0); otherwise the chunk runs serially.  The next kAffMaps chunks' maps are in flight while
+// one is evaluated (one ahead left the walk waiting for memory: 64 chunks of 200 neurons 39 -> 18 us).
+constexpr int kAffMaps = 4;
+constexpr int kAffCarryWaves = 4;  // waves of a workgroup, which adds its statistics once
+__global__ __launch_bounds__(WAVE* kAffCarryWaves) void k_aff_carry(
     const float* __restrict__ I, const float* __restrict__ u0, const float4* __restrict__ PC,
     const int* __restrict__ NP, const int* __restrict__ OVF, float* __restrict__ STARTS,
     WsHeader* hdr, int64_t N, int M, int C, int K, float beta, float theta, float gamma,
     float delta) {
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x % WAVE;
   const int half = lane >> 5;
   const int i = lane & 31;
   const int hb = half << 5;
-  const int64_t n = (int64_t)blockIdx.x * 2 + half;
+  const int64_t n = ((int64_t)blockIdx.x * kAffCarryWaves + threadIdx.x / WAVE) * 2 + half;
   const bool valid_n = n < N;
   const int64_t nn = valid_n ? n : N - 1;
   const unsigned long long hmask = 0xffffffffull << hb;
@@ -236,51 +376,53 @@ __global__ __launch_bounds__(64) void k_aff_carry(
   float u = u0[nn];
   unsigned long long ovf_acc = 0, pcs_acc = 0;
   int pmax = 0;
-  float4 q = PC[(size_t)nn * K + ks];
-  int cnt = NP[nn], ovf = OVF[nn];
-  for (int m = 0; m < M; ++m) {
-    const size_t o = (size_t)m * N + nn;
-    float4 qn = q;
-    int cntn = 0, ovfn = 0;
-    if (m + 1 < M) {
-      const size_t on = o + (size_t)N;
-      qn = PC[on * K + ks];
-      cntn = NP[on];
-      ovfn = OVF[on];
+  float4 qs[kAffMaps];
+  int cnts[kAffMaps], ovfs[kAffMaps];
+  const auto load = [&](int k, int m) {
+    const size_t o = (size_t)min(m, M - 1) * N + nn;
+    qs[k] = PC[o * K + ks];
+    cnts[k] = NP[o];
+    ovfs[k] = OVF[o];
+    // the loads stay in the chunks' order: with a later chunk's issued first, the wait for the
+    // current chunk covers them all
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int k = 0; k < kAffMaps; ++k) load(k, k);
+  for (int m0 = 0; m0 < M; m0 += kAffMaps) {
+#pragma unroll
+    for (int k = 0; k < kAffMaps; ++k) {
+      const int m = m0 + k;
+      if (m < M) {
+        const float4 q = qs[k];
+        const int cnt = cnts[k], ovf = ovfs[k];
+        if (valid_n && i == 0) STARTS[(size_t)m * N + nn] = u;
+        const bool hit = i < cnt && q.x <= u && u < q.y;
+        const unsigned long long hm = (wave_ballot(hit) & hmask) >> hb;
+        const int nh = __builtin_popcountll(hm);
+        const int hl = hm ? __builtin_ctzll(hm) : 0;
+        const float val = __fadd_rn(__fmul_rn(q.z, u), q.w);
+        float nu = __shfl(val, hl, 32) + 0.0f;  // all lanes shuffle
+        if (ovf != 0 || nh != 1) {
+          float w = u;
+          stream_rows<16>(I + (size_t)m * C * N + nn, (size_t)N, C, [&](int64_t, float x) {
+            bool s;
+            w = aff_step(w, x, beta, theta, gamma, delta, s);
+          });
+          nu = w;
+        }
+        if (valid_n && i == 0) {
+          ovf_acc += ovf ? 1ull : 0ull;
+          pcs_acc += (unsigned long long)cnt;
+          pmax = max(pmax, cnt);
+        }
+        u = nu;
+      }
+      load(k, m + kAffMaps);
     }
-    if (valid_n && i == 0) STARTS[o] = u;
-    const bool hit = i < cnt && q.x <= u && u < q.y;
-    const unsigned long long hm = (__ballot(hit) & hmask) >> hb;
-    const int nh = __builtin_popcountll(hm);
-    const int hl = hm ? __builtin_ctzll(hm) : 0;
-    const float val = __fadd_rn(__fmul_rn(q.z, u), q.w);
-    float nu = __shfl(val, hl, 32) + 0.0f;  // all lanes shuffle
-    if (ovf != 0 || nh != 1) {
-      float w = u;
-      stream_rows<16>(I + (size_t)m * C * N + nn, (size_t)N, C, [&](int64_t, float x) {
-        bool s;
-        w = aff_step(w, x, beta, theta, gamma, delta, s);
-      });
-      nu = w;
-    }
-    if (valid_n && i == 0) {
-      ovf_acc += ovf ? 1ull : 0ull;
-      pcs_acc += (unsigned long long)cnt;
-      pmax = max(pmax, cnt);
-    }
-    u = nu;
-    q = qn;
-    cnt = cntn;
-    ovf = ovfn;
   }
-  ovf_acc = wave_sum_u64(ovf_acc);
-  pcs_acc = wave_sum_u64(pcs_acc);
-  pmax = wave_max_i(pmax);
-  if (lane == 0) {
-    atomicAdd(&hdr->ovf_count, ovf_acc);
-    atomicAdd(&hdr->pieces_sum, pcs_acc);
-    atomicMax(&hdr->pieces_max, (unsigned int)pmax);
-  }
+  add_map_stats(hdr, ovf_acc, pcs_acc, pmax);
 }
 
 // Jacobi repair of the chunk starts on device (triton_affine.py:188-194): chunk m (> 0) whose
@@ -498,10 +640,12 @@ extern "C" int lsh_aff_scan_fwd(const float* I, const float* u0, float* U, float
                      delta, r_theta);
   hipLaunchKernelGGL(k_aff_env_carry, dim3((unsigned)NB), dim3(WAVE), 0, st, u0, F(L.EC), F(L.EA),
                      F(L.EB), F(L.HC), F(L.HA), F(L.HB), F(L.LO), F(L.HI), N, M);
-  hipLaunchKernelGGL(k_aff_build, dim3((unsigned)((int64_t)M * NBLK)), dim3(WAVE * kAffNPW / 2), 0,
+  hipLaunchKernelGGL(k_aff_build, dim3((unsigned)((int64_t)M * NBLK)), dim3(WAVE * kAffWaves), 0,
                      st, I, F(L.LO), F(L.HI), PC, Iq(L.NP), Iq(L.OVF), N, NBLK, C, K, beta, theta,
                      gamma, delta);
-  hipLaunchKernelGGL(k_aff_carry, dim3((unsigned)((N + 1) / 2)), dim3(WAVE), 0, st, I, u0, PC,
+  hipLaunchKernelGGL(k_aff_carry,
+                     dim3((unsigned)((N + 2 * kAffCarryWaves - 1) / (2 * kAffCarryWaves))),
+                     dim3(WAVE * kAffCarryWaves), 0, st, I, u0, PC,
                      Iq(L.NP), Iq(L.OVF), F(L.STARTS), h, N, M, C, K, beta, theta, gamma, delta);
   hipLaunchKernelGGL((k_aff_fwd<16>), dim3((unsigned)((int64_t)M * NB)), dim3(WAVE), 0, st, I,
                      F(L.STARTS), U, S, F(L.ENDS), N, (int64_t)C, NB, beta, theta, gamma, delta);
