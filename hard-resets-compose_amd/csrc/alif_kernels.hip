@@ -109,6 +109,10 @@ __global__ __launch_bounds__(64) void k_alif_fwd(const float* __restrict__ I,
   }
 }
 
+// Rows read ahead by the warm-up predictor and the chunk envelopes: one chain a lane, which waited
+// for every load without it (N 1024, T 16384, C 128: predictor 201 -> 38 us, envelopes 50 -> 11 us).
+constexpr int kEnvRows = 16;
+
 // Warm-up predictor (triton_alif.py:75-92): chunk m simulates chunks max(m-Wn,0)..m-1.
 __global__ __launch_bounds__(64) void k_alif_warm(const float* __restrict__ I,
                                                   const float* __restrict__ u0,
@@ -134,10 +138,10 @@ __global__ __launch_bounds__(64) void k_alif_warm(const float* __restrict__ I,
     u = u_init;
     w = w_init;
   }
-  for (int64_t t = s0 * C; t < m * C; ++t) {
+  stream_rows<kEnvRows>(I + (size_t)s0 * C * N + n, (size_t)N, (m - s0) * C, [&](int64_t, float x) {
     bool s;
-    u = alif_step(u, w, I[(size_t)t * N + n], beta, rho, q, theta0, u_r, s);
-  }
+    u = alif_step(u, w, x, beta, rho, q, theta0, u_r, s);
+  });
   WP[m * N + n] = w;
 }
 
@@ -152,13 +156,11 @@ __global__ __launch_bounds__(64) void k_env_chunks(const float* __restrict__ I,
   const int64_t n = (int64_t)nb * WAVE + threadIdx.x;
   if (n >= N) return;
   float c = INFINITY, a = 1.0f, b = 0.0f;
-  const float* __restrict__ Ip = I + (size_t)m * C * N + n;
-  for (int j = 0; j < C; ++j) {
-    const float x = Ip[(size_t)j * N];
+  stream_rows<kEnvRows>(I + (size_t)m * C * N + n, (size_t)N, C, [&](int64_t, float x) {
     c = fminf(u_r, lif_v(c, x, beta));
     a = beta * a;
     b = lif_v(b, x, beta);
-  }
+  });
   EC[m * N + n] = c;
   EA[m * N + n] = a;
   EB[m * N + n] = b;
