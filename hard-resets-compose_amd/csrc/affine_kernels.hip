@@ -21,7 +21,7 @@ namespace lsh {
 
 // ---------------------------------------------------------------------------------------
 // Serial / replay over segments of Ls steps from su (triton_affine.py:143-162).
-template <int D>
+template <int D, bool NT>
 __global__ __launch_bounds__(64) void k_aff_fwd(const float* __restrict__ I,
                                                 const float* __restrict__ su, float* __restrict__ U,
                                                 float* __restrict__ S, float* __restrict__ eu,
@@ -37,8 +37,8 @@ __global__ __launch_bounds__(64) void k_aff_fwd(const float* __restrict__ I,
     bool s;
     u = aff_step(u, x, beta, theta, gamma, delta, s);
     const size_t o = base + (size_t)j * N;
-    st_nt(U + o, u);
-    st_nt(S + o, s ? 1.0f : 0.0f);
+    st_out<NT>(U + o, u);
+    st_out<NT>(S + o, s ? 1.0f : 0.0f);
   });
   if (eu) eu[m * N + n] = u;
 }
@@ -647,8 +647,10 @@ extern "C" int lsh_aff_scan_fwd(const float* I, const float* u0, float* U, float
                      dim3((unsigned)((N + 2 * kAffCarryWaves - 1) / (2 * kAffCarryWaves))),
                      dim3(WAVE * kAffCarryWaves), 0, st, I, u0, PC,
                      Iq(L.NP), Iq(L.OVF), F(L.STARTS), h, N, M, C, K, beta, theta, gamma, delta);
-  hipLaunchKernelGGL((k_aff_fwd<16>), dim3((unsigned)((int64_t)M * NB)), dim3(WAVE), 0, st, I,
+  with_store_policy(N, [&](auto nt) {
+    hipLaunchKernelGGL((k_aff_fwd<16, decltype(nt)::value>), dim3((unsigned)((int64_t)M * NB)), dim3(WAVE), 0, st, I,
                      F(L.STARTS), U, S, F(L.ENDS), N, (int64_t)C, NB, beta, theta, gamma, delta);
+  });
   if (repair > 0 && M > 1) {
     const int64_t rounds = repair < (int64_t)M ? repair : (int64_t)M;
     hipLaunchKernelGGL(k_aff_repair, dim3((unsigned)NB), dim3(256), 0, st, I, U, S, F(L.STARTS),

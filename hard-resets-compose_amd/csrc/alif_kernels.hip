@@ -49,7 +49,7 @@ __device__ __forceinline__ float nmax(float a, float b) {
 
 // ---------------------------------------------------------------------------------------
 // Serial / replay forward over segments of Ls steps from (su, sw) (triton_alif.py:46-71).
-template <int D>
+template <int D, bool NT>
 __global__ __launch_bounds__(64) void k_alif_fwd(const float* __restrict__ I,
                                                  const float* __restrict__ su,
                                                  const float* __restrict__ sw, float* __restrict__ U,
@@ -86,9 +86,9 @@ __global__ __launch_bounds__(64) void k_alif_fwd(const float* __restrict__ I,
       bool s;
       u = alif_step(u, w, xa[j], beta, rho, q, theta0, u_r, s);
       const size_t o = base + (size_t)(b * D + j) * N;
-      st_nt(U + o, u);
-      st_nt(W + o, w);
-      st_nt(S + o, s ? 1.0f : 0.0f);
+      st_out<NT>(U + o, u);
+      st_out<NT>(W + o, w);
+      st_out<NT>(S + o, s ? 1.0f : 0.0f);
     }
     if (more) {
 #pragma unroll
@@ -99,9 +99,9 @@ __global__ __launch_bounds__(64) void k_alif_fwd(const float* __restrict__ I,
     bool s;
     u = alif_step(u, w, Ip[(size_t)t * N], beta, rho, q, theta0, u_r, s);
     const size_t o = base + (size_t)t * N;
-    st_nt(U + o, u);
-    st_nt(W + o, w);
-    st_nt(S + o, s ? 1.0f : 0.0f);
+    st_out<NT>(U + o, u);
+    st_out<NT>(W + o, w);
+    st_out<NT>(S + o, s ? 1.0f : 0.0f);
   }
   if (eu) {
     eu[m * N + n] = u;
@@ -1164,6 +1164,7 @@ constexpr int ALIF_FPIPE_D = LSH_ALIF_FPIPE_D;
 // With mstar (the box scan's repair to convergence): the rows from chunk c0 on, c0 the least
 // mstar of the block's neurons, from the exact exits (eu, ew) of chunk c0 - 1 (which the replay
 // of the chunks below mstar wrote); rows before c0 C are left as they are.
+template <bool NT>
 __global__ __launch_bounds__(WAVE*(ALIF_PIPE_P + 1)) void k_alif_fwd_pipe(
     const float* __restrict__ I, const float* __restrict__ u0, const float* __restrict__ w0,
     float* __restrict__ U, float* __restrict__ W, float* __restrict__ S, int64_t N, int64_t T,
@@ -1262,9 +1263,9 @@ __global__ __launch_bounds__(WAVE*(ALIF_PIPE_P + 1)) void k_alif_fwd_pipe(
           const float2 o = sUW[buf][j][lane];
           const float2 pr = j == 0 ? sEntry[buf][lane] : sUW[buf][j - 1][lane];
           const bool sp = lif_v(pr.x, x2[r], beta) >= theta0 + pr.y;
-          st_row_nt(U + row, sb, o.x);
-          st_row_nt(W + row, sb, o.y);
-          st_row_nt(S + row, sb, sp ? 1.0f : 0.0f);
+          st_row<NT>(U + row, sb, o.x);
+          st_row<NT>(W + row, sb, o.y);
+          st_row<NT>(S + row, sb, sp ? 1.0f : 0.0f);
         }
       }
     }
@@ -1365,8 +1366,8 @@ __global__ __launch_bounds__(WAVE*(ALIF_PIPE_P + 1)) void k_alif_bwd_pipe(
           if (j < nr) {
             const float4 o = sOut[buf][j][lane];
             const size_t row = (size_t)(lo + j) * (size_t)N + (size_t)nb0;
-            if (WLW) st_row_nt(LW + row, sb, o.y);
-            st_row_nt(LV + row, sb, o.x);
+            if (WLW) st_row(LW + row, sb, o.y);
+            st_row(LV + row, sb, o.x);
             if constexpr (PS) acc.add(o.x, keep[0][r], o.y, keep[1][r], keep[2][r], keep[3][r], o.z);
           }
         }
@@ -1438,7 +1439,7 @@ __global__ __launch_bounds__(WAVE*(ALIF_PIPE_P + 1)) void k_alif_bwd_pipe(
 // and s_t are recomputed with the forward's own step (alif_step, reset value u_r) from that
 // entry state, which gives the stored bits when U, W, S come from one serial trajectory.  The
 // adjoint arithmetic is unchanged, so the outputs equal the stored-state variant's bit for bit.
-template <int C, int WV, bool WLW, bool PS, bool RC = false>
+template <int C, int WV, bool WLW, bool PS, bool RC = false, bool NT = true>
 __global__ __launch_bounds__(WAVE* WV) void k_alif_bwd_fused(
     const float* __restrict__ I, const float* __restrict__ u0, const float* __restrict__ w0,
     const float* __restrict__ U, const float* __restrict__ W, const float* __restrict__ S,
@@ -1561,8 +1562,8 @@ __global__ __launch_bounds__(WAVE* WV) void k_alif_bwd_fused(
         const float d = g[j] + q * lwv[j];
         lam = s1[j] * beta * lam + sg[j] * d;
         if (valid) {
-          if (WLW) bo.st_nt(sb, j * rstride, lwv[j]);
-          bv.st_nt(sb, j * rstride, lam);
+          if (WLW) bo.st<NT>(sb, j * rstride, lwv[j]);
+          bv.st<NT>(sb, j * rstride, lam);
         }
         if (PS) {
           cb = fmaf(lam, upv[j], cb);
@@ -1619,7 +1620,7 @@ constexpr int ALIF_LB_C = 16;
 constexpr int ALIF_LB_W = 8;
 constexpr int ALIF_LB_SEG = ALIF_LB_C * ALIF_LB_W;
 
-template <bool WLW, bool PS, bool RC = false>
+template <bool WLW, bool PS, bool RC = false, bool NT = true>
 __global__ __launch_bounds__(WAVE* ALIF_LB_W) void k_alif_bwd_lookback(
     const float* __restrict__ I, const float* __restrict__ u0, const float* __restrict__ w0,
     const float* __restrict__ U, const float* __restrict__ W, const float* __restrict__ S,
@@ -1789,8 +1790,8 @@ __global__ __launch_bounds__(WAVE* ALIF_LB_W) void k_alif_bwd_lookback(
       const float d = g[j] + q * lwv[j];
       lam = s1[j] * beta * lam + sg[j] * d;
       if (valid) {
-        if (WLW) bo.st_nt(sb, j * rstride, lwv[j]);
-        bv.st_nt(sb, j * rstride, lam);
+        if (WLW) bo.st<NT>(sb, j * rstride, lwv[j]);
+        bv.st<NT>(sb, j * rstride, lam);
       }
       if (PS) {
         cb = fmaf(lam, upv[j], cb);
@@ -1898,8 +1899,10 @@ static void launch_alif_fwd(const float* I, const float* su, const float* sw, fl
                             float beta, float rho, float q, float theta0, float u_r, hipStream_t st,
                             const float* dpar = nullptr, const int* mstar = nullptr) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  hipLaunchKernelGGL(k_alif_fwd<D>, dim3((unsigned)(M * NB)), dim3(WAVE), 0, st, I, su, sw, U, W, S,
-                     eu, ew, N, Ls, NB, beta, rho, q, theta0, u_r, dpar, mstar);
+  with_store_policy(N, [&](auto nt) {
+    hipLaunchKernelGGL((k_alif_fwd<D, decltype(nt)::value>), dim3((unsigned)(M * NB)), dim3(WAVE), 0, st,
+                       I, su, sw, U, W, S, eu, ew, N, Ls, NB, beta, rho, q, theta0, u_r, dpar, mstar);
+  });
 }
 
 }  // namespace lsh
@@ -1914,9 +1917,11 @@ extern "C" int lsh_alif_serial_fwd(const float* I, const float* u0, const float*
   if (T < 0 || N < 0 || N > (int64_t)1 << 31) return LSH_ERR_SHAPE;
   if (T == 0 || N == 0) return LSH_OK;
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  hipLaunchKernelGGL(k_alif_fwd_pipe, dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0,
-                     (hipStream_t)stream, I, u0, w0, U, W, S, N, T, beta, rho, q, theta0, u_r,
-                     nullptr, nullptr, nullptr, nullptr, 1);
+  with_store_policy(N, [&](auto nt) {
+    hipLaunchKernelGGL((k_alif_fwd_pipe<decltype(nt)::value>), dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0,
+                       (hipStream_t)stream, I, u0, w0, U, W, S, N, T, beta, rho, q, theta0, u_r,
+                       nullptr, nullptr, nullptr, nullptr, 1);
+  });
   LSH_CHECK_LAUNCH();
   return LSH_OK;
 }
@@ -1930,9 +1935,11 @@ extern "C" int lsh_alif_serial_fwd_dparams(const float* I, const float* u0, cons
   if (T < 0 || N < 0 || N > (int64_t)1 << 31) return LSH_ERR_SHAPE;
   if (T == 0 || N == 0) return LSH_OK;
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  hipLaunchKernelGGL(k_alif_fwd_pipe, dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0,
-                     (hipStream_t)stream, I, u0, w0, U, W, S, N, T, 0.0f, 0.0f, 0.0f, 0.0f, u_r,
-                     params, nullptr, nullptr, nullptr, 1);
+  with_store_policy(N, [&](auto nt) {
+    hipLaunchKernelGGL((k_alif_fwd_pipe<decltype(nt)::value>), dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0,
+                       (hipStream_t)stream, I, u0, w0, U, W, S, N, T, 0.0f, 0.0f, 0.0f, 0.0f, u_r,
+                       params, nullptr, nullptr, nullptr, 1);
+  });
   LSH_CHECK_LAUNCH();
   return LSH_OK;
 }
@@ -2035,9 +2042,11 @@ extern "C" int lsh_alif_scan_fwd(const float* I, const float* u0, const float* w
                       u_r, st, nullptr, chain ? Iq(L.MSTAR) : nullptr);
   mark(4);
   if (chain) {
-    hipLaunchKernelGGL(k_alif_fwd_pipe, dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0, st,
-                       I, u0, w0, U, W, S, N, T, beta, rho, q, theta0, u_r, nullptr, Iq(L.MSTAR),
-                       F(L.EU), F(L.EW), C);
+    with_store_policy(N, [&](auto nt) {
+      hipLaunchKernelGGL((k_alif_fwd_pipe<decltype(nt)::value>), dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0, st,
+                         I, u0, w0, U, W, S, N, T, beta, rho, q, theta0, u_r, nullptr, Iq(L.MSTAR),
+                         F(L.EU), F(L.EW), C);
+    });
   } else if (repair > 0 && M > 1) {
     const int64_t rounds = repair < (int64_t)M ? repair : (int64_t)M;
     hipLaunchKernelGGL(k_alif_repair, dim3((unsigned)NB), dim3(256), 0, st, I, U, W, S, F(L.SU),
@@ -2076,9 +2085,15 @@ static void launch_alif_fused_w(const float* I, const float* u0, const float* w0
                                 float* LV, float* DW0, double* partials, int64_t N, int M, int NB,
                                 float beta, float rho, float q, float theta0, float alpha,
                                 float u_r, hipStream_t st, const float* dpar) {
-  hipLaunchKernelGGL((k_alif_bwd_fused<C, W, WLW, PS, RC>), dim3((unsigned)NB), dim3(WAVE * W), 0, st,
-                     I, u0, w0, U, W_, S, GS, LW, LV, DW0, partials, N, M, beta, rho, q, theta0,
-                     alpha, u_r, dpar);
+  const auto launch = [&](auto nt) {
+    hipLaunchKernelGGL((k_alif_bwd_fused<C, W, WLW, PS, RC, decltype(nt)::value>), dim3((unsigned)NB),
+                       dim3(WAVE * W), 0, st, I, u0, w0, U, W_, S, GS, LW, LV, DW0, partials, N, M, beta,
+                       rho, q, theta0, alpha, u_r, dpar);
+  };
+  if constexpr (RC && !WLW)  // the layer's adjoint
+    with_store_policy(N, launch);
+  else
+    launch(std::true_type{});
 }
 
 // RC (recompute the states) keeps the stored-state variant's wave count, so both sum the
@@ -2136,10 +2151,18 @@ static void alif_lookback_launch(const float* I, const float* U, const float* W,
   hipLaunchKernelGGL(k_ws_header_reset, dim3(1), dim3(64), 0, st, hdr);
   fill_i32_launch(flags, 2 * (int64_t)NSEG * NB, 0, st);
   const bool wlw = LW != nullptr, ps = partials != nullptr;
-#define LSH_LB(WL, P)                                                                              \
-  hipLaunchKernelGGL((k_alif_bwd_lookback<WL, P, RC>), dim3((unsigned)((int64_t)NSEG * NB)),       \
+#define LSH_LB_NT(WL, P, NT)                                                                       \
+  hipLaunchKernelGGL((k_alif_bwd_lookback<WL, P, RC, NT>), dim3((unsigned)((int64_t)NSEG * NB)),   \
                      dim3(WAVE * ALIF_LB_W), 0, st, I, u0, w0, U, W, S, GS, LW, LV, DW0, partials,  \
                      agg, flags, hdr, N, NB, NSEG, beta, rho, q, theta0, alpha, u_r, dpar)
+#define LSH_LB(WL, P) LSH_LB_NT(WL, P, true)
+  if (RC && !wlw && !rows_aligned(N)) {  // the layer's adjoint
+    if (ps)
+      LSH_LB_NT(false, true, false);
+    else
+      LSH_LB_NT(false, false, false);
+    return;
+  }
   if (wlw && ps)
     LSH_LB(true, true);
   else if (wlw)
@@ -2149,6 +2172,7 @@ static void alif_lookback_launch(const float* I, const float* U, const float* W,
   else
     LSH_LB(false, false);
 #undef LSH_LB
+#undef LSH_LB_NT
 }
 
 static int alif_bwd(const float* I, const float* U, const float* W, const float* S,

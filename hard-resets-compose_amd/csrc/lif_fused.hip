@@ -38,7 +38,7 @@ __device__ __forceinline__ bool lds_wait(int* flag, int want) {
 // SO (starts only): U is [M, N] and receives each chunk's exact entry state instead of the
 // trajectory, S as usual; the adjoint recomputes the trajectory from those states
 // (k_lif_bwd_fused<..., RC = true>), so the forward writes 4 B per neuron-step instead of 8.
-template <int KMAX, int C, int W, bool SPEC, bool SO = false>
+template <int KMAX, int C, int W, bool SPEC, bool SO = false, bool NT = true>
 __global__ __launch_bounds__(WAVE* W) void k_lif_fwd_fused(const float* __restrict__ I,
                                                            const float* __restrict__ u0,
                                                            float* __restrict__ U,
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_fwd_fused(const float* __restri
         for (int j = 0; j < C; ++j) {
           bool s;
           u = lif_step(u, x[j], beta, theta, u_r, s);
-          bs.st_nt(sb, j * rstride, s ? 1.0f : 0.0f);
+          bs.st<NT>(sb, j * rstride, s ? 1.0f : 0.0f);
         }
       } else if (valid) {
         const Buf bu(Ub + row0 * N), bs(Sb + row0 * N);
@@ -181,8 +181,8 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_fwd_fused(const float* __restri
         for (int j = 0; j < C; ++j) {
           bool s;
           u = lif_step(u, x[j], beta, theta, u_r, s);
-          bu.st_nt(sb, j * rstride, u);
-          bs.st_nt(sb, j * rstride, s ? 1.0f : 0.0f);
+          bu.st<NT>(sb, j * rstride, u);
+          bs.st<NT>(sb, j * rstride, s ? 1.0f : 0.0f);
         }
       }
     }
@@ -215,7 +215,7 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_fwd_fused(const float* __restri
 // SO forward and S is not read; the wave replays its chunk's forward from the entry state in
 // registers (the forward's own arithmetic, so u_{t-1} and s_t are the forward's bits) while it
 // forms the coefficients: 8 B read per neuron-step instead of 16.
-template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0, bool RC = false>
+template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0, bool RC = false, bool NT = true>
 __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_fused(
     const float* __restrict__ I, const float* __restrict__ u0, const float* __restrict__ U,
     const float* __restrict__ S, const float* __restrict__ GS, const float* __restrict__ GU,
@@ -318,7 +318,7 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_fused(
         else
           lam = b[j] + a[j] * lam;
         if (valid) {
-          bl.st_nt(sb, j * rstride, lam);
+          bl.st<NT>(sb, j * rstride, lam);
           if (PS) {
             acc_b += (double)lam * (double)upk[j];
             if ((sbits >> j) & 1ull) {
@@ -368,8 +368,14 @@ static void launch_fwd_fused(const float* I, const float* u0, float* U, float* S
                              int64_t N, int M, int K, float beta, float theta, float u_r,
                              hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  hipLaunchKernelGGL((k_lif_fwd_fused<KMAX, C, W, SPEC, SO>), dim3((unsigned)NB), dim3(WAVE * W), 0,
-                     st, I, u0, U, S, h, N, M, K, beta, theta, u_r);
+  const auto launch = [&](auto nt) {
+    hipLaunchKernelGGL((k_lif_fwd_fused<KMAX, C, W, SPEC, SO, decltype(nt)::value>), dim3((unsigned)NB),
+                       dim3(WAVE * W), 0, st, I, u0, U, S, h, N, M, K, beta, theta, u_r);
+  };
+  if constexpr (SPEC)
+    launch(std::true_type{});
+  else
+    with_store_policy(N, launch);
 }
 
 // The chunked-serial exact forward (no maps) writing S and the chunk entry states only.
@@ -442,8 +448,15 @@ static void launch_bwd_fused(const float* I, const float* u0, const float* U, co
                              const float* GS, const float* GU, float* Lam, int64_t N, int M,
                              float beta, float theta, float u_r, float alpha, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  hipLaunchKernelGGL((k_lif_bwd_fused<C, W, DETACH, HAS_GU>), dim3((unsigned)NB), dim3(WAVE * W), 0,
-                     st, I, u0, U, S, GS, GU, Lam, nullptr, N, M, beta, theta, u_r, alpha);
+  const auto launch = [&](auto nt) {
+    hipLaunchKernelGGL((k_lif_bwd_fused<C, W, DETACH, HAS_GU, 0, false, decltype(nt)::value>),
+                       dim3((unsigned)NB), dim3(WAVE * W), 0, st, I, u0, U, S, GS, GU, Lam, nullptr, N, M,
+                       beta, theta, u_r, alpha);
+  };
+  if constexpr (DETACH && !HAS_GU)
+    with_store_policy(N, launch);
+  else
+    launch(std::true_type{});
 }
 
 template <int C, int W>
@@ -493,14 +506,17 @@ static void launch_bwd_rc(const float* I, const float* STARTS, const float* GS, 
                           double* partials, int64_t N, int M, float beta, float theta, float u_r,
                           float alpha, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  if (partials)
-    hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 1, true>), dim3((unsigned)NB),
-                       dim3(WAVE * W), 0, st, I, STARTS, STARTS, nullptr, GS, nullptr, Lam, partials,
-                       N, M, beta, theta, u_r, alpha);
-  else
-    hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 0, true>), dim3((unsigned)NB),
-                       dim3(WAVE * W), 0, st, I, STARTS, STARTS, nullptr, GS, nullptr, Lam, nullptr,
-                       N, M, beta, theta, u_r, alpha);
+  with_store_policy(N, [&](auto nt) {
+    constexpr bool NT = decltype(nt)::value;
+    if (partials)
+      hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 1, true, NT>), dim3((unsigned)NB),
+                         dim3(WAVE * W), 0, st, I, STARTS, STARTS, nullptr, GS, nullptr, Lam, partials,
+                         N, M, beta, theta, u_r, alpha);
+    else
+      hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 0, true, NT>), dim3((unsigned)NB),
+                         dim3(WAVE * W), 0, st, I, STARTS, STARTS, nullptr, GS, nullptr, Lam, nullptr,
+                         N, M, beta, theta, u_r, alpha);
+  });
 }
 
 template <int C>
@@ -532,12 +548,17 @@ static void launch_param_fused(const float* I, const float* u0, const float* U, 
                                float beta, float theta, float u_r, float alpha, int ps,
                                hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  if (ps == 2)
-    hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 2>), dim3((unsigned)NB), dim3(WAVE * W), 0,
-                       st, I, u0, U, S, GS, nullptr, Lam, partials, N, M, beta, theta, u_r, alpha);
-  else
-    hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 1>), dim3((unsigned)NB), dim3(WAVE * W), 0,
-                       st, I, u0, U, S, GS, nullptr, Lam, partials, N, M, beta, theta, u_r, alpha);
+  with_store_policy(N, [&](auto nt) {
+    constexpr bool NT = decltype(nt)::value;
+    if (ps == 2)
+      hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 2, false, NT>), dim3((unsigned)NB),
+                         dim3(WAVE * W), 0, st, I, u0, U, S, GS, nullptr, Lam, partials, N, M, beta,
+                         theta, u_r, alpha);
+    else
+      hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 1, false, NT>), dim3((unsigned)NB),
+                         dim3(WAVE * W), 0, st, I, u0, U, S, GS, nullptr, Lam, partials, N, M, beta,
+                         theta, u_r, alpha);
+  });
 }
 
 template <int C>

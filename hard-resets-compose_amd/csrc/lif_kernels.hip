@@ -37,7 +37,7 @@ __global__ void k_ws_header_reset(WsHeader* h) {
 constexpr int kFbRows = 32;
 // done (or null): one flag per (chunk, 64-neuron block), set where the carry has already
 // replayed the block's chunk from its start (U, S and the end written); those blocks return.
-template <int D>
+template <int D, bool NT>
 __global__ __launch_bounds__(64) void k_lif_fwd(const float* __restrict__ I,
                                                 const float* __restrict__ starts,
                                                 float* __restrict__ U, float* __restrict__ S,
@@ -74,8 +74,8 @@ __global__ __launch_bounds__(64) void k_lif_fwd(const float* __restrict__ I,
     for (int j = 0; j < D; ++j) {
       bool s;
       u = lif_step(u, xa[j], beta, theta, u_r, s);
-      st_nt(Ub + (size_t)j * N, u);
-      st_nt(Sb + (size_t)j * N, s ? 1.0f : 0.0f);
+      st_out<NT>(Ub + (size_t)j * N, u);
+      st_out<NT>(Sb + (size_t)j * N, s ? 1.0f : 0.0f);
     }
     if (more) {
 #pragma unroll
@@ -85,8 +85,8 @@ __global__ __launch_bounds__(64) void k_lif_fwd(const float* __restrict__ I,
   for (int64_t t = nt * D; t < Ls; ++t) {
     bool s;
     u = lif_step(u, Ip[(size_t)t * N], beta, theta, u_r, s);
-    st_nt(Up + (size_t)t * N, u);
-    st_nt(Sp + (size_t)t * N, s ? 1.0f : 0.0f);
+    st_out<NT>(Up + (size_t)t * N, u);
+    st_out<NT>(Sp + (size_t)t * N, s ? 1.0f : 0.0f);
   }
   if (ends) ends[m * N + n] = u;
 }
@@ -1040,8 +1040,10 @@ static void launch_fwd(const float* I, const float* starts, float* U, float* S, 
                        int64_t N, int64_t Ls, int64_t M, float beta, float theta, float u_r,
                        hipStream_t st, const int* done = nullptr) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  hipLaunchKernelGGL(k_lif_fwd<D>, dim3((unsigned)(M * NB)), dim3(WAVE), 0, st, I, starts, U, S,
-                     ends, N, Ls, NB, beta, theta, u_r, done);
+  with_store_policy(N, [&](auto nt) {
+    hipLaunchKernelGGL((k_lif_fwd<D, decltype(nt)::value>), dim3((unsigned)(M * NB)), dim3(WAVE), 0, st,
+                       I, starts, U, S, ends, N, Ls, NB, beta, theta, u_r, done);
+  });
 }
 
 static void launch_fwd_auto(const float* I, const float* starts, float* U, float* S, float* ends,

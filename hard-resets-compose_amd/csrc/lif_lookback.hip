@@ -45,7 +45,7 @@ void fill_i32_launch(int* p, int64_t n, int v, hipStream_t st) {
 // end of time and adds nothing to the sums; its loads read the chunk's last row, its store is
 // left out.  Its own instantiation, since the tests cost the whole-segment kernel 2 % (N 1024,
 // T 2^18: 0.94 ms).
-template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0, bool RAG = false>
+template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0, bool RAG = false, bool NT = true>
 __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
     const float* __restrict__ I, const float* __restrict__ u0, const float* __restrict__ U,
     const float* __restrict__ S, const float* __restrict__ GS, const float* __restrict__ GU,
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
     else
       lam = b[j] + a[j] * lam;
     if (valid && (!RAG || j < rows)) {
-      bl.st_nt(sb, j * rstride, lam);
+      bl.st<NT>(sb, j * rstride, lam);
       if (PS) {
         acc_b += (double)lam * (double)upk[j];
         if ((sbits >> j) & 1ull) {
@@ -248,10 +248,17 @@ static void launch_lookback(const float* I, const float* u0, const float* U, con
                        aggP, aggQ, incl, flags, reinterpret_cast<WsHeader*>(ws), partials, T, N, NB,
                        NSEG, beta, theta, u_r, alpha);
   };
-  if (T % kLookbackSeg == 0)
-    launch(k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS, false>);
+  const auto by_length = [&](auto nt) {
+    constexpr bool NT = decltype(nt)::value;
+    if (T % kLookbackSeg == 0)
+      launch(k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS, false, NT>);
+    else
+      launch(k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS, true, NT>);
+  };
+  if constexpr (C == 16 && DETACH && !HAS_GU)
+    with_store_policy(N, by_length);
   else
-    launch(k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS, true>);
+    by_length(std::true_type{});
 }
 
 template <int C, int W>

@@ -37,6 +37,7 @@ namespace lsh {
 constexpr int WARM_D = 16;
 
 // T need not be a multiple of C: the last chunk is short.
+template <bool NT>
 __global__ __launch_bounds__(64) void k_lif_fwd_warm(const float* __restrict__ I,
                                                      const float* __restrict__ u0,
                                                      float* __restrict__ U, float* __restrict__ S,
@@ -65,8 +66,8 @@ __global__ __launch_bounds__(64) void k_lif_fwd_warm(const float* __restrict__ I
   stream_rows<WARM_D>(Ip, (size_t)N, min<int64_t>(C, T - t0), [&](int64_t j, float x) {
     bool s;
     u = lif_step(u, x, beta, theta, u_r, s);
-    st_nt(Up + (size_t)j * N, u);
-    st_nt(Sp + (size_t)j * N, s ? 1.0f : 0.0f);
+    st_out<NT>(Up + (size_t)j * N, u);
+    st_out<NT>(Sp + (size_t)j * N, s ? 1.0f : 0.0f);
   });
   ends[(size_t)m * N + n] = u;
 }
@@ -164,8 +165,10 @@ static int warm_run(const float* I, const float* u0, float* U, float* S, int64_t
   const int NB = (int)((N + WAVE - 1) / WAVE);
   float* starts = reinterpret_cast<float*>(w + L.STARTS);
   float* ends = reinterpret_cast<float*>(w + L.ENDS);
-  hipLaunchKernelGGL(k_lif_fwd_warm, dim3((unsigned)((int64_t)M * NB)), dim3(WAVE), 0, st, I, u0, U, S,
+  with_store_policy(N, [&](auto nt) {
+    hipLaunchKernelGGL((k_lif_fwd_warm<decltype(nt)::value>), dim3((unsigned)((int64_t)M * NB)), dim3(WAVE), 0, st, I, u0, U, S,
                      starts, ends, T, N, C, W, NB, beta, theta, u_r);
+  });
   // The per-block repair counts the missed predictions, so count them here first (the wide
   // round fixes most of them before that repair looks).
   if (M > 1) {

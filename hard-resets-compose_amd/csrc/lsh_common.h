@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 namespace lsh {
@@ -123,14 +125,38 @@ __device__ __forceinline__ void st_nt(T* p, T v) { __builtin_nontemporal_store(v
 template <typename T>
 __device__ __forceinline__ T ld_nt(const T* p) { return __builtin_nontemporal_load(p); }
 
+// The policy of a streaming output's stores by the rows' alignment.  Rows of whole 64-byte pieces
+// (N % 16 == 0) are written non-temporally; otherwise neighbouring waves share a piece at either
+// end of each row, and a non-temporal store writes its part through by itself where a plain one
+// waits in L2 for the rest.  Measured, non-temporal -> plain: N 14083, T 1000 serial forward 60 ->
+// 45 us; N 51453, T 512 136 -> 94 us, its spikes and entry states 90 -> 58, recomputing adjoint 115
+// -> 85; but N 12800, T 1000 27 -> 32 us, N 65536, T 4096 406 -> 423 us.
+inline bool rows_aligned(int64_t N) { return N % 16 == 0; }
+// f(std::true_type) for non-temporal stores, f(std::false_type) for plain ones
+template <class F>
+inline void with_store_policy(int64_t N, F&& f) {
+  if (rows_aligned(N))
+    f(std::true_type{});
+  else
+    f(std::false_type{});
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void st_out(T* p, T v) {
+  if constexpr (NT)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
+}
+
 // Row access with a wave-uniform row pointer and a 32-bit per-lane byte offset, so the
 // compiler can address with an SGPR base + VGPR offset instead of a 64-bit VGPR pair per
 // access (fewer VGPRs and address instructions in the unrolled time loops).
 __device__ __forceinline__ float ld_row(const float* __restrict__ row, unsigned boff) {
   return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(row) + boff);
 }
-__device__ __forceinline__ void st_row_nt(float* __restrict__ row, unsigned boff, float v) {
-  __builtin_nontemporal_store(v, reinterpret_cast<float*>(reinterpret_cast<char*>(row) + boff));
+template <bool NT = true>
+__device__ __forceinline__ void st_row(float* __restrict__ row, unsigned boff, float v) {
+  st_out<NT>(reinterpret_cast<float*>(reinterpret_cast<char*>(row) + boff), v);
 }
 
 // Raw buffer access (CDNA3/4): a 128-bit SGPR descriptor for a wave-uniform base address,
@@ -153,9 +179,10 @@ struct Buf {
   __device__ __forceinline__ float ld(unsigned voff, unsigned soff) const {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, LSH_LD_POLICY));
   }
-  // non-temporal store (cache policy bit 1 = nt on gfx94x/gfx950)
-  __device__ __forceinline__ void st_nt(unsigned voff, unsigned soff, float v) const {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, voff, soff, 2);
+  // cache policy bit 1 = nt on gfx94x/gfx950
+  template <bool NT = true>
+  __device__ __forceinline__ void st(unsigned voff, unsigned soff, float v) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, voff, soff, NT ? 2 : 0);
   }
 };
 

@@ -50,7 +50,7 @@ __device__ __forceinline__ int pipe_tile_rows(int64_t T, int64_t k) {
 // serial_bwd_kernel, :1088-1135 bwd_tiled_pf_kernel): tiles from the end of time, coefficients
 // as k_lif_bwd's (v = fl(fl(beta*u_{t-1}) + x_t), sg = surrogate'(v - theta), J = 1 - s_t
 // (+ (u_r - v)*sg when the reset is not detached), a = beta*J, b = gs*sg + J*gu).
-template <bool DETACH, bool HAS_GU>
+template <bool DETACH, bool HAS_GU, bool NT>
 __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_bwd_pipe(
     const float* __restrict__ I, const float* __restrict__ u0, const float* __restrict__ U,
     const float* __restrict__ S, const float* __restrict__ GS, const float* __restrict__ GU,
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_bwd_pipe(
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int j = p + r * P;
-        if (j < nr) st_row_nt(Lam + (size_t)(lo + j) * (size_t)N + (size_t)nb0, sb, sL[buf][j][lane]);
+        if (j < nr) st_row<NT>(Lam + (size_t)(lo + j) * (size_t)N + (size_t)nb0, sb, sL[buf][j][lane]);
       }
     }
     __syncthreads();
@@ -188,7 +188,7 @@ struct AffStep {
 // tile ahead and store U, S of the tile finished one round earlier, recomputing each spike
 // from the state before it and their own loaded rows (kept two rounds in registers) with the
 // step's operations, so the consumer's chain carries no spike-to-float select.
-template <class Step>
+template <class Step, bool NT>
 __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
     const float* __restrict__ I, const float* __restrict__ u0, float* __restrict__ U,
     float* __restrict__ S, int64_t N, int64_t T, Step step) {
@@ -279,8 +279,8 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
           const size_t row = (size_t)((k - 2) * D + j) * (size_t)N + (size_t)nb0;
           const float u = sU[buf][j][lane];
           const float up = j == 0 ? sEntry[buf][lane] : sU[buf][j - 1][lane];
-          st_row_nt(U + row, sb, u);
-          st_row_nt(S + row, sb, step.spike(up, x2[r]) ? 1.0f : 0.0f);
+          st_row<NT>(U + row, sb, u);
+          st_row<NT>(S + row, sb, step.spike(up, x2[r]) ? 1.0f : 0.0f);
         }
       }
     }
@@ -296,15 +296,20 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
 void lif_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, int64_t N, int64_t T,
                          float beta, float theta, float u_r, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  hipLaunchKernelGGL((k_serial_fwd_pipe<LifStep>), dim3((unsigned)NB), dim3(WAVE * (PIPE_P + 1)), 0,
-                     st, I, u0, U, S, N, T, LifStep{beta, theta, u_r});
+  with_store_policy(N, [&](auto nt) {
+    hipLaunchKernelGGL((k_serial_fwd_pipe<LifStep, decltype(nt)::value>), dim3((unsigned)NB),
+                       dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, U, S, N, T, LifStep{beta, theta, u_r});
+  });
 }
 
 void aff_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, int64_t N, int64_t T,
                          float beta, float theta, float gamma, float delta, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  hipLaunchKernelGGL((k_serial_fwd_pipe<AffStep>), dim3((unsigned)NB), dim3(WAVE * (PIPE_P + 1)), 0,
-                     st, I, u0, U, S, N, T, AffStep{beta, theta, gamma, delta});
+  with_store_policy(N, [&](auto nt) {
+    hipLaunchKernelGGL((k_serial_fwd_pipe<AffStep, decltype(nt)::value>), dim3((unsigned)NB),
+                       dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, U, S, N, T,
+                       AffStep{beta, theta, gamma, delta});
+  });
 }
 
 template <bool DETACH, bool HAS_GU>
@@ -312,8 +317,11 @@ static void launch_lif_bwd_pipe(const float* I, const float* u0, const float* U,
                                 const float* GS, const float* GU, float* Lam, int64_t N, int64_t T,
                                 float beta, float theta, float u_r, float alpha, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  hipLaunchKernelGGL((k_lif_bwd_pipe<DETACH, HAS_GU>), dim3((unsigned)NB), dim3(WAVE * (PIPE_P + 1)),
-                     0, st, I, u0, U, S, GS, GU, Lam, N, T, beta, theta, u_r, alpha);
+  with_store_policy(N, [&](auto nt) {
+    hipLaunchKernelGGL((k_lif_bwd_pipe<DETACH, HAS_GU, decltype(nt)::value>), dim3((unsigned)NB),
+                       dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, U, S, GS, GU, Lam, N, T, beta, theta,
+                       u_r, alpha);
+  });
 }
 
 void lif_serial_bwd_pipe(const float* I, const float* u0, const float* U, const float* S,

@@ -111,3 +111,38 @@ def test_warm_any_plan_and_auto_layer(dev):
     db, = torch.autograd.grad(S, [b], gpu(GS, dev))
     up = np.concatenate([u0[None], Uo[:-1]]).astype(np.float64)
     assert rel(db.item(), (want * up).sum()) < 1e-4
+
+
+@pytest.mark.parametrize("N", [15, 16, 48, 49, 80, 129])
+def test_row_alignment_store_policies(dev, N):
+    """Both store policies (N % 16) of the serial sweeps, the recomputing pair, the replay and the
+    ALIF layer: the oracle's bits and adjoints."""
+    from lifscan import hip_lif as L
+    from lifscan import triton_alif as A
+    from oracle import alif_oracle as AO
+    T = 160
+    I, GS, u0 = normal(T, N, 0.15, 0.4, N), normal(T, N, 0.0, 1.0, N + 1), uniform(N, 0.0, 1.0, 3)
+    Ig, Gg, ug = gpu(I, dev), gpu(GS, dev), gpu(u0, dev)
+    Uo, So = O.serial_forward(I, 0.95, 1.0, 0.0, u0)
+    want = O.serial_backward(I, u0, Uo, So, GS, None, 0.95, 1.0, 0.0, 4.0, True, dtype=np.float64)
+    U, S = L.serial_forward(Ig, 0.95, 1.0, 0.0, ug)
+    assert np.array_equal(host(U), Uo) and np.array_equal(host(S), So)
+    S2, ST = L.scan_forward_exact_starts(Ig, 0.95, 1.0, 0.0, ug)
+    assert np.array_equal(host(S2), So)
+    lams = [L.serial_backward(Ig, ug, U, S, Gg, None, 0.95, 1.0, 0.0),
+            L.scan_backward_fused_starts(Ig, ST, Gg, 0.95, 1.0, 0.0)[0],
+            L.scan_backward_fused(Ig, ug, U, S, Gg, None, 0.95, 1.0, 0.0),
+            L._lookback(Ig, ug, U, S, Gg, None, 0.95, 1.0, 0.0, 4.0, True)]
+    for lam in lams:
+        assert rel(host(lam), want) < 1e-6
+    U3, S3 = L.scan_forward_mapscan(Ig, 0.95, 1.0, 0.0, ug, C=32, K=16, repair=10 ** 6)
+    assert np.array_equal(host(U3), Uo) and np.array_equal(host(S3), So)
+    w0 = np.zeros(N, np.float32)
+    Ua, Wa, Sa = AO.serial_forward(I, 0.95, 0.995, 0.2, 1.0, 0.0, u0, w0)
+    leaf = Ig.clone().requires_grad_(True)
+    ps = [torch.tensor(v, device=dev, requires_grad=True) for v in (0.95, 0.995, 0.2, 1.0)]
+    s, u, w = A.alif(leaf, ug, gpu(w0, dev), *ps)
+    assert np.array_equal(host(s), Sa) and np.array_equal(host(u), Ua) and np.array_equal(host(w), Wa)
+    dI, = torch.autograd.grad(s, [leaf], Gg)
+    LV, _ = A.alif_backward(Ig, u, w, s, Gg, 0.95, 0.995, 0.2, 1.0, ug, gpu(w0, dev), mode="serial")
+    assert rel(host(dI), host(LV)) < 1e-6
