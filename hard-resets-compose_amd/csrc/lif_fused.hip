@@ -36,15 +36,18 @@ __device__ __forceinline__ bool lds_wait(int* flag, int want) {
 }
 
 // SO (starts only): U is [M, N] and receives each chunk's exact entry state instead of the
-// trajectory, S as usual; the adjoint recomputes the trajectory from those states
+// trajectory (NULL: not wanted), S as usual; the adjoint recomputes the trajectory from those states
 // (k_lif_bwd_fused<..., RC = true>), so the forward writes 4 B per neuron-step instead of 8.
-template <int KMAX, int C, int W, bool SPEC, bool SO = false, bool NT = true>
+// RAG: T is no multiple of C and the last chunk (m = M - 1) is short; its steps past T read its last
+// row and store nothing.  Its own instantiation, as the look-back adjoint's.
+template <int KMAX, int C, int W, bool SPEC, bool SO = false, bool NT = true, bool RAG = false>
 __global__ __launch_bounds__(WAVE* W) void k_lif_fwd_fused(const float* __restrict__ I,
                                                            const float* __restrict__ u0,
                                                            float* __restrict__ U,
                                                            float* __restrict__ S, WsHeader* hdr,
-                                                           int64_t N, int M, int K, float beta,
-                                                           float theta, float u_r) {
+                                                           int64_t T, int64_t N, int M, int K,
+                                                           float beta, float theta, float u_r) {
+  static_assert(!RAG || (SO && !SPEC), "a short last chunk: the starts-only forward");
   constexpr int KL = SPEC ? KMAX : 1;
   __shared__ float sA[W][WAVE], sB[W][WAVE];
   __shared__ float sXd[W][KL][WAVE], sCd[W][KL][WAVE];
@@ -75,10 +78,14 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_fwd_fused(const float* __restri
   // Without speculation the round's inputs are loaded one round ahead (xn), so the loads of
   // round r+1 are in flight during round r's hand-off chain (barriers wait on LDS only).
   float x[C], xn[SPEC ? 1 : C];
+  const auto rows_of = [&](int m) {  // rows of chunk m < M
+    return !RAG || m + 1 < M ? C : (int)(T - (int64_t)m * C);
+  };
   if (!SPEC && w < M) {
     const Buf bi(Ib + (size_t)w * C * N);
+    const int rows = rows_of(w);
 #pragma unroll
-    for (int j = 0; j < C; ++j) x[j] = bi.ld(lb, j * rstride);
+    for (int j = 0; j < C; ++j) x[j] = bi.ld(lb, (!RAG || j < rows ? j : rows - 1) * rstride);
   }
   for (int r = 0; r < rounds; ++r) {
     const int m = r * W + w;
@@ -86,8 +93,9 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_fwd_fused(const float* __restri
     const size_t row0 = (size_t)m * C;
     if (!SPEC && m + W < M) {
       const Buf bn(Ib + (row0 + (size_t)W * C) * N);
+      const int rows = rows_of(m + W);
 #pragma unroll
-      for (int j = 0; j < C; ++j) xn[j] = bn.ld(lb, j * rstride);
+      for (int j = 0; j < C; ++j) xn[j] = bn.ld(lb, (!RAG || j < rows ? j : rows - 1) * rstride);
     }
     if (active) {
       if (SPEC) {
@@ -165,14 +173,15 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_fwd_fused(const float* __restri
       unknown += (SPEC && !known && valid) ? 1ull : 0ull;
       // (4) the stored trajectory, from the exact entry
       if (valid && SO) {
-        U[(size_t)m * N + nb0 + lane] = start;
+        if (U != nullptr) U[(size_t)m * N + nb0 + lane] = start;
         const Buf bs(Sb + row0 * N);
+        const int rows = rows_of(m);
         float u = start;
 #pragma unroll
         for (int j = 0; j < C; ++j) {
           bool s;
           u = lif_step(u, x[j], beta, theta, u_r, s);
-          bs.st<NT>(sb, j * rstride, s ? 1.0f : 0.0f);
+          if (!RAG || j < rows) bs.st<NT>(sb, j * rstride, s ? 1.0f : 0.0f);
         }
       } else if (valid) {
         const Buf bu(Ub + row0 * N), bs(Sb + row0 * N);
@@ -215,12 +224,16 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_fwd_fused(const float* __restri
 // SO forward and S is not read; the wave replays its chunk's forward from the entry state in
 // registers (the forward's own arithmetic, so u_{t-1} and s_t are the forward's bits) while it
 // forms the coefficients: 8 B read per neuron-step instead of 16.
-template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0, bool RC = false, bool NT = true>
+// RAG: T is no multiple of C and the last chunk is short; its steps past T have a = b = 0 (lam = 0 at
+// the end of time, nothing added to the sums), read its last row and store nothing.
+template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0, bool RC = false, bool NT = true,
+          bool RAG = false>
 __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_fused(
     const float* __restrict__ I, const float* __restrict__ u0, const float* __restrict__ U,
     const float* __restrict__ S, const float* __restrict__ GS, const float* __restrict__ GU,
-    float* __restrict__ Lam, double* __restrict__ partials, int64_t N, int M, float beta,
+    float* __restrict__ Lam, double* __restrict__ partials, int64_t T, int64_t N, int M, float beta,
     float theta, float u_r, float alpha) {
+  static_assert(!RAG || RC, "a short last chunk: the recomputing adjoint");
   static_assert(!PS || (DETACH && !HAS_GU && C <= 64), "parameter sums: detached, no GU");
   static_assert(!RC || (DETACH && !HAS_GU && PS != 2), "recompute: hard reset, detached, no GU");
   constexpr bool AFF = PS == 2;
@@ -255,6 +268,7 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_fused(
     float lam = 0.0f;
     const size_t row0 = (size_t)(active ? m : 0) * C;
     const unsigned rstride = (unsigned)(N * 4);
+    const int rows = !RAG || m + 1 < M ? C : (int)(T - (int64_t)row0);
     if (active) {
       const Buf bi(Ib + row0 * N), bs_(Sb + row0 * N), bg(Gb + row0 * N), bp(Ub + row0 * N);
       // state before the chunk's first step: the previous chunk's last U row, or u0 (RC: the
@@ -264,7 +278,8 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_fused(
       float ur = up0;  // RC: the recomputed state
 #pragma unroll
       for (int j = 0; j < C; ++j) {
-        const unsigned so = j * rstride;
+        const bool in = !RAG || j < rows;
+        const unsigned so = (in ? j : rows - 1) * rstride;
         const float x = bi.ld(lb, so);
         float s, up;
         if constexpr (RC) {
@@ -281,11 +296,12 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_fused(
         const float sg = surrogate(v, theta, alpha);
         float J = 1.0f - s;
         if (!DETACH) J = J + (u_r - v) * sg;
-        if constexpr (!AFF) a[j] = beta * J;
+        if constexpr (!AFF) a[j] = in ? beta * J : 0.0f;
         b[j] = HAS_GU ? gs * sg + J * Buf(Hb + row0 * N).ld(lb, so) : gs * sg;
+        if (!in) b[j] = 0.0f;
         if (PS) {
           upk[j] = up;
-          if (s != 0.0f) sbits |= 1ull << j;
+          if (s != 0.0f && in) sbits |= 1ull << j;
           if (PS == 1 && valid) acc_t += (double)b[j];
           if constexpr (AFF) vpk[j] = v;
         }
@@ -317,7 +333,7 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_fused(
           lam = b[j] + (((sbits >> j) & 1ull) ? gbeta : beta) * lam;
         else
           lam = b[j] + a[j] * lam;
-        if (valid) {
+        if (valid && (!RAG || j < rows)) {
           bl.st<NT>(sb, j * rstride, lam);
           if (PS) {
             acc_b += (double)lam * (double)upk[j];
@@ -368,14 +384,33 @@ static void launch_fwd_fused(const float* I, const float* u0, float* U, float* S
                              int64_t N, int M, int K, float beta, float theta, float u_r,
                              hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
+  const int64_t T = (int64_t)M * C;
   const auto launch = [&](auto nt) {
     hipLaunchKernelGGL((k_lif_fwd_fused<KMAX, C, W, SPEC, SO, decltype(nt)::value>), dim3((unsigned)NB),
-                       dim3(WAVE * W), 0, st, I, u0, U, S, h, N, M, K, beta, theta, u_r);
+                       dim3(WAVE * W), 0, st, I, u0, U, S, h, T, N, M, K, beta, theta, u_r);
   };
   if constexpr (SPEC)
     launch(std::true_type{});
   else
     with_store_policy(N, launch);
+}
+
+// The starts-only forward of any T with chunks of 32 (STARTS may be NULL).
+template <int W>
+static void launch_fwd_starts_any(const float* I, const float* u0, float* STARTS, float* S, WsHeader* h,
+                                  int64_t T, int64_t N, float beta, float theta, float u_r,
+                                  hipStream_t st) {
+  const int NB = (int)((N + WAVE - 1) / WAVE);
+  const int M = (int)((T + 31) / 32);
+  with_store_policy(N, [&](auto nt) {
+    constexpr bool NT = decltype(nt)::value;
+    const auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)NB), dim3(WAVE * W), 0, st, I, u0, STARTS, S, h, T, N, M,
+                         1, beta, theta, u_r);
+    };
+    T % 32 == 0 ? launch(k_lif_fwd_fused<1, 32, W, false, true, NT>)
+                : launch(k_lif_fwd_fused<1, 32, W, false, true, NT, true>);
+  });
 }
 
 // The chunked-serial exact forward (no maps) writing S and the chunk entry states only.
@@ -450,8 +485,8 @@ static void launch_bwd_fused(const float* I, const float* u0, const float* U, co
   const int NB = (int)((N + WAVE - 1) / WAVE);
   const auto launch = [&](auto nt) {
     hipLaunchKernelGGL((k_lif_bwd_fused<C, W, DETACH, HAS_GU, 0, false, decltype(nt)::value>),
-                       dim3((unsigned)NB), dim3(WAVE * W), 0, st, I, u0, U, S, GS, GU, Lam, nullptr, N, M,
-                       beta, theta, u_r, alpha);
+                       dim3((unsigned)NB), dim3(WAVE * W), 0, st, I, u0, U, S, GS, GU, Lam, nullptr,
+                       (int64_t)M * C, N, M, beta, theta, u_r, alpha);
   };
   if constexpr (DETACH && !HAS_GU)
     with_store_policy(N, launch);
@@ -503,25 +538,31 @@ static void bwd_fused_c(const float* I, const float* u0, const float* U, const f
 // fit.py parameter sums.
 template <int C, int W>
 static void launch_bwd_rc(const float* I, const float* STARTS, const float* GS, float* Lam,
-                          double* partials, int64_t N, int M, float beta, float theta, float u_r,
-                          float alpha, hipStream_t st) {
+                          double* partials, int64_t T, int64_t N, int M, float beta, float theta,
+                          float u_r, float alpha, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
+  const bool rag = T != (int64_t)M * C;
   with_store_policy(N, [&](auto nt) {
     constexpr bool NT = decltype(nt)::value;
-    if (partials)
-      hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 1, true, NT>), dim3((unsigned)NB),
-                         dim3(WAVE * W), 0, st, I, STARTS, STARTS, nullptr, GS, nullptr, Lam, partials,
-                         N, M, beta, theta, u_r, alpha);
-    else
-      hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 0, true, NT>), dim3((unsigned)NB),
-                         dim3(WAVE * W), 0, st, I, STARTS, STARTS, nullptr, GS, nullptr, Lam, nullptr,
-                         N, M, beta, theta, u_r, alpha);
+    const auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)NB), dim3(WAVE * W), 0, st, I, STARTS, STARTS, nullptr,
+                         GS, nullptr, Lam, partials, T, N, M, beta, theta, u_r, alpha);
+    };
+    if constexpr (C == 32) {  // the layers' chunk takes every T
+      if (rag) {
+        partials ? launch(k_lif_bwd_fused<C, W, true, false, 1, true, NT, true>)
+                 : launch(k_lif_bwd_fused<C, W, true, false, 0, true, NT, true>);
+        return;
+      }
+    }
+    partials ? launch(k_lif_bwd_fused<C, W, true, false, 1, true, NT>)
+             : launch(k_lif_bwd_fused<C, W, true, false, 0, true, NT>);
   });
 }
 
 template <int C>
 static void bwd_rc_c(const float* I, const float* STARTS, const float* GS, float* Lam,
-                     double* partials, int64_t N, int M, float beta, float theta, float u_r,
+                     double* partials, int64_t T, int64_t N, int M, float beta, float theta, float u_r,
                      float alpha, hipStream_t st) {
   // registers as the plain adjoint (with the sums as the parameter variant)
   constexpr int WMAX = C == 16 ? 16 : (C == 32 ? 8 : 4);
@@ -529,17 +570,17 @@ static void bwd_rc_c(const float* I, const float* STARTS, const float* GS, float
   const int W = fused_waves((N + WAVE - 1) / WAVE, wmax);
   if constexpr (WMAX >= 16) {
     if (W == 16) {
-      launch_bwd_rc<C, 16>(I, STARTS, GS, Lam, partials, N, M, beta, theta, u_r, alpha, st);
+      launch_bwd_rc<C, 16>(I, STARTS, GS, Lam, partials, T, N, M, beta, theta, u_r, alpha, st);
       return;
     }
   }
   if constexpr (WMAX >= 8) {
     if (W == 8) {
-      launch_bwd_rc<C, 8>(I, STARTS, GS, Lam, partials, N, M, beta, theta, u_r, alpha, st);
+      launch_bwd_rc<C, 8>(I, STARTS, GS, Lam, partials, T, N, M, beta, theta, u_r, alpha, st);
       return;
     }
   }
-  launch_bwd_rc<C, 4>(I, STARTS, GS, Lam, partials, N, M, beta, theta, u_r, alpha, st);
+  launch_bwd_rc<C, 4>(I, STARTS, GS, Lam, partials, T, N, M, beta, theta, u_r, alpha, st);
 }
 
 template <int C, int W>
@@ -552,12 +593,12 @@ static void launch_param_fused(const float* I, const float* u0, const float* U, 
     constexpr bool NT = decltype(nt)::value;
     if (ps == 2)
       hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 2, false, NT>), dim3((unsigned)NB),
-                         dim3(WAVE * W), 0, st, I, u0, U, S, GS, nullptr, Lam, partials, N, M, beta,
-                         theta, u_r, alpha);
+                         dim3(WAVE * W), 0, st, I, u0, U, S, GS, nullptr, Lam, partials, (int64_t)M * C, N,
+                         M, beta, theta, u_r, alpha);
     else
       hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 1, false, NT>), dim3((unsigned)NB),
-                         dim3(WAVE * W), 0, st, I, u0, U, S, GS, nullptr, Lam, partials, N, M, beta,
-                         theta, u_r, alpha);
+                         dim3(WAVE * W), 0, st, I, u0, U, S, GS, nullptr, Lam, partials, (int64_t)M * C, N,
+                         M, beta, theta, u_r, alpha);
   });
 }
 
@@ -605,6 +646,21 @@ int lif_param_bwd_fused(const float* I, const float* u0, const float* U, const f
 }  // namespace lsh
 
 using namespace lsh;
+
+// Which kernels run a layer of any T and N (lsh_lif_layer_fwd, lsh_lif_layer_bwd), measured as
+// single pass / serial sweep and single pass / look-back, us:
+//   forward   N 64 T 100 4.5 / 7.5, T 500 12.4 / 14.6, T 1000 23.3 / 23.3, T 4000 82 / 76;
+//             N 8192 T 500 14.2 / 15.3, T 1000 27.0 / 24.5; N 16384 T 500 16.1 / 16.0, T 1000 30.1 /
+//             25.3; N 51200 T 256 25 / 35, T 1000 95 / 109.
+//   adjoint   N 1000 T 500 13.1 / 13.8, T 1000 25 / 15, T 4000 94 / 22; N 4096 T 1000 26 / 18;
+//             N 8192 T 1000 28.5 / 32.0, T 2000 58 / 50; N 12800 T 1000 33 / 41, T 2000 65 / 68;
+//             N 16384 T 4000 147 / 155; N 51200 T 500 66 / 70.
+// A single pass hands states from wave to wave inside a workgroup, once a 32-row chunk: cheap
+// while there are few chunks or many workgroups.
+static bool layer_fwd_pipe(int64_t T, int64_t N) { return T > 768 && N <= 16384; }
+static bool layer_bwd_lookback(int64_t T, int64_t N) {
+  return T > 512 && (N <= 4096 || (N <= 8192 && T >= 1536));
+}
 
 extern "C" size_t lsh_lif_scan_exact_workspace(void) { return kWsHeaderBytes; }
 
@@ -685,10 +741,63 @@ extern "C" int lsh_lif_scan_fused_bwd_starts(const float* I, const float* STARTS
   hipStream_t st = (hipStream_t)stream;
   const int M = (int)(T / C);
   switch (C) {
-    case 16: bwd_rc_c<16>(I, STARTS, GS, Lam, partials, N, M, beta, theta, u_r, alpha, st); break;
-    case 32: bwd_rc_c<32>(I, STARTS, GS, Lam, partials, N, M, beta, theta, u_r, alpha, st); break;
-    default: bwd_rc_c<64>(I, STARTS, GS, Lam, partials, N, M, beta, theta, u_r, alpha, st); break;
+    case 16: bwd_rc_c<16>(I, STARTS, GS, Lam, partials, T, N, M, beta, theta, u_r, alpha, st); break;
+    case 32: bwd_rc_c<32>(I, STARTS, GS, Lam, partials, T, N, M, beta, theta, u_r, alpha, st); break;
+    default: bwd_rc_c<64>(I, STARTS, GS, Lam, partials, T, N, M, beta, theta, u_r, alpha, st); break;
   }
+  LSH_CHECK_LAUNCH();
+  return LSH_OK;
+}
+
+extern "C" int lsh_lif_layer_fwd(const float* I, const float* u0, float* STARTS, float* S, int64_t T,
+                                 int64_t N, float beta, float theta, float u_r, void* ws,
+                                 size_t ws_bytes, void* stream) {
+  if (bad_ptr(I) || bad_ptr(u0) || bad_ptr(S)) return LSH_ERR_ARG;
+  if (T < 0 || N < 0 || N > (int64_t)1 << 31) return LSH_ERR_SHAPE;
+  if ((uint64_t)N * 32u * 4u >= ((uint64_t)1 << 32)) return LSH_ERR_SHAPE;
+  if (ws != nullptr &&
+      (ws_bytes < kWsHeaderBytes || (reinterpret_cast<uintptr_t>(ws) & 255u) != 0))
+    return LSH_ERR_WORKSPACE;
+  if (T == 0 || N == 0) return LSH_OK;
+  hipStream_t st = (hipStream_t)stream;
+  if (layer_fwd_pipe(T, N)) {
+    lif_starts_fwd_pipe(I, u0, STARTS, S, N, T, beta, theta, u_r, st);
+  } else {
+    WsHeader* h = reinterpret_cast<WsHeader*>(ws);
+    const int64_t NB = (N + WAVE - 1) / WAVE;
+    const int W = fused_waves(NB, 16);
+    if (W == 16)
+      launch_fwd_starts_any<16>(I, u0, STARTS, S, h, T, N, beta, theta, u_r, st);
+    else if (W == 8)
+      launch_fwd_starts_any<8>(I, u0, STARTS, S, h, T, N, beta, theta, u_r, st);
+    else
+      launch_fwd_starts_any<4>(I, u0, STARTS, S, h, T, N, beta, theta, u_r, st);
+  }
+  LSH_CHECK_LAUNCH();
+  return LSH_OK;
+}
+
+extern "C" size_t lsh_lif_layer_bwd_workspace(int64_t T, int64_t N) {
+  return T < 0 || N < 0 || !layer_bwd_lookback(T, N) ? 0 : lsh_lif_scan_lookback_any_bwd_workspace(T, N);
+}
+
+extern "C" int64_t lsh_lif_layer_partials(int64_t T, int64_t N) {
+  if (T < 0 || N < 0) return -1;
+  return (N + WAVE - 1) / WAVE * (layer_bwd_lookback(T, N) ? (T + 255) / 256 : 1);
+}
+
+extern "C" int lsh_lif_layer_bwd(const float* I, const float* STARTS, const float* GS, float* Lam,
+                                 double* partials, int64_t T, int64_t N, float beta, float theta,
+                                 float u_r, float alpha, void* ws, size_t ws_bytes, void* stream) {
+  if (bad_ptr(I) || bad_ptr(STARTS) || bad_ptr(GS) || bad_ptr(Lam)) return LSH_ERR_ARG;
+  if (T < 0 || N < 0 || N > (int64_t)1 << 31) return LSH_ERR_SHAPE;
+  if ((uint64_t)N * 32u * 4u >= ((uint64_t)1 << 32)) return LSH_ERR_SHAPE;
+  if (T == 0 || N == 0) return LSH_OK;
+  hipStream_t st = (hipStream_t)stream;
+  if (layer_bwd_lookback(T, N))
+    return lif_starts_bwd_lookback(I, STARTS, GS, Lam, partials, ws, ws_bytes, T, N, beta, theta, u_r,
+                                   alpha, st);
+  bwd_rc_c<32>(I, STARTS, GS, Lam, partials, T, N, (int)((T + 31) / 32), beta, theta, u_r, alpha, st);
   LSH_CHECK_LAUNCH();
   return LSH_OK;
 }

@@ -45,7 +45,10 @@ void fill_i32_launch(int* p, int64_t n, int v, hipStream_t st) {
 // end of time and adds nothing to the sums; its loads read the chunk's last row, its store is
 // left out.  Its own instantiation, since the tests cost the whole-segment kernel 2 % (N 1024,
 // T 2^18: 0.94 ms).
-template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0, bool RAG = false, bool NT = true>
+// RC (detached, no GU, hard reset): U is [ceil(T/C), N], the state before each chunk, and S is not
+// read; the chunk's forward is replayed from that state in registers (as k_lif_bwd_fused's RC).
+template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0, bool RAG = false, bool NT = true,
+          bool RC = false>
 __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
     const float* __restrict__ I, const float* __restrict__ u0, const float* __restrict__ U,
     const float* __restrict__ S, const float* __restrict__ GS, const float* __restrict__ GU,
@@ -53,6 +56,7 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
     float* __restrict__ incl, int* __restrict__ flags, WsHeader* hdr, double* __restrict__ partials,
     int64_t T, int64_t N, int NB, int NSEG, float beta, float theta, float u_r, float alpha) {
   static_assert(!PS || (DETACH && !HAS_GU && C <= 64), "parameter sums: detached, no GU");
+  static_assert(!RC || (DETACH && !HAS_GU && PS != 2), "recompute: hard reset, detached, no GU");
   constexpr bool AFF = PS == 2;
   __shared__ float sP[W][WAVE], sQ[W][WAVE];
   __shared__ float sLamEnd[WAVE];
@@ -74,7 +78,7 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
   const size_t row0 = ((size_t)seg * W + (W - 1 - w)) * C;  // wave 0 holds the latest chunk
   // RAG: rows of this chunk (wave-uniform; <= 0 for a chunk past the end of the last segment)
   const int rows = !RAG || (int64_t)row0 + C <= T ? C : (int)(T - (int64_t)row0);
-  const float u0n = u0[nb0 + ln];
+  const float u0n = RC ? 0.0f : u0[nb0 + ln];
 
   // 1. coefficients of the chunk and its map
   float a[AFF ? 1 : C], b[C];
@@ -86,15 +90,25 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
   if (!RAG || rows > 0) {
     const Buf bi(I + nb0 + row0 * N), bs(S + nb0 + row0 * N), bg(GS + nb0 + row0 * N);
     const Buf bp(U + nb0 + row0 * N);
-    const float up0 = row0 > 0 ? ld_row(U + nb0 + (row0 - 1) * N, lb) : u0n;
+    const float up0 = RC ? ld_row(U + nb0 + (row0 / C) * N, lb)
+                         : (row0 > 0 ? ld_row(U + nb0 + (row0 - 1) * N, lb) : u0n);
+    float ur = up0;  // RC: the recomputed state
 #pragma unroll
     for (int j = 0; j < C; ++j) {
       const bool in = !RAG || j < rows;
       const unsigned so = (in ? j : rows - 1) * rstride;  // steps past T read the last row
       const float x = bi.ld(lb, so);
-      const float s = bs.ld(lb, so);
       const float gs = bg.ld(lb, so);
-      const float up = j == 0 ? up0 : bp.ld(lb, in ? so - rstride : so);
+      float s, up;
+      if constexpr (RC) {
+        up = ur;
+        bool sp;
+        ur = lif_step(ur, x, beta, theta, u_r, sp);
+        s = sp ? 1.0f : 0.0f;
+      } else {
+        s = bs.ld(lb, so);
+        up = j == 0 ? up0 : bp.ld(lb, in ? so - rstride : so);
+      }
       const float v = lif_v(up, x, beta);
       const float sg = surrogate(v, theta, alpha);
       float J = 1.0f - s;
@@ -227,7 +241,7 @@ static size_t lookback_ws(int64_t T, int64_t N) {
   return kWsHeaderBytes + 3 * align_up(NSEG * (size_t)N * 4, 256) + align_up(NSEG * NB * 4, 256);
 }
 
-template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0>
+template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0, bool RC = false>
 static void launch_lookback(const float* I, const float* u0, const float* U, const float* S,
                             const float* GS, const float* GU, float* Lam, char* ws, int64_t T,
                             int64_t N, float beta, float theta, float u_r, float alpha,
@@ -251,11 +265,11 @@ static void launch_lookback(const float* I, const float* u0, const float* U, con
   const auto by_length = [&](auto nt) {
     constexpr bool NT = decltype(nt)::value;
     if (T % kLookbackSeg == 0)
-      launch(k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS, false, NT>);
+      launch(k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS, false, NT, RC>);
     else
-      launch(k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS, true, NT>);
+      launch(k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS, true, NT, RC>);
   };
-  if constexpr (C == 16 && DETACH && !HAS_GU)
+  if constexpr ((C == 16 && DETACH && !HAS_GU) || RC)
     with_store_policy(N, by_length);
   else
     by_length(std::true_type{});
@@ -405,6 +419,24 @@ int lsh::lif_param_bwd_lookback(const float* I, const float* u0, const float* U,
   else
     launch_lookback<16, 16, true, false, 1>(I, u0, U, S, GS, nullptr, Lam, static_cast<char*>(ws), T, N,
                                             beta, theta, u_r, alpha, st, partials);
+  LSH_CHECK_LAUNCH();
+  return LSH_OK;
+}
+
+int lsh::lif_starts_bwd_lookback(const float* I, const float* STARTS, const float* GS, float* Lam,
+                                 double* partials, void* ws, size_t ws_bytes, int64_t T, int64_t N,
+                                 float beta, float theta, float u_r, float alpha, hipStream_t st) {
+  if (bad_ptr(ws)) return LSH_ERR_ARG;
+  if (ws_bytes < lookback_ws(T, N) || (reinterpret_cast<uintptr_t>(ws) & 255u) != 0)
+    return LSH_ERR_WORKSPACE;
+  if (lookback_segments(T) * ((N + WAVE - 1) / WAVE) > ((int64_t)1 << 31) - 1) return LSH_ERR_SHAPE;
+  char* w = static_cast<char*>(ws);
+  if (partials)
+    launch_lookback<32, 8, true, false, 1, true>(I, nullptr, STARTS, nullptr, GS, nullptr, Lam, w, T, N,
+                                                 beta, theta, u_r, alpha, st, partials);
+  else
+    launch_lookback<32, 8, true, false, 0, true>(I, nullptr, STARTS, nullptr, GS, nullptr, Lam, w, T, N,
+                                                 beta, theta, u_r, alpha, st);
   LSH_CHECK_LAUNCH();
   return LSH_OK;
 }

@@ -111,6 +111,12 @@ int lif_param_bwd_lookback(const float* I, const float* u0, const float* U, cons
                            size_t ws_bytes, int64_t T, int64_t N, float beta, float theta,
                            float u_r, float alpha, int ps, hipStream_t st);
 
+// The look-back adjoint from the state before every 32 rows (lsh_lif_layer_bwd); partials NULL or
+// one row of 3 doubles per (256-step segment, 64-neuron block).
+int lif_starts_bwd_lookback(const float* I, const float* STARTS, const float* GS, float* Lam,
+                            double* partials, void* ws, size_t ws_bytes, int64_t T, int64_t N,
+                            float beta, float theta, float u_r, float alpha, hipStream_t st);
+
 // Device repair rounds of the two-level scan (lif_kernels.hip, k_lif_repair) after a replay that
 // wrote U, S and ends from starts: at most min(repair, M) rounds; list0/list1 hold
 // ceil(N/64)*M*64 ints each.  repair = -1: to convergence without the round count (the ordered
@@ -126,6 +132,9 @@ void fill_i32_launch(int* p, int64_t n, int v, hipStream_t st);
 // Wave-specialised serial sweeps (serial_pipe.hip): the serial entry points' kernels at every
 // neuron count; the one-wave serial kernels remain for scan replays and the parameter sums.
 void lif_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, int64_t N, int64_t T,
+                         float beta, float theta, float u_r, hipStream_t st);
+// S and the state before every 32 rows (STARTS [ceil(T/32), N], or NULL) instead of U
+void lif_starts_fwd_pipe(const float* I, const float* u0, float* STARTS, float* S, int64_t N, int64_t T,
                          float beta, float theta, float u_r, hipStream_t st);
 void aff_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, int64_t N, int64_t T,
                          float beta, float theta, float gamma, float delta, hipStream_t st);

@@ -188,7 +188,9 @@ struct AffStep {
 // tile ahead and store U, S of the tile finished one round earlier, recomputing each spike
 // from the state before it and their own loaded rows (kept two rounds in registers) with the
 // step's operations, so the consumer's chain carries no spike-to-float select.
-template <class Step, bool NT>
+// SO: no U; `U` is [ceil(T/32), N] and receives the state before rows 0, 32, 64, ... (NULL: not
+// wanted), so the spikes alone are written per step.
+template <class Step, bool NT, bool SO = false>
 __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
     const float* __restrict__ I, const float* __restrict__ u0, float* __restrict__ U,
     float* __restrict__ S, int64_t N, int64_t T, Step step) {
@@ -277,9 +279,14 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
         const int j = p + r * P;
         if (j < nr) {
           const size_t row = (size_t)((k - 2) * D + j) * (size_t)N + (size_t)nb0;
-          const float u = sU[buf][j][lane];
           const float up = j == 0 ? sEntry[buf][lane] : sU[buf][j - 1][lane];
-          st_row<NT>(U + row, sb, u);
+          if constexpr (SO) {
+            static_assert(D % 32 == 0, "the states fall on rows 0, 32, ... of a tile");
+            if (j % 32 == 0 && U != nullptr)
+              st_row<NT>(U + (size_t)((k - 2) * (D / 32) + j / 32) * (size_t)N + (size_t)nb0, sb, up);
+          } else {
+            st_row<NT>(U + row, sb, sU[buf][j][lane]);
+          }
           st_row<NT>(S + row, sb, step.spike(up, x2[r]) ? 1.0f : 0.0f);
         }
       }
@@ -299,6 +306,16 @@ void lif_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, in
   with_store_policy(N, [&](auto nt) {
     hipLaunchKernelGGL((k_serial_fwd_pipe<LifStep, decltype(nt)::value>), dim3((unsigned)NB),
                        dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, U, S, N, T, LifStep{beta, theta, u_r});
+  });
+}
+
+void lif_starts_fwd_pipe(const float* I, const float* u0, float* STARTS, float* S, int64_t N, int64_t T,
+                         float beta, float theta, float u_r, hipStream_t st) {
+  const int NB = (int)((N + WAVE - 1) / WAVE);
+  with_store_policy(N, [&](auto nt) {
+    hipLaunchKernelGGL((k_serial_fwd_pipe<LifStep, decltype(nt)::value, true>), dim3((unsigned)NB),
+                       dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, STARTS, S, N, T,
+                       LifStep{beta, theta, u_r});
   });
 }
 

@@ -64,15 +64,15 @@ class LIFParamFn(torch.autograd.Function):
     (fit.py:15-48).  fwd_mode / bwd_mode: "serial" or "scan", or lif_param's own choices."""
 
     @staticmethod
-    def forward(ctx, I, u0, beta, theta, u_r, alpha, fwd_mode, bwd_mode, K):
+    def forward(ctx, I, u0, beta, theta, u_r, alpha, fwd_mode, bwd_mode, K, choose=False):
         b, th, ur = _f32s(beta, theta, u_r)
         I = I.contiguous()
         ctx.cfg = (b, th, ur, float(alpha), bwd_mode)
         T, N = I.shape
-        # the serial forward's bits are the single-pass exact forward's: with the single-pass
-        # adjoint behind it, keep the chunk entry states instead of U (same S and gradients)
-        if fwd_mode == "serial" and bwd_mode == "scan" and L._recompute_ok(T, N, K, T):
-            S, ST = L.scan_forward_exact_starts(I, b, th, ur, u0)
+        # lif_param's own choice: the exact forward's bits are the serial one's, so the states before
+        # every 32 rows are kept instead of U
+        if choose and L._layer_ok(N) and T > 0 and not L._auto_states(T, N, b):
+            S, ST = L._layer_forward(I, b, th, ur, u0)
             ctx.save_for_backward(I, u0, ST)
             ctx.recompute = True
             return S
@@ -91,7 +91,7 @@ class LIFParamFn(torch.autograd.Function):
         b, th, ur, alpha, bwd_mode = ctx.cfg
         if ctx.recompute:
             I, u0, ST = ctx.saved_tensors
-            lam, sums = L.scan_backward_fused_starts(I, ST, gS.contiguous(), b, th, ur, alpha, True)
+            lam, sums = L._layer_backward(I, ST, gS.contiguous(), b, th, ur, alpha, True)
         else:
             I, u0, U, S = ctx.saved_tensors
             lam, sums = _param_backward(I, u0, U, S, gS.contiguous(), b, th, ur, alpha, bwd_mode)
@@ -99,7 +99,7 @@ class LIFParamFn(torch.autograd.Function):
         need = ctx.needs_input_grad  # a gradient only for the parameters given as tensors
         du0 = b * lam[0] if ctx.needs_input_grad[1] else None
         return (lam, du0, sums[0] if need[2] else None, -sums[1] if need[3] else None,
-                b * sums[2] if need[4] else None, None, None, None, None)
+                b * sums[2] if need[4] else None, None, None, None, None, None)
 
 
 def lif_param(I, u0, beta, theta, u_r, alpha=4.0, mode="auto", K=16):
@@ -112,7 +112,7 @@ def lif_param(I, u0, beta, theta, u_r, alpha=4.0, mode="auto", K=16):
         fwd, bwd = L._auto_fwd(fwd, N, T), L._auto_bwd(bwd, N, T)
     else:
         fwd = bwd = mode
-    return LIFParamFn.apply(I, u0, beta, theta, u_r, alpha, fwd, bwd, K)
+    return LIFParamFn.apply(I, u0, beta, theta, u_r, alpha, fwd, bwd, K, mode == "auto")
 
 
 class LIFSoftFn(torch.autograd.Function):

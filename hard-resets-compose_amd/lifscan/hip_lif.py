@@ -472,7 +472,7 @@ WARM_ANY_WIDE_N = 1024
 
 def warm_any_plan(T, N, beta):
     """(C, W) of the warm-started forward for any T, or None where the serial sweep is as fast."""
-    if N > WARM_FEW_MAX_N or N < 1:
+    if N > WARM_FEW_MAX_N or N < 1 or T < 4 * 256:
         return None
     b = abs(_f32(beta))
     if not b < 1.0:
@@ -912,6 +912,62 @@ def scan_backward_fused_starts(I, STARTS, GS, beta, theta, u_r, alpha=4.0, want_
     return Lam, (parts.sum(0) if want_sums else None)
 
 
+def _layer_ok(N):
+    """The layer pair's kernels address a 32-row chunk with 32-bit byte offsets."""
+    return RECOMPUTE_BWD and 1 <= N < 1 << 25
+
+
+def _converged_layer(T, N, beta, K, repair):
+    """True when a converged scan layer (lif_tuned) takes the layer pair: scan_forward_auto would
+    give the serial recurrence's bits and neither warm-started nor long chunks are faster."""
+    C = _chunk_or_none(T, 16)
+    return (C is not None and T > 0 and _layer_ok(N) and int(K) <= 16 and int(repair) >= T // C
+            and warm_plan(T, N, beta) is None and warm_any_plan(T, N, beta) is None
+            and not long_sequence_C(T, N))
+
+
+def _layer_forward(I, beta, theta, u_r, u0, want_states=True):
+    """The layers' forward for every T -> (S, STATES [ceil(T/32), N] or None): the serial
+    recurrence's spikes and the state before rows 0, 32, 64, ..."""
+    I = _input(I)
+    T, N = I.shape
+    u0 = _vec(u0, N, I)
+    S = torch.empty_like(I)
+    ST = torch.empty((T + 31) // 32, N, device=I.device, dtype=torch.float32) if want_states else None
+    hdr = _wait_header(I.device)
+    with _n.on_device(I):
+        _n.check(_n.lib().lsh_lif_layer_fwd(
+            _n.ptr(I), _n.ptr(u0), _n.ptr(ST), _n.ptr(S), T, N, _f32(beta), _f32(theta), _f32(u_r),
+            _n.ptr(hdr), hdr.numel(), _n.stream_of(I)), "lsh_lif_layer_fwd")
+    if CHECK_WAITS and int(_n.read_stats(hdr, 1).spin_timeouts) != 0:
+        raise RuntimeError("lsh_lif_layer_fwd: a chunk hand-off wait gave up; S and the states are "
+                           "not valid")
+    return S, ST
+
+
+def _layer_backward(I, STATES, GS, beta, theta, u_r, alpha=4.0, want_sums=False):
+    """The layers' adjoint from _layer_forward's states (detached reset, no GU) -> (Lam, sums), sums
+    as scan_backward_fused_starts."""
+    I = _input(I)
+    T, N = I.shape
+    GS = _same(GS, I, "GS")
+    Lam = torch.empty_like(I)
+    if T == 0 or N == 0:
+        return Lam, torch.zeros(3, device=I.device, dtype=torch.float64) if want_sums else None
+    L = _n.lib()
+    nbytes = L.lsh_lif_layer_bwd_workspace(T, N)
+    ws = _n.workspace(nbytes, I.device) if nbytes else None
+    parts = None
+    if want_sums:
+        parts = torch.empty(L.lsh_lif_layer_partials(T, N), 3, device=I.device, dtype=torch.float64)
+    with _n.on_device(I):
+        _n.check(L.lsh_lif_layer_bwd(
+            _n.ptr(I), _n.ptr(STATES), _n.ptr(GS), _n.ptr(Lam), _n.ptr(parts), T, N, _f32(beta),
+            _f32(theta), _f32(u_r), _f32(alpha), _n.ptr(ws), nbytes, _n.stream_of(I)),
+            "lsh_lif_layer_bwd")
+    return Lam, (parts.sum(0) if want_sums else None)
+
+
 def _recompute_ok(T, N, K, repair):
     """True when scan_forward_auto and scan_backward_auto would both take the single-pass
     kernels (converged forward without maps, fused adjoint): then the recomputing pair gives
@@ -1101,6 +1157,13 @@ def _auto_fwd(fwd, N, T):
     return "auto" if 1 <= N <= WARM_FEW_MAX_N and T >= 4 * 256 else fwd
 
 
+def _auto_states(T, N, beta):
+    """True when a layer that chooses keeps U and S for its adjoint (warm-started chunks, or the map
+    scan where they do not apply) instead of the layer pair's states."""
+    return warm_any_plan(T, N, beta) is not None or (
+        T >= AUTO_FWD_MIN_T and auto_modes(N, T)[0] == "scan")
+
+
 def _auto_forward(I, beta, theta, u_r, u0, K, repair):
     """(U, S) of a layer's own choice: warm-started chunks (the serial recurrence's bits, faster than
     the serial sweep and than the map scan: N = 64, T = 50000 0.91 ms of map scan -> 0.06 ms), else
@@ -1187,14 +1250,19 @@ class LIFTuned(torch.autograd.Function):
             # U is kept only for the backward: store the chunk entry states instead
             S, ST = scan_forward_exact_starts(I, b, theta, u_r, u0)
             ctx.save_for_backward(I, u0, ST)
-            ctx.recompute = True
+            ctx.recompute = "single"
+            return S
+        if mode != "serial" and _converged_layer(T, N, b, K, repair):
+            S, ST = _layer_forward(I, b, theta, u_r, u0)
+            ctx.save_for_backward(I, u0, ST)
+            ctx.recompute = "layer"
             return S
         if mode == "serial":
             U, S = serial_forward_auto(I, b, theta, u_r, u0)
         else:
             U, S = scan_forward_auto(I, b, theta, u_r, u0, K=K, repair=repair)
         ctx.save_for_backward(I, u0, U, S)
-        ctx.recompute = False
+        ctx.recompute = None
         return S
 
     @staticmethod
@@ -1204,7 +1272,8 @@ class LIFTuned(torch.autograd.Function):
         if ctx.recompute:
             I, u0, ST = ctx.saved_tensors
             need_b = ctx.needs_input_grad[2]
-            Lam, sums = scan_backward_fused_starts(I, ST, gS, b, theta, u_r, alpha, need_b)
+            bwd = scan_backward_fused_starts if ctx.recompute == "single" else _layer_backward
+            Lam, sums = bwd(I, ST, gS, b, theta, u_r, alpha, need_b)
             db = sums[0].float().reshape(()) if need_b else None
             du0 = b * Lam[0] if ctx.needs_input_grad[1] else None
             return (Lam, du0, db, None, None, None, None, None, None)
@@ -1265,11 +1334,9 @@ class LIFAuto(torch.autograd.Function):
         b = _f32(beta)
         ctx.cfg = (b, theta, u_r, alpha, bwd_mode)
         T, N = I.shape
-        # the serial forward's bits are the single-pass exact forward's; with the fused adjoint
-        # behind it the recomputing pair applies (U is kept only for the backward)
-        if (fwd_mode == "serial" and bwd_mode == "scan"
-                and _recompute_ok(T, N, K, max(int(repair), T))):
-            S, ST = scan_forward_exact_starts(I, b, theta, u_r, u0)
+        # the exact forward's bits are the serial one's: U, kept only for the backward, is left out
+        if fwd_mode in ("serial", "auto") and _layer_ok(N) and T > 0 and not _auto_states(T, N, b):
+            S, ST = _layer_forward(I, b, theta, u_r, u0)
             ctx.save_for_backward(I, u0, ST)
             ctx.recompute = True
             return S
@@ -1290,7 +1357,7 @@ class LIFAuto(torch.autograd.Function):
         if ctx.recompute:
             I, u0, ST = ctx.saved_tensors
             need_b = ctx.needs_input_grad[2]
-            Lam, sums = scan_backward_fused_starts(I, ST, gS, b, theta, u_r, alpha, need_b)
+            Lam, sums = _layer_backward(I, ST, gS, b, theta, u_r, alpha, need_b)
             db = sums[0].float().reshape(()) if need_b else None
             du0 = b * Lam[0] if ctx.needs_input_grad[1] else None
             return (Lam, du0, db, None, None, None, None, None, None, None)
@@ -1306,11 +1373,25 @@ class LIFAuto(torch.autograd.Function):
                 None, None, None, None, None, None, None)
 
 
+def _plain_call(*tensors):
+    """True when a layer call needs no autograd function: no gradient is recorded, and neither
+    forward-mode differentiation nor a function transform is looking."""
+    if torch.is_grad_enabled() and any(torch.is_tensor(t) and t.requires_grad for t in tensors):
+        return False
+    return (torch.autograd.forward_ad._current_level < 0
+            and not torch._C._are_functorch_transforms_active())
+
+
 def lif_auto(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, K=16, repair=0):
     T, N = I.shape
+    if _layer_ok(N) and T > 0 and _plain_call(I, u0, beta) and (
+            not torch.is_tensor(u0) or (u0.dim() == 1 and u0.shape[0] == N)):
+        b = _f32(beta)
+        if not _auto_states(T, N, b):  # spikes alone
+            return _layer_forward(I, b, theta, u_r, u0, want_states=False)[0]
     fwd, bwd = auto_modes(N, T)
     fwd, bwd = _auto_fwd(fwd, N, T), _auto_bwd(bwd, N, T)
-    if fwd == bwd:  # one mode for both passes: lif_tuned's path (the same kernels and bits)
+    if not _layer_ok(N) and fwd == bwd:  # one mode for both passes: lif_tuned's path
         return lif_tuned(I, u0, beta, theta, u_r, alpha, mode=fwd, K=K, repair=repair)
     return LIFAuto.apply(I, u0, beta, theta, u_r, alpha, K, repair, fwd, bwd)
 

@@ -263,6 +263,20 @@ int lsh_lif_scan_fused_bwd_starts(const float* I, const float* STARTS, const flo
                                   double* partials, int64_t T, int64_t N, float beta, float theta,
                                   float u_r, float alpha, int C, void* stream);
 
+/* The same pair for every T and N, the layers' own: the forward writes S and, unless STARTS is NULL
+ * (spikes only), the state before rows 0, 32, 64, ..., STARTS[ceil(T/32)][N]; the adjoint replays
+ * each 32-row chunk from its state.  The kernels are chosen by T and N (single pass or serial sweep
+ * forward, single pass or look-back adjoint); S is the serial recurrence's bit for bit.  The
+ * forward's ws as above; the adjoint's is lsh_lif_layer_bwd_workspace(T, N) bytes, 256-byte aligned
+ * (0: NULL).  partials: NULL, or lsh_lif_layer_partials(T, N) rows of 3 doubles as above. */
+int lsh_lif_layer_fwd(const float* I, const float* u0, float* STARTS, float* S, int64_t T, int64_t N,
+                      float beta, float theta, float u_r, void* ws, size_t ws_bytes, void* stream);
+size_t lsh_lif_layer_bwd_workspace(int64_t T, int64_t N);
+int64_t lsh_lif_layer_partials(int64_t T, int64_t N);
+int lsh_lif_layer_bwd(const float* I, const float* STARTS, const float* GS, float* Lam,
+                      double* partials, int64_t T, int64_t N, float beta, float theta, float u_r,
+                      float alpha, void* ws, size_t ws_bytes, void* stream);
+
 /* ---------------------------------------------------------------------------------------
  * ALIF: v = fl(fl(beta*u) + x); s = v >= fl(theta0 + w); u' = s ? u_r : v;
  *       w' = s ? fl(fl(rho*w) + q) : fl(rho*w)          (triton_alif.py:26-31)

@@ -146,3 +146,65 @@ def test_row_alignment_store_policies(dev, N):
     dI, = torch.autograd.grad(s, [leaf], Gg)
     LV, _ = A.alif_backward(Ig, u, w, s, Gg, 0.95, 0.995, 0.2, 1.0, ug, gpu(w0, dev), mode="serial")
     assert rel(host(dI), host(LV)) < 1e-6
+
+
+# the single pass, the look-back adjoint (T > 512, few neurons), the serial sweep forward (T > 768)
+@pytest.mark.parametrize("T", [1, 31, 33, 257, 512, 513, 801])
+@pytest.mark.parametrize("N", [1, 70, 129])
+def test_layer_pair_any_length(dev, T, N):
+    """The layers' forward and adjoint: the oracle's spikes and states bit for bit, the fp64 adjoint
+    and parameter sums; rows behind the last one are NaN."""
+    _layer_pair(dev, T, N)
+
+
+def test_layer_pair_many_neurons(dev):
+    _layer_pair(dev, 801, 16390)  # the single pass in both directions, a short last chunk
+
+
+def _layer_pair(dev, T, N):
+    from lifscan import hip_lif as L
+    I, GS, u0 = normal(T, N, 0.15, 0.4, T), normal(T, N, 0.0, 1.0, T + 1), uniform(N, 0.0, 1.0, 3)
+    U, S = O.serial_forward(I, 0.95, 1.0, -0.1, u0)
+    want = O.serial_backward(I, u0, U, S, GS, None, 0.95, 1.0, -0.1, 4.0, True, dtype=np.float64)
+    pad = lambda a: torch.cat([gpu(a, dev), torch.full((40, N), float("nan"), device=dev)])[:T]
+    print(f"layer pair T={T} N={N}", flush=True)
+    s, st = L._layer_forward(pad(I), 0.95, 1.0, -0.1, gpu(u0, dev))
+    assert np.array_equal(host(s), S)
+    assert np.array_equal(host(st), np.concatenate([u0[None], U[:-1]])[::32])
+    s2, none = L._layer_forward(pad(I), 0.95, 1.0, -0.1, gpu(u0, dev), want_states=False)
+    assert none is None and torch.equal(s2, s)
+    lam, none = L._layer_backward(pad(I), st, pad(GS), 0.95, 1.0, -0.1)
+    lam2, sums = L._layer_backward(pad(I), st, pad(GS), 0.95, 1.0, -0.1, 4.0, True)
+    assert none is None and rel(host(lam), want) < 1e-6 and rel(host(lam2), want) < 1e-6
+    grads = O.param_grads(I, u0, U, S, GS, want, 0.95, 1.0, -0.1, 4.0)
+    for k, g in enumerate((sums[0], -sums[1], 0.95 * sums[2])):
+        assert abs(g.item() - grads[2 + k]) <= 1e-4 * abs(grads[2 + k]) + 1e-5, k
+    assert L.starts_forward_timeouts(dev) == 0
+
+
+@pytest.mark.parametrize("call", ["auto", "tuned", "param"])
+@pytest.mark.parametrize("T,N", [(96, 40), (1002, 130), (1504, 5000)])
+def test_layers_take_the_pair(dev, call, T, N):
+    """lif_auto, lif_tuned (converged; T with a chunk) and lif_param: spikes, dI, du0 and dbeta."""
+    from lifscan import hip_lif as L
+    from lifscan.fit import lif_param
+    if call == "tuned" and T == 1002:
+        with pytest.raises(ValueError):  # no chunk for T: refused, as ever
+            L.lif_tuned(torch.zeros(T, N, device=dev), torch.zeros(N, device=dev), repair=10 ** 6)
+        return
+    I, GS, u0 = normal(T, N, 0.15, 0.4, 1), normal(T, N, 0.0, 1.0, 2), uniform(N, 0.0, 1.0, 3)
+    Uo, So = O.serial_forward(I, 0.95, 1.0, 0.0, u0)
+    want = O.serial_backward(I, u0, Uo, So, GS, None, 0.95, 1.0, 0.0, 4.0, True, dtype=np.float64)
+    Ig, ug = gpu(I, dev).requires_grad_(True), gpu(u0, dev).requires_grad_(True)
+    b = torch.tensor(0.95, device=dev, requires_grad=True)
+    f = {"auto": lambda x: L.lif_auto(Ig, ug, x), "tuned": lambda x: L.lif_tuned(Ig, ug, x, repair=10 ** 6),
+         "param": lambda x: lif_param(Ig, ug, x, 1.0, 0.0)}[call]
+    for beta in (0.95, b):
+        S = f(beta)
+        grads = torch.autograd.grad(S, [Ig, ug] + ([b] if beta is b else []), gpu(GS, dev))
+        assert np.array_equal(host(S), So)
+        assert rel(host(grads[0]), want) < 1e-6 and rel(host(grads[1]), 0.95 * want[0]) < 1e-6
+    up = np.concatenate([u0[None], Uo[:-1]]).astype(np.float64)
+    assert abs(grads[2].item() - (want * up).sum()) <= 1e-4 * abs((want * up).sum()) + 1e-4
+    with torch.no_grad():
+        assert np.array_equal(host(f(0.95)), So)
