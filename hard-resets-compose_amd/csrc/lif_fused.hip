@@ -825,3 +825,53 @@ extern "C" int lsh_lif_scan_fused_bwd(const float* I, const float* u0, const flo
   LSH_CHECK_LAUNCH();
   return LSH_OK;
 }
+
+// What a layer's backward leaves to do after its adjoint: workgroup 0 sums the partials' columns
+// (each thread its rows in order, eight loads in flight, then a fixed tree), the others write du0.
+// Bound by latency; it replaces five or six small tensor operations (a reduction, a conversion, a
+// scaling a parameter, du0) of some 4 us of launch each.
+constexpr int kGradThreads = 512;
+template <int COLS>
+__global__ __launch_bounds__(kGradThreads) void k_layer_grads(
+    const double* __restrict__ parts, int64_t P, double s0, double s1, double s2,
+    float* __restrict__ sums, const float* __restrict__ Lam0, int64_t N, float beta,
+    float* __restrict__ du0) {
+  const int tid = threadIdx.x;
+  if (blockIdx.x > 0) {
+    const int64_t n = (int64_t)(blockIdx.x - 1) * kGradThreads + tid;
+    if (n < N) du0[n] = beta * Lam0[n];
+    return;
+  }
+  if (sums == nullptr) return;
+  __shared__ double acc[kGradThreads / WAVE][COLS];
+  double a[COLS] = {};
+#pragma unroll 8
+  for (int64_t p = tid; p < P; p += kGradThreads)
+    for (int k = 0; k < COLS; ++k) a[k] += parts[p * COLS + k];
+  for (int k = 0; k < COLS; ++k) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) a[k] += __shfl_xor(a[k], o, WAVE);
+    if (tid % WAVE == 0) acc[tid / WAVE][k] = a[k];
+  }
+  __syncthreads();
+  if (tid < COLS) {
+    double v = 0.0;
+    for (int w = 0; w < kGradThreads / WAVE; ++w) v += acc[w][tid];
+    sums[tid] = (float)((tid == 0 ? s0 : (tid == 1 ? s1 : s2)) * v);
+  }
+}
+
+extern "C" int lsh_layer_grads(const double* partials, int64_t P, int cols, double s0, double s1,
+                               double s2, float* sums, const float* Lam0, int64_t N, float beta,
+                               float* du0, void* stream) {
+  if (P < 0 || N < 0 || (sums != nullptr && cols != 1 && cols != 3)) return LSH_ERR_SHAPE;
+  if ((sums != nullptr && bad_ptr(partials)) || (du0 != nullptr && N > 0 && bad_ptr(Lam0)))
+    return LSH_ERR_ARG;
+  const int64_t blocks = 1 + (du0 != nullptr ? (N + kGradThreads - 1) / kGradThreads : 0);
+  if (blocks > ((int64_t)1 << 31) - 1) return LSH_ERR_SHAPE;
+  hipLaunchKernelGGL(cols == 1 ? k_layer_grads<1> : k_layer_grads<3>, dim3((unsigned)blocks),
+                     dim3(kGradThreads), 0, (hipStream_t)stream, partials, P, s0, s1, s2, sums, Lam0, N,
+                     beta, du0);
+  LSH_CHECK_LAUNCH();
+  return LSH_OK;
+}

@@ -106,7 +106,7 @@ OPS_PATH = os.path.join(OPS_DIR, OPS_NAME + ".so")
 
 
 def build_ops(verbose=False):
-    """Compile lifscan/_ops.cpp (the C++ autograd function of lif_tuned's recomputing pair) into
+    """Compile lifscan/_ops.cpp (the C++ autograd functions of the layers) into
     the in-tree lifscan/_lib/_ops/lifscan_ops.so with torch's extension builder (host compiler,
     torch and HIP headers; it calls the HIP library through addresses handed over at load)."""
     import torch  # noqa: F401  (the builder needs torch's headers and libraries)
@@ -116,7 +116,7 @@ def build_ops(verbose=False):
     cpp_extension.load(
         name=OPS_NAME, sources=[os.path.join(PKG_DIR, "_ops.cpp")], build_directory=OPS_DIR,
         extra_cflags=["-O2", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"],
-        extra_include_paths=["/opt/rocm/include"],
+        extra_include_paths=["/opt/rocm/include", os.path.join(REPO, "include")],
         extra_ldflags=[f"-L{torch_lib}", "-lc10_hip", f"-Wl,-rpath,{torch_lib}"],
         with_cuda=False, is_python_module=True, verbose=verbose)
     return OPS_PATH

@@ -112,6 +112,8 @@ SIGNATURES = {
     "lsh_lif_scan_fused_bwd_starts": (c_i, [c_p, c_p, c_p, c_p, c_p, c_i64, c_i64, c_f, c_f, c_f, c_f,
                                             c_i, c_p]),
     "lsh_lif_layer_fwd": (c_i, [c_p, c_p, c_p, c_p, c_i64, c_i64, c_f, c_f, c_f, c_p, c_sz, c_p]),
+    "lsh_layer_grads": (c_i, [c_p, c_i64, c_i, ctypes.c_double, ctypes.c_double, ctypes.c_double,
+                              c_p, c_p, c_i64, c_f, c_p, c_p]),
     "lsh_lif_layer_bwd_workspace": (c_sz, [c_i64, c_i64]),
     "lsh_lif_layer_partials": (c_i64, [c_i64, c_i64]),
     "lsh_lif_layer_bwd": (c_i, [c_p, c_p, c_p, c_p, c_p, c_i64, c_i64, c_f, c_f, c_f, c_f, c_p, c_sz,
@@ -200,9 +202,9 @@ _OPS = None
 
 
 def ops():
-    """The C++ autograd module of lif_tuned's recomputing pair (lifscan/_ops.cpp, built in-tree
-    by build()) with the library's entry points handed over, or None when it is not built (the
-    layer then runs the same kernels through its Python autograd function)."""
+    """The C++ autograd module of the layers (lifscan/_ops.cpp, built in-tree by build()) with the
+    library's entry points handed over, or None when it is not built (the layers then run the same
+    kernels through their Python autograd functions)."""
     global _OPS
     if _OPS is None:
         if not os.path.exists(_build.OPS_PATH):
@@ -212,9 +214,8 @@ def ops():
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)
         L = lib()
-        addr = lambda f: ctypes.cast(f, ctypes.c_void_p).value
-        mod.set_entry_points(addr(L.lsh_lif_scan_exact_fwd_starts),
-                             addr(L.lsh_lif_scan_fused_bwd_starts), addr(L.lsh_status_string))
+        mod.set_entry_points({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value
+                              for name in SIGNATURES})
         _OPS = mod
     return _OPS
 

@@ -19,6 +19,18 @@ from . import hip_lif as L
 from .hip_lif import _f32, _f32s, _input, _vec, _same
 
 
+def _param_plan(T, N, mode):
+    """lsh_lif_param_bwd's mode code and chunk for an adjoint mode name."""
+    if mode == "scan":
+        if N >= L.FUSED_BWD_MIN_N and T % L.FUSED_BWD_C == 0:
+            return 2, L.FUSED_BWD_C
+        if L.LOOKBACK_BWD and T % L.LOOKBACK_SEG == 0:
+            return 3, 16
+        C = L.chunked_bwd_C(T, N, min(128, L._pick_C(T, D=2)))
+        return (4, 16) if L.lookback_any(N) else (1, C)
+    return (4, 16) if mode == "lookback" else (0, 1)
+
+
 def _param_backward(I, u0, U, S, GS, beta, theta, u_r, alpha, mode):
     """lsh_lif_param_bwd -> (Lam, sums [3] fp64)."""
     I = _input(I)
@@ -26,19 +38,7 @@ def _param_backward(I, u0, U, S, GS, beta, theta, u_r, alpha, mode):
     u0 = _vec(u0, N, I)
     U, S, GS = (_same(a, I, nm) for a, nm in ((U, "U"), (S, "S"), (GS, "GS")))
     lib = _n.lib()
-    if mode == "scan":
-        if N >= L.FUSED_BWD_MIN_N and T % L.FUSED_BWD_C == 0:
-            code, C = 2, L.FUSED_BWD_C
-        elif L.LOOKBACK_BWD and T % L.LOOKBACK_SEG == 0:
-            code, C = 3, 16
-        else:
-            code, C = 1, L.chunked_bwd_C(T, N, min(128, L._pick_C(T, D=2)))
-            if L.lookback_any(N):
-                code, C = 4, 16
-    elif mode == "lookback":
-        code, C = 4, 16
-    else:
-        code, C = 0, 1
+    code, C = _param_plan(T, N, mode)
     P = lib.lsh_lif_param_partials(T, N, code, C)
     if P < 0:
         raise ValueError(f"T={T} must be divisible by C={C}")
@@ -61,11 +61,12 @@ def _param_backward(I, u0, U, S, GS, beta, theta, u_r, alpha, mode):
 
 class LIFParamFn(torch.autograd.Function):
     """S = LIF(I; u0, beta, theta, u_r) with gradients for I, u0 and the three parameters
-    (fit.py:15-48).  fwd_mode / bwd_mode: "serial" or "scan", or lif_param's own choices."""
+    (fit.py:15-48).  fwd_mode / bwd_mode: "serial" or "scan", or lif_param's own choices (choose: True,
+    or the three parameters' values already read)."""
 
     @staticmethod
     def forward(ctx, I, u0, beta, theta, u_r, alpha, fwd_mode, bwd_mode, K, choose=False):
-        b, th, ur = _f32s(beta, theta, u_r)
+        b, th, ur = choose if isinstance(choose, tuple) else _f32s(beta, theta, u_r)
         I = I.contiguous()
         ctx.cfg = (b, th, ur, float(alpha), bwd_mode)
         T, N = I.shape
@@ -107,12 +108,24 @@ def lif_param(I, u0, beta, theta, u_r, alpha=4.0, mode="auto", K=16):
     0-d tensors or floats; floats go to the kernels as they are (the reference wraps them in
     device tensors and reads them back: the same fp32 values, one synchronizing copy more)."""
     T, N = I.shape
-    if mode == "auto":
+    choose = mode == "auto"
+    if choose:
         fwd, bwd = L.auto_modes(N, T)
         fwd, bwd = L._auto_fwd(fwd, N, T), L._auto_bwd(bwd, N, T)
+        u0v = L._cpp_u0(I, u0, alpha) if L._layer_ok(N) else None
+        if u0v is not None:  # the same kernels as LIFParamFn's, from C++
+            b, th, ur = choose = _f32s(beta, theta, u_r)
+            plan = L.warm_any_plan(T, N, b)
+            if not L._auto_states(T, N, b):
+                plan = (0, 0)
+            elif plan is None or _param_plan(T, N, bwd)[0] < 3:
+                plan = None
+            if plan is not None:
+                return _n.ops().lif_layer(I, u0v, *map(L._grad_param, (beta, theta, u_r)), b, th, ur,
+                                          float(alpha), L._wait_header(I.device), *plan)
     else:
         fwd = bwd = mode
-    return LIFParamFn.apply(I, u0, beta, theta, u_r, alpha, fwd, bwd, K, mode == "auto")
+    return LIFParamFn.apply(I, u0, beta, theta, u_r, alpha, fwd, bwd, K, choose)
 
 
 class LIFSoftFn(torch.autograd.Function):
@@ -177,4 +190,11 @@ class LIFSoftScanFn(torch.autograd.Function):
 
 def lif_soft_scan(I, u0, beta, theta=1.0, alpha=4.0, mode="scan", C=128, K=32):
     """fit.py:152-153."""
+    from . import hip_affine as AF
+    from . import hip_soft as TS
+    u0v = AF._cpp_layer_u0(I, u0, mode, C, K, theta, alpha)
+    if u0v is not None:  # the same kernels as LIFSoftScanFn's, from C++
+        b, th = _f32s(beta, theta)
+        return AF._cpp_layer(I, u0v, (beta, None, None), (b, th, 1.0, -th, float(alpha)), True, mode, C,
+                             K, 0, TS._soft_C(*I.shape))
     return LIFSoftScanFn.apply(I, u0, beta, theta, alpha, mode, C, K)

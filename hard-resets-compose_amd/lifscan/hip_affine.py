@@ -116,14 +116,8 @@ def reverse_affine_scan(a, b):
     return out
 
 
-def _aff_backward(I, u0, U, S, GS, beta, theta, gamma, alpha, mode="auto", C=None):
-    """lsh_aff_bwd -> (Lam, sums [3] fp64: sum lam*u_{t-1}, sum s*v*lam_{t+1}, sum s*lam_{t+1}).
-    mode "auto" picks the adjoint by shape as the LIF scan adjoint does; "serial", "chunked",
-    "fused" and "lookback" force one."""
-    I = _input(I)
-    T, N = I.shape
-    u0 = _vec(u0, N, I)
-    U, S, GS = (_same(a, I, nm) for a, nm in ((U, "U"), (S, "S"), (GS, "GS")))
+def _aff_plan(T, N, mode="auto", C=None):
+    """lsh_aff_bwd's mode code and chunk for an adjoint mode name."""
     if mode == "auto":
         if N >= L.FUSED_BWD_MIN_N and T % L.FUSED_BWD_C == 0:
             mode = "fused"
@@ -135,17 +129,27 @@ def _aff_backward(I, u0, U, S, GS, beta, theta, gamma, alpha, mode="auto", C=Non
             mode = "lookback_any" if L.lookback_any(N) else (
                 "chunked" if T >= L.AUTO_BWD_MIN_T else "serial")
     if mode == "fused":
-        code, C = 2, int(C or L.FUSED_BWD_C)
-    elif mode == "lookback":
-        code, C = 3, 16
-    elif mode == "lookback_any":
-        code, C = 4, 16
-    elif mode == "chunked":
-        code, C = 1, int(C or L.chunked_bwd_C(T, N, min(128, L._pick_C(T, D=2))))
-    elif mode == "serial":
-        code, C = 0, 1
-    else:
-        raise ValueError(f"unknown mode {mode!r}")
+        return 2, int(C or L.FUSED_BWD_C)
+    if mode == "lookback":
+        return 3, 16
+    if mode == "lookback_any":
+        return 4, 16
+    if mode == "chunked":
+        return 1, int(C or L.chunked_bwd_C(T, N, min(128, L._pick_C(T, D=2))))
+    if mode == "serial":
+        return 0, 1
+    raise ValueError(f"unknown mode {mode!r}")
+
+
+def _aff_backward(I, u0, U, S, GS, beta, theta, gamma, alpha, mode="auto", C=None):
+    """lsh_aff_bwd -> (Lam, sums [3] fp64: sum lam*u_{t-1}, sum s*v*lam_{t+1}, sum s*lam_{t+1}).
+    mode "auto" picks the adjoint by shape as the LIF scan adjoint does; "serial", "chunked",
+    "fused" and "lookback" force one."""
+    I = _input(I)
+    T, N = I.shape
+    u0 = _vec(u0, N, I)
+    U, S, GS = (_same(a, I, nm) for a, nm in ((U, "U"), (S, "S"), (GS, "GS")))
+    code, C = _aff_plan(T, N, mode, C)
     lib = _n.lib()
     P = lib.lsh_lif_param_partials(T, N, code, C)
     if P < 0:
@@ -195,8 +199,38 @@ class LIFAffineFn(torch.autograd.Function):
         return (lam, b * lam[0] if need[1] else None, db, dg, dd, None, None, None, None, None)
 
 
+def _cpp_layer_u0(I, u0, mode, C, K, *fixed):
+    """hip_lif._cpp_u0 for a layer of the given mode and chunks, or None where the call is one that
+    the Python functions refuse."""
+    u0v = L._cpp_u0(I, u0, *fixed)
+    if u0v is None or (mode == "scan" and not (int(C) >= 1 and I.shape[0] % int(C) == 0
+                                               and 1 <= int(K) <= 32)):
+        return None
+    return u0v
+
+
+def _cpp_layer(I, u0, params, c, soft, mode, C, K, code, Cb):
+    """The affine or soft layer's C++ autograd function; c: beta, theta, gamma, delta, alpha."""
+    global _LAST_AFF
+    C, K = (int(C), int(K)) if mode == "scan" else (0, 0)
+    T, N = I.shape
+    ws = _n.workspace(_n.lib().lsh_aff_scan_workspace(T, N, C, K) if C else 0, I.device)
+    S = _n.ops().aff_layer(I, u0, *map(L._grad_param, params), c, soft, ws, C, K, code, Cb)
+    if C:
+        _LAST_AFF = _AffRun(ws, T, N, C, K)
+    return S
+
+
 def lif_affine(I, u0, beta, gamma, delta, theta=1.0, alpha=4.0, mode="scan", C=128, K=32):
     """triton_affine.py:245-246: spikes S [T, N]; mode "scan" (the two-level scan with the
     reference's default repair = 0: chunk starts from the verified maps, serial fallback on a
     miss) or "serial"."""
+    u0v = _cpp_layer_u0(I, u0, mode, C, K, theta, alpha)
+    T, N = I.shape
+    if u0v is not None and (T < L.AUTO_BWD_MIN_T or L._chunk_or_none(T, 2) is not None):
+        code, Cb = _aff_plan(T, N)
+        if code != 1:  # the same kernels as LIFAffineFn's, from C++
+            b, g, dl, th = _f32s(beta, gamma, delta, theta)
+            return _cpp_layer(I, u0v, (beta, gamma, delta), (b, th, _gamma(g), dl, float(alpha)), False,
+                              mode, C, K, code, Cb)
     return LIFAffineFn.apply(I, u0, beta, gamma, delta, theta, alpha, mode, C, K)

@@ -57,6 +57,11 @@ def _f32s(*xs):
            (None if i in dev else float(x)) for i, x in enumerate(xs)]
     if len(dev) == 1:
         out[dev[0]] = float(xs[dev[0]].detach().item())
+    elif dev and _n.ops() is not None and all(
+            xs[i].numel() == 1 and xs[i].is_floating_point() and xs[i].device == xs[dev[0]].device
+            and xs[i].dtype == xs[dev[0]].dtype for i in dev):
+        for i, v in zip(dev, _n.ops().read_scalars([xs[i] for i in dev])):
+            out[i] = v
     elif dev:
         vals = torch.stack([xs[i].detach().reshape(()).to(torch.float64) for i in dev]).cpu().tolist()
         for i, v in zip(dev, vals):
@@ -1287,41 +1292,60 @@ class LIFTuned(torch.autograd.Function):
                 None, None, None, None, None, None)
 
 
-_RC_OK = {}
+def _untransformed():
+    """True when neither forward-mode differentiation, a function transform nor a trace is looking at
+    the calls: the C++ functions and the calls outside autograd are for plain ones."""
+    return (torch.autograd.forward_ad._current_level < 0
+            and not torch._C._are_functorch_transforms_active()
+            and torch._C._get_tracing_state() is None)
 
 
-def _rc_path(I, u0, beta, mode, K, repair):
-    """u0 as the [N] vector of the C++ recomputing pair (lifscan/_ops.cpp) when lif_tuned can take
-    it: the recomputing pair applies, beta needs no gradient, u0 is already the layer's [N] fp32
-    vector (or needs none) and the module is built; else None."""
-    if mode == "serial" or CHECK_WAITS or not torch.is_tensor(I) or I.dim() != 2:
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def _cpp_u0(I, u0, *fixed):
+    """u0 as the [N] vector of the C++ autograd functions (lifscan/_ops.cpp) when a layer call can
+    take them: the module is built, I is an fp32 [T, N] GPU tensor with elements, u0 is already the
+    layer's [N] fp32 vector (or needs no gradient), none of the fixed parameters asks for a gradient
+    and the call is a plain one; else None (the Python functions take, or refuse, everything else)."""
+    if type(I) not in _PLAIN_TYPES or I.dim() != 2 or not I.is_cuda or I.dtype != torch.float32:
         return None
-    if not I.is_cuda or I.dtype != torch.float32:
+    if CHECK_WAITS or I.numel() == 0 or _n.ops() is None or not _untransformed():
         return None
-    if torch.is_tensor(beta) and beta.requires_grad:
+    if any(_grad_param(p) is not None for p in fixed):
+        return None
+    if torch.is_tensor(u0):
+        if type(u0) not in _PLAIN_TYPES:
+            return None
+        if not (u0.dim() == 1 and u0.shape[0] == I.shape[1] and u0.dtype == torch.float32
+                and u0.device == I.device and u0.is_contiguous()) and (
+                u0.requires_grad or u0.numel() != I.shape[1]):
+            return None
+    return _vec(u0, I.shape[1], I)
+
+
+def _grad_param(p):
+    """A parameter as the C++ functions take it: the tensor when it wants a gradient, else None."""
+    return p if torch.is_tensor(p) and p.requires_grad else None
+
+
+def _rc_path(I, u0, beta, mode, K, repair, *fixed):
+    """u0 as the [N] vector when lif_tuned takes the C++ layer (_cpp_u0) over the recomputing pair
+    of a converged forward, else None."""
+    if mode == "serial":
+        return None
+    u0v = _cpp_u0(I, u0, *fixed)
+    if u0v is None or not _layer_ok(I.shape[1]):
         return None
     T, N = I.shape
-    key = (T, N, int(K), int(repair))
-    ok = _RC_OK.get(key)
-    if ok is None:
-        ok = _RC_OK[key] = _recompute_ok(T, N, K, repair)
-    if not ok:
-        return None
-    if (torch.is_tensor(u0) and u0.dim() == 1 and u0.shape[0] == N and u0.dtype == torch.float32
-            and u0.device == I.device and u0.is_contiguous()):
-        u0v = u0
-    elif torch.is_tensor(u0) and u0.requires_grad:
-        return None
-    else:
-        u0v = _vec(u0, N, I)
-    return u0v if _n.ops() is not None else None
+    return u0v if _recompute_ok(T, N, K, repair) or _converged_layer(T, N, beta, K, repair) else None
 
 
 def lif_tuned(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, mode="scan", K=16, repair=0):
-    u0v = _rc_path(I, u0, beta, mode, K, repair)
-    if u0v is not None:  # the same kernels and bits as LIFTuned's recomputing pair, from C++
-        return _n.ops().lif_tuned_rc(I, u0v, _f32(beta), float(theta), float(u_r), float(alpha),
-                                     _wait_header(I.device), FUSED_FWD_C)
+    u0v = _rc_path(I, u0, beta, mode, K, repair, theta, u_r, alpha)
+    if u0v is not None:  # the same kernels and bits as LIFTuned's recomputing pairs, from C++
+        return _n.ops().lif_layer(I, u0v, _grad_param(beta), None, None, *_f32s(beta, theta, u_r),
+                                  _f32(alpha), _wait_header(I.device), 0, 0)
     return LIFTuned.apply(I, u0, beta, theta, u_r, alpha, mode, K, repair)
 
 
@@ -1373,22 +1397,20 @@ class LIFAuto(torch.autograd.Function):
                 None, None, None, None, None, None, None)
 
 
-def _plain_call(*tensors):
-    """True when a layer call needs no autograd function: no gradient is recorded, and neither
-    forward-mode differentiation nor a function transform is looking."""
-    if torch.is_grad_enabled() and any(torch.is_tensor(t) and t.requires_grad for t in tensors):
-        return False
-    return (torch.autograd.forward_ad._current_level < 0
-            and not torch._C._are_functorch_transforms_active())
-
-
 def lif_auto(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, K=16, repair=0):
     T, N = I.shape
-    if _layer_ok(N) and T > 0 and _plain_call(I, u0, beta) and (
-            not torch.is_tensor(u0) or (u0.dim() == 1 and u0.shape[0] == N)):
-        b = _f32(beta)
-        if not _auto_states(T, N, b):  # spikes alone
-            return _layer_forward(I, b, theta, u_r, u0, want_states=False)[0]
+    if _layer_ok(N) and T > 0:
+        u0v = _cpp_u0(I, u0, theta, u_r, alpha)
+        if u0v is not None:  # the same kernels and bits as LIFAuto's layer pair, from C++
+            b, th, ur = _f32s(beta, theta, u_r)
+            if not _auto_states(T, N, b):
+                hdr = _wait_header(I.device)
+                if torch.is_grad_enabled() and (I.requires_grad or u0v.requires_grad
+                                                or _grad_param(beta) is not None):
+                    return _n.ops().lif_layer(I, u0v, _grad_param(beta), None, None, b, th, ur,
+                                              _f32(alpha), hdr, 0, 0)
+                return _n.ops().lif_spikes(I, u0v, b, th, ur, hdr)
+            beta, theta, u_r = (b if _grad_param(beta) is None else beta), th, ur  # read once
     fwd, bwd = auto_modes(N, T)
     fwd, bwd = _auto_fwd(fwd, N, T), _auto_bwd(bwd, N, T)
     if not _layer_ok(N) and fwd == bwd:  # one mode for both passes: lif_tuned's path

@@ -277,6 +277,12 @@ int lsh_lif_layer_bwd(const float* I, const float* STARTS, const float* GS, floa
                       double* partials, int64_t T, int64_t N, float beta, float theta, float u_r,
                       float alpha, void* ws, size_t ws_bytes, void* stream);
 
+/* What is left of a layer's backward after its adjoint, in one launch: sums[k] = s_k times the sum
+ * of column k of partials [P][cols] (cols 1 or 3; fp64 sums in a fixed order, rounded to fp32 once;
+ * sums NULL: none) and du0[n] = beta * Lam0[n], Lam0 the adjoint's first row (du0 NULL: none). */
+int lsh_layer_grads(const double* partials, int64_t P, int cols, double s0, double s1, double s2,
+                    float* sums, const float* Lam0, int64_t N, float beta, float* du0, void* stream);
+
 /* ---------------------------------------------------------------------------------------
  * ALIF: v = fl(fl(beta*u) + x); s = v >= fl(theta0 + w); u' = s ? u_r : v;
  *       w' = s ? fl(fl(rho*w) + q) : fl(rho*w)          (triton_alif.py:26-31)
