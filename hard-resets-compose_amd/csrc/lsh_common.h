@@ -56,33 +56,40 @@ __device__ __forceinline__ float lane_f(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-// L serial LIF steps of column n from row r0, for a walk with one wave per neuron (every lane
+// A LIF step for long serial walks, carried by p = fl(beta*u): v = fl(p + x), and the next p is
+// kr = fl(beta*u_r) after a spike, else fl(beta*v).  lif_step's values bit for bit, but the product
+// runs beside the threshold test, so the dependent chain of a step is sum, product, selection
+// where carrying u also waits for the test.
+__device__ __forceinline__ float lif_walk(float& p, float x, float beta, float theta, float kr) {
+  const float v = __fadd_rn(p, x);
+  const float bv = __fmul_rn(beta, v);
+  p = v >= theta ? kr : bv;
+  return v;
+}
+
+// L >= 1 serial LIF steps of column n from row r0, for a walk with one wave per neuron (every lane
 // holds the same state u): the rows are read 64 at a time, one per lane, the next 64 (index
 // clamped to the last row) while a block is walked, and each step takes its input from its lane.
-// The same step arithmetic as the replay.
+// The same values as the replay's.
 __device__ __forceinline__ float wave_serial_rows(const float* __restrict__ I, int64_t N,
                                                   int64_t n, int64_t r0, int64_t L, float u,
                                                   float beta, float theta, float u_r) {
   const int lane = threadIdx.x & 63;
   const float* Ip = I + (size_t)r0 * N + n;
+  const float kr = __fmul_rn(beta, u_r);
+  float p = __fmul_rn(beta, u), v = 0.0f;
   float xv = Ip[(size_t)min<int64_t>(lane, L - 1) * N];
   for (int64_t t0 = 0; t0 < L; t0 += 64) {
     const float xn = Ip[(size_t)min<int64_t>(t0 + 64 + lane, L - 1) * N];
     if (L - t0 >= 64) {
-#pragma unroll 16
-      for (int j = 0; j < 64; ++j) {
-        bool s;
-        u = lif_step(u, lane_f(xv, j), beta, theta, u_r, s);
-      }
+#pragma unroll
+      for (int j = 0; j < 64; ++j) v = lif_walk(p, lane_f(xv, j), beta, theta, kr);
     } else {
-      for (int j = 0; j < (int)(L - t0); ++j) {
-        bool s;
-        u = lif_step(u, lane_f(xv, j), beta, theta, u_r, s);
-      }
+      for (int j = 0; j < (int)(L - t0); ++j) v = lif_walk(p, lane_f(xv, j), beta, theta, kr);
     }
     xv = xn;
   }
-  return u;
+  return v >= theta ? u_r : v;
 }
 
 // Neuron of workgroup b for kernels with one wave per neuron: eight contiguous ranges, range x

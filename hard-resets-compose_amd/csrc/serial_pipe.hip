@@ -164,30 +164,38 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_bwd_pipe(
 }
 
 // The two serial forwards' steps: hard reset (triton_lif.py:21-25) and affine reset
-// (triton_affine.py:20-24), with the one-wave kernels' arithmetic (lif_step, aff_step).
-// spike(u, x): the step's threshold decision from the state before it, with the step's own
-// operations (the producers recompute S with it).
+// (triton_affine.py:20-24), with the values of the one-wave kernels' lif_step and aff_step.  A step
+// takes the carried value p (start(u) from a state u) to the next one and gives its potential v;
+// after(v) is the state u it leaves, spike(v) its decision.
 struct LifStep {
-  float beta, theta, u_r;
-  __device__ __forceinline__ float operator()(float u, float x, bool& s) const {
-    return lif_step(u, x, beta, theta, u_r, s);
+  float beta, theta, u_r, kr;
+  LifStep(float b, float t, float r) : beta(b), theta(t), u_r(r), kr(b * r) {}
+  __device__ __forceinline__ float start(float u) const { return __fmul_rn(beta, u); }
+  __device__ __forceinline__ float operator()(float& p, float x) const {
+    return lif_walk(p, x, beta, theta, kr);
   }
-  __device__ __forceinline__ bool spike(float u, float x) const { return lif_v(u, x, beta) >= theta; }
+  __device__ __forceinline__ float after(float v) const { return v >= theta ? u_r : v; }
+  __device__ __forceinline__ bool spike(float v) const { return v >= theta; }
 };
 struct AffStep {
   float beta, theta, gamma, delta;
-  __device__ __forceinline__ float operator()(float u, float x, bool& s) const {
-    return aff_step(u, x, beta, theta, gamma, delta, s);
+  __device__ __forceinline__ float start(float u) const { return u; }
+  __device__ __forceinline__ float operator()(float& p, float x) const {
+    const float v = lif_v(p, x, beta);
+    p = after(v);
+    return v;
   }
-  __device__ __forceinline__ bool spike(float u, float x) const { return lif_v(u, x, beta) >= theta; }
+  __device__ __forceinline__ float after(float v) const {
+    return v >= theta ? __fadd_rn(__fmul_rn(gamma, v), delta) : v;
+  }
+  __device__ __forceinline__ bool spike(float v) const { return v >= theta; }
 };
 
 // Serial forward from u0 (triton_lif.py:30-39 serial_fwd_kernel, :460-466
 // serial_forward_tiled; triton_affine.py:143-162): tiles in time order; the consumer runs the
-// step and writes u per step (and each tile's entry state), the producers stage I into LDS one
-// tile ahead and store U, S of the tile finished one round earlier, recomputing each spike
-// from the state before it and their own loaded rows (kept two rounds in registers) with the
-// step's operations, so the consumer's chain carries no spike-to-float select.
+// recurrence and writes v per step (and each tile's entry state), the producers stage I into LDS
+// one tile ahead and store U, S of the tile finished one round earlier, both from its v, so the
+// consumer's chain carries neither the selection of u nor a spike-to-float select.
 // SO: no U; `U` is [ceil(T/32), N] and receives the state before rows 0, 32, 64, ... (NULL: not
 // wanted), so the spikes alone are written per step.
 template <class Step, bool NT, bool SO = false>
@@ -196,7 +204,7 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
     float* __restrict__ S, int64_t N, int64_t T, Step step) {
   constexpr int D = PIPE_FD, P = PIPE_P, R = PIPE_FR;
   __shared__ float sX[2][D][WAVE];
-  __shared__ float sU[2][D][WAVE];
+  __shared__ float sV[2][D][WAVE];
   __shared__ float sEntry[2][WAVE];  // u before row 0 of the tile in the same buffer
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const unsigned lane = threadIdx.x % WAVE;
@@ -209,12 +217,13 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
 
   if (w == 0) {  // consumer: tile k - 1 in round k
     __builtin_amdgcn_s_setprio(3);
-    float u = u0[nb0 + ln];
+    const float u = u0[nb0 + ln];
+    float p = step.start(u), v = 0.0f;
     for (int64_t k = 0; k <= ntiles + 1; ++k) {
       if (k >= 1 && k <= ntiles) {
         const int buf = (int)((k - 1) & 1);
         const int nr = rows(k - 1);
-        sEntry[buf][lane] = u;
+        if constexpr (SO) sEntry[buf][lane] = k == 1 ? u : step.after(v);
         if (nr == D) {
 #pragma unroll
           for (int g = 0; g < D; g += 16) {
@@ -223,16 +232,14 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
             for (int i = 0; i < 16; ++i) x[i] = sX[buf][g + i][lane];
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-              bool sp;
-              u = step(u, x[i], sp);
-              sU[buf][g + i][lane] = u;
+              v = step(p, x[i]);
+              sV[buf][g + i][lane] = v;
             }
           }
         } else {
           for (int j = 0; j < nr; ++j) {
-            bool sp;
-            u = step(u, sX[buf][j][lane], sp);
-            sU[buf][j][lane] = u;
+            v = step(p, sX[buf][j][lane]);
+            sV[buf][j][lane] = v;
           }
         }
       }
@@ -241,13 +248,9 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
     return;
   }
 
-  // producers: I of tile k into LDS (loaded one round ahead) and U, S of tile k - 2 in round k;
-  // xr: the rows of the tile being loaded; at the start of round k, x1 and x2 hold this
-  // producer's rows of tiles k - 1 and k - 2
+  // producers: I of tile k into LDS (loaded one round ahead) and U, S of tile k - 2 in round k
   const int p = w - 1;
-  float xr[R], x1[R], x2[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) xr[r] = x1[r] = x2[r] = 0.0f;
+  float xr[R];
   auto load = [&](int64_t k) {
     const int nr = rows(k);
 #pragma unroll
@@ -258,9 +261,6 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
   };
   if (ntiles > 0) load(0);
   for (int64_t k = 0; k <= ntiles + 1; ++k) {
-    float xk[R];  // this producer's rows of tile k
-#pragma unroll
-    for (int r = 0; r < R; ++r) xk[r] = xr[r];
     if (k < ntiles) {
       const int buf = (int)(k & 1);
       const int nr = rows(k);
@@ -279,22 +279,18 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
         const int j = p + r * P;
         if (j < nr) {
           const size_t row = (size_t)((k - 2) * D + j) * (size_t)N + (size_t)nb0;
-          const float up = j == 0 ? sEntry[buf][lane] : sU[buf][j - 1][lane];
+          const float v = sV[buf][j][lane];
           if constexpr (SO) {
             static_assert(D % 32 == 0, "the states fall on rows 0, 32, ... of a tile");
             if (j % 32 == 0 && U != nullptr)
-              st_row<NT>(U + (size_t)((k - 2) * (D / 32) + j / 32) * (size_t)N + (size_t)nb0, sb, up);
+              st_row<NT>(U + (size_t)((k - 2) * (D / 32) + j / 32) * (size_t)N + (size_t)nb0, sb,
+                         j == 0 ? sEntry[buf][lane] : step.after(sV[buf][j - 1][lane]));
           } else {
-            st_row<NT>(U + row, sb, sU[buf][j][lane]);
+            st_row<NT>(U + row, sb, step.after(v));
           }
-          st_row<NT>(S + row, sb, step.spike(up, x2[r]) ? 1.0f : 0.0f);
+          st_row<NT>(S + row, sb, step.spike(v) ? 1.0f : 0.0f);
         }
       }
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      x2[r] = x1[r];
-      x1[r] = xk[r];
     }
     __syncthreads();
   }
@@ -305,7 +301,7 @@ void lif_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, in
   const int NB = (int)((N + WAVE - 1) / WAVE);
   with_store_policy(N, [&](auto nt) {
     hipLaunchKernelGGL((k_serial_fwd_pipe<LifStep, decltype(nt)::value>), dim3((unsigned)NB),
-                       dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, U, S, N, T, LifStep{beta, theta, u_r});
+                       dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, U, S, N, T, LifStep(beta, theta, u_r));
   });
 }
 
@@ -315,7 +311,7 @@ void lif_starts_fwd_pipe(const float* I, const float* u0, float* STARTS, float* 
   with_store_policy(N, [&](auto nt) {
     hipLaunchKernelGGL((k_serial_fwd_pipe<LifStep, decltype(nt)::value, true>), dim3((unsigned)NB),
                        dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, STARTS, S, N, T,
-                       LifStep{beta, theta, u_r});
+                       LifStep(beta, theta, u_r));
   });
 }
 
