@@ -1,9 +1,10 @@
 // C++ autograd functions of the layers over the lifscan C ABI: a layer step costs one Python -> C++
 // crossing in the forward and none in the backward.  (A Python autograd function's backward takes
-// the interpreter lock on the engine's thread and makes some ten small torch calls.  A step of a 1000 x
-// 12800 layer: 122 -> 57 us; 512 x 1024: 116 -> 38 us; a 49999 x 64 parameter fit 254 -> 132 us.)  They launch the kernels that the Python
-// functions of the same layers launch (lifscan/hip_lif.py, hip_affine.py, fit.py); the parameter
-// sums and dL/du0 are finished by one kernel (lsh_layer_grads).
+// the interpreter lock on the engine's thread and makes some ten small torch calls.  A step of a
+// 1000 x 12800 layer: 122 -> 57 us; 512 x 1024: 116 -> 38 us; a 50000 x 64 parameter fit 254 -> 132
+// us.)  They launch the kernels that the Python functions of the same layers launch
+// (lifscan/hip_lif.py, hip_affine.py, fit.py); the parameter sums and dL/du0 are finished by one
+// kernel (lsh_layer_grads).
 // Reference: triton_lif.py:654-687 (LIFTuned), :1003-1026 (LIFAuto), fit.py:15-57 (LIFParamFn),
 // :121-153 (LIFSoftScanFn), triton_affine.py:214-246 (LIFAffineFn).
 // The entry points' addresses are handed over once from the library the Python package has loaded

@@ -44,6 +44,8 @@ AUTO_BWD_WIDE_MIN_T = 256
 # ----------------------------------------------------------------------------- helpers
 def _f32(x):
     """Scalar parameter as a Python float (the kernels take fp32)."""
+    if type(x) is float:
+        return x
     if torch.is_tensor(x):
         return float(x.detach().item())
     return float(x)
@@ -52,6 +54,8 @@ def _f32(x):
 def _f32s(*xs):
     """Several scalar parameters as Python floats with at most one device-to-host transfer
     (each .item() on a GPU tensor is a synchronizing copy)."""
+    if all(type(x) is float for x in xs):
+        return xs
     dev = [i for i, x in enumerate(xs) if torch.is_tensor(x) and x.device.type != "cpu"]
     out = [float(x.detach().item()) if torch.is_tensor(x) and i not in dev else
            (None if i in dev else float(x)) for i, x in enumerate(xs)]
@@ -1292,12 +1296,16 @@ class LIFTuned(torch.autograd.Function):
                 None, None, None, None, None, None)
 
 
+_FORWARD_AD = torch.autograd.forward_ad
+_functorch_active = torch._C._are_functorch_transforms_active
+_tracing_state = torch._C._get_tracing_state
+
+
 def _untransformed():
     """True when neither forward-mode differentiation, a function transform nor a trace is looking at
     the calls: the C++ functions and the calls outside autograd are for plain ones."""
-    return (torch.autograd.forward_ad._current_level < 0
-            and not torch._C._are_functorch_transforms_active()
-            and torch._C._get_tracing_state() is None)
+    return (_FORWARD_AD._current_level < 0 and not _functorch_active()
+            and _tracing_state() is None)
 
 
 _PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
@@ -1312,21 +1320,24 @@ def _cpp_u0(I, u0, *fixed):
         return None
     if CHECK_WAITS or I.numel() == 0 or _n.ops() is None or not _untransformed():
         return None
-    if any(_grad_param(p) is not None for p in fixed):
+    for p in fixed:
+        if _grad_param(p) is not None:
+            return None
+    N = I.shape[1]
+    if type(u0) in _PLAIN_TYPES:
+        if (u0.dim() == 1 and u0.shape[0] == N and u0.dtype == torch.float32
+                and u0.device == I.device and u0.is_contiguous()):
+            return u0
+        if u0.requires_grad or u0.numel() != N:
+            return None
+    elif torch.is_tensor(u0):
         return None
-    if torch.is_tensor(u0):
-        if type(u0) not in _PLAIN_TYPES:
-            return None
-        if not (u0.dim() == 1 and u0.shape[0] == I.shape[1] and u0.dtype == torch.float32
-                and u0.device == I.device and u0.is_contiguous()) and (
-                u0.requires_grad or u0.numel() != I.shape[1]):
-            return None
-    return _vec(u0, I.shape[1], I)
+    return _vec(u0, N, I)
 
 
 def _grad_param(p):
     """A parameter as the C++ functions take it: the tensor when it wants a gradient, else None."""
-    return p if torch.is_tensor(p) and p.requires_grad else None
+    return p if type(p) is not float and torch.is_tensor(p) and p.requires_grad else None
 
 
 def _rc_path(I, u0, beta, mode, K, repair, *fixed):
