@@ -59,7 +59,9 @@ __device__ __forceinline__ float lane_f(float v, int lane) {
 // A LIF step for long serial walks, carried by p = fl(beta*u): v = fl(p + x), and the next p is
 // kr = fl(beta*u_r) after a spike, else fl(beta*v).  lif_step's values bit for bit, but the product
 // runs beside the threshold test, so the dependent chain of a step is sum, product, selection
-// where carrying u also waits for the test.
+// where carrying u also waits for the test.  Measured, u -> p: three-level scan of 65536 x 1024 (C 64,
+// G 16), super carry with 45 of 64 maps falling back 427 -> 363 us; serial forward (with v written
+// in u's place) 8000 x 1024 148 -> 143 us, 1000 x 8192 24.1 -> 23.3 us.
 __device__ __forceinline__ float lif_walk(float& p, float x, float beta, float theta, float kr) {
   const float v = __fadd_rn(p, x);
   const float bv = __fmul_rn(beta, v);
