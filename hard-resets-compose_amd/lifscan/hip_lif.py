@@ -61,9 +61,9 @@ def _f32s(*xs):
            (None if i in dev else float(x)) for i, x in enumerate(xs)]
     if len(dev) == 1:
         out[dev[0]] = float(xs[dev[0]].detach().item())
-    elif dev and _n.ops() is not None and all(
-            xs[i].numel() == 1 and xs[i].is_floating_point() and xs[i].device == xs[dev[0]].device
-            and xs[i].dtype == xs[dev[0]].dtype for i in dev):
+    elif dev and _n.ops() is not None and _untransformed() and all(
+            type(xs[i]) in _PLAIN_TYPES and xs[i].numel() == 1 and xs[i].is_floating_point()
+            and xs[i].device == xs[dev[0]].device and xs[i].dtype == xs[dev[0]].dtype for i in dev):
         for i, v in zip(dev, _n.ops().read_scalars([xs[i] for i in dev])):
             out[i] = v
     elif dev:

@@ -94,6 +94,23 @@ def test_calls_that_stay_with_the_python_functions(dev):
         assert L._cpp_u0(I, u0) is None
 
 
+def test_parameters_under_a_function_transform(dev):
+    """Parameters that a transform has wrapped have no storage of their own to copy; the scans read
+    their values as those of any other constant."""
+    from lifscan import hip_lif as L
+    I, _, u0 = _data(64, 32, dev)
+    want = L.serial_forward(I, 0.95, 1.0, 0.05, u0)
+    got = []
+
+    def loss(p):
+        got.append(L._f32s(p[0], p[1], p[2]))
+        return p.sum()
+
+    torch.func.grad(loss)(torch.tensor([0.95, 1.0, 0.05], device=dev))
+    assert got[0] == tuple(torch.tensor([0.95, 1.0, 0.05]).tolist())
+    assert all(map(torch.equal, L.serial_forward(I, *got[0], u0), want))
+
+
 @pytest.mark.parametrize("P,cols,N", [(0, 3, 5), (1, 1, 1), (511, 3, 512), (513, 1, 513), (70001, 3, 64)])
 def test_layer_grads_kernel(dev, P, cols, N):
     from lifscan import _native as n
