@@ -801,7 +801,7 @@ __global__ __launch_bounds__(256) void k_lif_repair(const float* __restrict__ I,
                                                     float* __restrict__ starts,
                                                     float* __restrict__ ends, int* __restrict__ list0,
                                                     int* __restrict__ list1, WsHeader* hdr,
-                                                    int64_t T, int64_t N, int M, int C, int64_t R,
+                                                    int64_t N, int M, int C, int64_t R,
                                                     float beta, float theta, float u_r) {
   __shared__ int s_nd, s_nc;
   const int nb = blockIdx.x;
@@ -844,8 +844,7 @@ __global__ __launch_bounds__(256) void k_lif_repair(const float* __restrict__ I,
       // function of the state and the input), so the replay stops there and the chunk's end
       // is unchanged: exact, and the round gives the same states as a full re-replay.
       const bool met = stream_rows_until<16>(
-          I + base, U + base, (size_t)N, min<int64_t>(C, T - (int64_t)m * C),
-          [&](int64_t j, float x, float u_old) {
+          I + base, U + base, (size_t)N, C, [&](int64_t j, float x, float u_old) {
             bool s;
             u = lif_step(u, x, beta, theta, u_r, s);
             U[base + (size_t)j * N] = u;
@@ -1267,7 +1266,7 @@ void lif_replay_repair_done_launch(const float* I, float* U, float* S, float* st
                                    int64_t repair, float beta, float theta, float u_r,
                                    hipStream_t st, const int* done) {
   launch_fwd_auto(I, starts, U, S, ends, N, C, M, beta, theta, u_r, st, done);
-  lif_repair_launch(I, U, S, starts, ends, list0, list1, hdr, (int64_t)M * C, N, M, C, repair, beta, theta, u_r,
+  lif_repair_launch(I, U, S, starts, ends, list0, list1, hdr, N, M, C, repair, beta, theta, u_r,
                     st);
 }
 
@@ -1314,7 +1313,7 @@ static int repair_seg_count(int NB, int M) {
 
 // The device repair rounds alone, after a replay that wrote U, S and ends from starts.
 void lif_repair_launch(const float* I, float* U, float* S, float* starts, float* ends, int* list0,
-                       int* list1, WsHeader* hdr, int64_t T, int64_t N, int M, int C, int64_t repair,
+                       int* list1, WsHeader* hdr, int64_t N, int M, int C, int64_t repair,
                        float beta, float theta, float u_r, hipStream_t st) {
   if (repair < 0 && M > 1) {
     // To convergence without the round count.  The ordered pass costs about 3-4 us per 16-row
@@ -1356,7 +1355,7 @@ void lif_repair_launch(const float* I, float* U, float* S, float* starts, float*
     const int64_t rounds = repair < (int64_t)M ? repair : (int64_t)M;
     const int NB = (int)((N + WAVE - 1) / WAVE);
     hipLaunchKernelGGL(k_lif_repair, dim3((unsigned)NB), dim3(256), 0, st, I, U, S, starts, ends,
-                       list0, list1, hdr, T, N, M, C, rounds, beta, theta, u_r);
+                       list0, list1, hdr, N, M, C, rounds, beta, theta, u_r);
   }
 }
 

@@ -19,12 +19,14 @@
 //                   from its predecessor's exit, stopping as soon as it meets the trajectory
 //                   already stored for it, so a wrong prediction costs only the steps until the
 //                   two trajectories coalesce;
-//   k_lif_repair    (lif_kernels.hip) the device repair of the two-level scan, with the same
-//                   early stop, until no chunk's start differs from its predecessor's exit.
+//   k_lif_warm_finish   (serial_pipe.hip) more rounds per 64 neurons, with the same early stop, while
+//                   they are cheap, then the serial sweep from the first chunk whose start still
+//                   differs from its predecessor's exit.
 //
-// The result is the serial recurrence bit for bit (the repair's fixed point is the serial
-// trajectory; M rounds always reach it), the result of scan_forward_v3 (triton_lif.py:782-817)
-// with repair >= T/C.  Traffic: I read over W + C rows per chunk (the warm-up rows are the
+// The result is the serial recurrence bit for bit, the result of scan_forward_v3
+// (triton_lif.py:782-817) with repair >= T/C, in at most about the warm pass and one serial sweep:
+// under a nearly constant current trajectories of different phase never spike together, and every
+// prediction is wrong.  Traffic: I read over W + C rows per chunk (the warm-up rows are the
 // previous chunk's, read at the same time by that chunk's wave, so mostly from cache), U and S
 // written once: 12 B per neuron-step from HBM when the re-read hits.  No chunk maps, no carry.
 #include "lsh_abi.h"
@@ -91,8 +93,8 @@ __global__ __launch_bounds__(64) void k_lif_count_missed(const float* __restrict
 // missed predictions this spreads their replays over the whole chip instead of one workgroup
 // per 64 neurons.  A chunk may read its predecessor's exit before or after the predecessor's
 // own replay in this round rewrites it; either way it replays a consistent trajectory from the
-// value it read and records that value as its start, and the per-block repair that follows
-// checks every chunk again, so the result is the same fixed point (the serial recurrence).
+// value it read and records that value as its start, and k_lif_warm_finish checks every chunk
+// again.
 __global__ __launch_bounds__(64) void k_lif_repair_wide(const float* __restrict__ I,
                                                         float* __restrict__ U,
                                                         float* __restrict__ S,
@@ -105,7 +107,7 @@ __global__ __launch_bounds__(64) void k_lif_repair_wide(const float* __restrict_
   const int64_t n = (int64_t)nb * WAVE + threadIdx.x;
   if (n >= N) return;
   const float prev = __builtin_nontemporal_load(ends + (size_t)(m - 1) * N + n);
-  if (prev == starts[(size_t)m * N + n]) return;
+  if (same_bits(prev, starts[(size_t)m * N + n])) return;
   starts[(size_t)m * N + n] = prev;
   float u = prev;
   const size_t base = (size_t)m * C * N + n;
@@ -169,18 +171,16 @@ static int warm_run(const float* I, const float* u0, float* U, float* S, int64_t
     hipLaunchKernelGGL((k_lif_fwd_warm<decltype(nt)::value>), dim3((unsigned)((int64_t)M * NB)), dim3(WAVE), 0, st, I, u0, U, S,
                      starts, ends, T, N, C, W, NB, beta, theta, u_r);
   });
-  // The per-block repair counts the missed predictions, so count them here first (the wide
-  // round fixes most of them before that repair looks).
+  // the missed predictions are counted before the wide round fixes most of them
   if (M > 1) {
     const dim3 rest((unsigned)((int64_t)(M - 1) * NB));
     if (count)
       hipLaunchKernelGGL(k_lif_count_missed, rest, dim3(WAVE), 0, st, starts, ends, h, N, NB);
     hipLaunchKernelGGL(k_lif_repair_wide, rest, dim3(WAVE), 0, st, I, U, S, starts, ends, T, N, C, NB,
                        beta, theta, u_r);
+    lif_warm_finish_launch(I, U, S, starts, ends, reinterpret_cast<int*>(w + L.LIST0),
+                           reinterpret_cast<int*>(w + L.LIST1), h, T, N, M, C, beta, theta, u_r, st);
   }
-  lif_repair_launch(I, U, S, starts, ends, reinterpret_cast<int*>(w + L.LIST0),
-                    reinterpret_cast<int*>(w + L.LIST1), h, T, N, M, C, (int64_t)M, beta, theta, u_r,
-                    st);
   LSH_CHECK_LAUNCH();
   return LSH_OK;
 }

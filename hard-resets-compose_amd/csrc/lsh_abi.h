@@ -120,11 +120,16 @@ int lif_starts_bwd_lookback(const float* I, const float* STARTS, const float* GS
 // Device repair rounds of the two-level scan (lif_kernels.hip, k_lif_repair) after a replay that
 // wrote U, S and ends from starts: at most min(repair, M) rounds; list0/list1 hold
 // ceil(N/64)*M*64 ints each.  repair = -1: to convergence without the round count (the ordered
-// pass k_lif_repair_ordered where it is faster, else M rounds).  T = M*C, or with repair >= 0 any
-// T of M = ceil(T/C) chunks (the last one short).
+// pass k_lif_repair_ordered where it is faster, else M rounds).
 void lif_repair_launch(const float* I, float* U, float* S, float* starts, float* ends, int* list0,
-                       int* list1, WsHeader* hdr, int64_t T, int64_t N, int M, int C, int64_t repair,
+                       int* list1, WsHeader* hdr, int64_t N, int M, int C, int64_t repair,
                        float beta, float theta, float u_r, hipStream_t st);
+
+// The repair of the warm-started chunks (serial_pipe.hip, k_lif_warm_finish): M = ceil(T/C) > 1
+// chunks, the last one possibly short; lists as above.
+void lif_warm_finish_launch(const float* I, float* U, float* S, float* starts, float* ends, int* list0,
+                            int* list1, WsHeader* hdr, int64_t T, int64_t N, int M, int C, float beta,
+                            float theta, float u_r, hipStream_t st);
 
 // Fills n ints with v on the stream (lif_lookback.hip; look-back flags).
 void fill_i32_launch(int* p, int64_t n, int v, hipStream_t st);

@@ -191,24 +191,27 @@ struct AffStep {
   __device__ __forceinline__ bool spike(float v) const { return v >= theta; }
 };
 
-// Serial forward from u0 (triton_lif.py:30-39 serial_fwd_kernel, :460-466
-// serial_forward_tiled; triton_affine.py:143-162): tiles in time order; the consumer runs the
-// recurrence and writes v per step (and each tile's entry state), the producers stage I into LDS
-// one tile ahead and store U, S of the tile finished one round earlier, both from its v, so the
-// consumer's chain carries neither the selection of u nor a spike-to-float select.
+// Serial forward over T rows of 64 neurons from the states us (triton_lif.py:30-39
+// serial_fwd_kernel, :460-466 serial_forward_tiled; triton_affine.py:143-162), run by every wave of
+// a workgroup of PIPE_P + 1: tiles in time order; the consumer runs the recurrence and writes v per
+// step (and each tile's entry state), the producers stage I into LDS one tile ahead and store U, S
+// of the tile finished one round earlier, both from its v, so the consumer's chain carries neither
+// the selection of u nor a spike-to-float select.
 // SO: no U; `U` is [ceil(T/32), N] and receives the state before rows 0, 32, 64, ... (NULL: not
 // wanted), so the spikes alone are written per step.
-template <class Step, bool NT, bool SO = false>
-__global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
-    const float* __restrict__ I, const float* __restrict__ u0, float* __restrict__ U,
-    float* __restrict__ S, int64_t N, int64_t T, Step step) {
+struct FwdTiles {
+  float X[2][PIPE_FD][WAVE];
+  float V[2][PIPE_FD][WAVE];
+  float entry[2][WAVE];  // u before row 0 of the tile in the same buffer
+};
+template <class Step, bool NT, bool SO>
+__device__ __forceinline__ void serial_fwd_tiles(FwdTiles& sh, const float* __restrict__ I,
+                                                 const float* us, float* __restrict__ U,
+                                                 float* __restrict__ S, int64_t nb0, int64_t N,
+                                                 int64_t T, Step step) {
   constexpr int D = PIPE_FD, P = PIPE_P, R = PIPE_FR;
-  __shared__ float sX[2][D][WAVE];
-  __shared__ float sV[2][D][WAVE];
-  __shared__ float sEntry[2][WAVE];  // u before row 0 of the tile in the same buffer
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const unsigned lane = threadIdx.x % WAVE;
-  const int64_t nb0 = (int64_t)blockIdx.x * WAVE;
   const bool valid = nb0 + lane < N;
   const unsigned ln = valid ? lane : (unsigned)(N - 1 - nb0);
   const unsigned lb = ln * 4u, sb = lane * 4u;
@@ -217,29 +220,29 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
 
   if (w == 0) {  // consumer: tile k - 1 in round k
     __builtin_amdgcn_s_setprio(3);
-    const float u = u0[nb0 + ln];
+    const float u = us[nb0 + ln];
     float p = step.start(u), v = 0.0f;
     for (int64_t k = 0; k <= ntiles + 1; ++k) {
       if (k >= 1 && k <= ntiles) {
         const int buf = (int)((k - 1) & 1);
         const int nr = rows(k - 1);
-        if constexpr (SO) sEntry[buf][lane] = k == 1 ? u : step.after(v);
+        if constexpr (SO) sh.entry[buf][lane] = k == 1 ? u : step.after(v);
         if (nr == D) {
 #pragma unroll
           for (int g = 0; g < D; g += 16) {
             float x[16];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) x[i] = sX[buf][g + i][lane];
+            for (int i = 0; i < 16; ++i) x[i] = sh.X[buf][g + i][lane];
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
               v = step(p, x[i]);
-              sV[buf][g + i][lane] = v;
+              sh.V[buf][g + i][lane] = v;
             }
           }
         } else {
           for (int j = 0; j < nr; ++j) {
-            v = step(p, sX[buf][j][lane]);
-            sV[buf][j][lane] = v;
+            v = step(p, sh.X[buf][j][lane]);
+            sh.V[buf][j][lane] = v;
           }
         }
       }
@@ -267,7 +270,7 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int j = p + r * P;
-        if (j < nr) sX[buf][j][lane] = xr[r];
+        if (j < nr) sh.X[buf][j][lane] = xr[r];
       }
       if (k + 1 < ntiles) load(k + 1);
     }
@@ -279,12 +282,12 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
         const int j = p + r * P;
         if (j < nr) {
           const size_t row = (size_t)((k - 2) * D + j) * (size_t)N + (size_t)nb0;
-          const float v = sV[buf][j][lane];
+          const float v = sh.V[buf][j][lane];
           if constexpr (SO) {
             static_assert(D % 32 == 0, "the states fall on rows 0, 32, ... of a tile");
             if (j % 32 == 0 && U != nullptr)
               st_row<NT>(U + (size_t)((k - 2) * (D / 32) + j / 32) * (size_t)N + (size_t)nb0, sb,
-                         j == 0 ? sEntry[buf][lane] : step.after(sV[buf][j - 1][lane]));
+                         j == 0 ? sh.entry[buf][lane] : step.after(sh.V[buf][j - 1][lane]));
           } else {
             st_row<NT>(U + row, sb, step.after(v));
           }
@@ -294,6 +297,131 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
     }
     __syncthreads();
   }
+}
+
+template <class Step, bool NT, bool SO = false>
+__global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
+    const float* __restrict__ I, const float* __restrict__ u0, float* __restrict__ U,
+    float* __restrict__ S, int64_t N, int64_t T, Step step) {
+  __shared__ FwdTiles sh;
+  serial_fwd_tiles<Step, NT, SO>(sh, I, u0, U, S, (int64_t)blockIdx.x * WAVE, N, T, step);
+}
+
+// What the warm-started chunks (lif_warm.hip) leave to repair, in linear work: chunks m >= 1 whose
+// start is not the exit of the chunk before are replayed in Jacobi rounds, as k_lif_repair does, while
+// the rounds' replays stay within a budget; then, if a start is still wrong, the rows from the
+// block's first such chunk on are run once more by the serial sweep.  Every chunk below it has the
+// bits of the exit before it as its start, so that exit is exact.  The rounds suit the few misses that
+// noisy inputs leave (each meets its stored trajectory soon); with a nearly constant current no
+// trajectory ever meets another one of a different phase, every round makes one more chunk exact,
+// and rounds alone took M of them, some M^2/2 chunk replays.
+// One workgroup per 64 neurons.  A round of nd replays takes 1 + nd/256 units of the budget: a few
+// lanes walk a row in some 45 ns (the sweep in 17), all 1024 in 250, for their rows lie apart.
+// Measured, N 64, T 50000, beta 0.93 (C 256; the serial sweep alone 0.86 ms), rounds alone -> this:
+// constant current 104.8 -> 0.95 ms, current steps 12.5 -> 0.93 ms, noise 60 -> 39 us (the first
+// comparison by 16 waves instead of 4); N 4096, T 16001, beta 0.95 (C 2000; sweep 0.30 ms) constant
+// current 1.41 -> 0.62 ms.
+constexpr int kWarmScanAhead = 8;  // chunks a wave compares at once
+template <bool NT>
+__global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_warm_finish(
+    const float* __restrict__ I, float* __restrict__ U, float* __restrict__ S, float* starts,
+    float* ends, int* list0, int* list1, WsHeader* hdr, int64_t T, int64_t N, int M, int C,
+    int budget, LifStep step) {
+  constexpr int NW = PIPE_P + 1, NT_ALL = WAVE * NW;
+  __shared__ FwdTiles sh;
+  __shared__ int s_nd, s_nc, s_first;
+  const int tid = threadIdx.x, lane = tid % WAVE;
+  const int64_t nb0 = (int64_t)blockIdx.x * WAVE;
+  const size_t cap = (size_t)M * WAVE;
+  int* dl = list0 + (size_t)blockIdx.x * cap;  // chunks (as m*64 + lane) whose start is wrong
+  int* cl = list1 + (size_t)blockIdx.x * cap;  // successors of chunks whose end changed
+  if (tid == 0) {
+    s_nd = 0;
+    s_first = M;
+  }
+  __syncthreads();
+  {
+    const bool valid = nb0 + lane < N;
+    const int64_t n = valid ? nb0 + lane : N - 1;
+    for (int m0 = 1 + tid / WAVE; m0 < M; m0 += NW * kWarmScanAhead) {
+      float st[kWarmScanAhead], en[kWarmScanAhead];
+#pragma unroll
+      for (int k = 0; k < kWarmScanAhead; ++k) {
+        const size_t o = (size_t)min(m0 + k * NW, M - 1) * N + n;
+        st[k] = starts[o];
+        en[k] = ends[o - N];
+      }
+#pragma unroll
+      for (int k = 0; k < kWarmScanAhead; ++k) {
+        const int m = m0 + k * NW;
+        if (valid && m < M && !same_bits(st[k], en[k])) dl[atomicAdd(&s_nd, 1)] = m * WAVE + lane;
+      }
+    }
+  }
+  __syncthreads();
+  int rounds = 0, nd = s_nd;
+  while (nd > 0) {
+    const int units = 1 + nd / 256;
+    if (units > budget) break;
+    budget -= units;
+    ++rounds;
+    for (int i = tid; i < nd; i += NT_ALL) {
+      const size_t o = (size_t)(dl[i] / WAVE) * N + (size_t)(nb0 + dl[i] % WAVE);
+      starts[o] = ends[o - N];
+    }
+    if (tid == 0) s_nc = 0;
+    __syncthreads();
+    for (int i = tid; i < nd; i += NT_ALL) {
+      const int e = dl[i], m = e / WAVE;
+      const size_t o = (size_t)m * N + (size_t)(nb0 + e % WAVE);
+      const size_t base = (size_t)m * C * N + (size_t)(nb0 + e % WAVE);
+      float u = starts[o];
+      const bool met = stream_rows_until<16>(
+          I + base, U + base, (size_t)N, min<int64_t>(C, T - (int64_t)m * C),
+          [&](int64_t j, float x, float u_old) {
+            bool s;
+            u = lif_step(u, x, step.beta, step.theta, step.u_r, s);
+            U[base + (size_t)j * N] = u;
+            S[base + (size_t)j * N] = s ? 1.0f : 0.0f;
+            return same_bits(u, u_old);
+          });
+      if (!met && !same_bits(u, ends[o])) {
+        ends[o] = u;
+        if (m + 1 < M) cl[atomicAdd(&s_nc, 1)] = e + WAVE;
+      }
+    }
+    if (tid == 0) s_nd = 0;
+    __syncthreads();
+    for (int i = tid; i < s_nc; i += NT_ALL) {
+      const int e = cl[i];
+      const size_t o = (size_t)(e / WAVE) * N + (size_t)(nb0 + e % WAVE);
+      if (!same_bits(ends[o - N], starts[o])) dl[atomicAdd(&s_nd, 1)] = e;
+    }
+    __syncthreads();
+    nd = s_nd;
+  }
+  if (tid == 0) atomicMax(&hdr->repair_iters, (unsigned int)(rounds + (nd > 0 ? 1 : 0)));
+  if (nd == 0) return;
+  for (int i = tid; i < nd; i += NT_ALL) atomicMin(&s_first, dl[i] / WAVE);
+  __builtin_amdgcn_s_waitcnt(0);  // the rounds' stores land before the sweep's to the same rows
+  __syncthreads();
+  const int c0 = s_first;
+  const size_t row0 = (size_t)c0 * C;
+  serial_fwd_tiles<LifStep, NT, false>(sh, I + row0 * N, ends + (size_t)(c0 - 1) * N, U + row0 * N,
+                                       S + row0 * N, nb0, N, T - (int64_t)row0, step);
+}
+
+// The budget of the rounds: M/16 units, a fifth of the serial sweep's time; below 16 chunks the sweep
+// from a wrong start on takes no longer than a round.
+void lif_warm_finish_launch(const float* I, float* U, float* S, float* starts, float* ends, int* list0,
+                            int* list1, WsHeader* hdr, int64_t T, int64_t N, int M, int C, float beta,
+                            float theta, float u_r, hipStream_t st) {
+  const int NB = (int)((N + WAVE - 1) / WAVE);
+  with_store_policy(N, [&](auto nt) {
+    hipLaunchKernelGGL((k_lif_warm_finish<decltype(nt)::value>), dim3((unsigned)NB),
+                       dim3(WAVE * (PIPE_P + 1)), 0, st, I, U, S, starts, ends, list0, list1, hdr, T, N, M,
+                       C, M / 16, LifStep(beta, theta, u_r));
+  });
 }
 
 void lif_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, int64_t N, int64_t T,

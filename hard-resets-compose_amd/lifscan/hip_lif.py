@@ -525,8 +525,9 @@ def scan_forward_warm(I, beta, theta, u_r, u0, C=2048, W=None, stats=None):
     """Converged exact forward by warm-started chunks (lsh_lif_scan_warm_fwd) -> (U, S), the
     serial recurrence: chunk m's entry is predicted by W steps of the recurrence from u_r over
     the rows before it (W defaults to C), every chunk is replayed from its prediction, and the
-    device repair replays the chunks whose prediction missed.  stats receives repair_iters
-    (rounds) and missed_frac (the fraction of chunk entries m >= 1 whose prediction differed
+    device repair replays the chunks whose prediction missed: a round over all chunks, rounds per
+    64 neurons within a budget, then one serial sweep from the first wrong start on.  stats receives
+    repair_iters (the rounds within the budget, and 1 for the sweep) and missed_frac (the fraction of chunk entries m >= 1 whose prediction differed
     from the exit of chunk m-1 replayed from its own prediction, before the repair)."""
     I = _input(I)
     T, N = I.shape

@@ -114,10 +114,11 @@ int lsh_lif_scan_v3_assoc_fwd(const float* I, const float* u0, float* U, float* 
 /* The converged lsh_lif_scan_v3_fwd (repair to convergence, no statistics) by warm-started
  * chunks, for few neurons and long T: the entry state of chunk m >= 1 is predicted by W steps
  * of the recurrence over the W rows before the chunk, started from u_r (from u0 when those rows
- * reach row 0: then it is exact), every chunk is replayed from its prediction, and the device
- * repair of the two-level scan replays each chunk whose prediction differs from its
- * predecessor's replayed exit, stopping where the new trajectory meets the stored one, until
- * nothing changes.  U and S are the serial recurrence bit for bit.  The path of scan_forward_v3
+ * reach row 0: then it is exact), every chunk is replayed from its prediction, and each chunk whose
+ * prediction differs from its predecessor's replayed exit is replayed again, stopping where the new
+ * trajectory meets the stored one, in rounds within a fixed budget; if a start is still wrong then,
+ * the rows from the first such chunk on are swept serially (repair_iters: the rounds within the
+ * budget, and 1 for the sweep).  U and S are the serial recurrence bit for bit.  The path of scan_forward_v3
  * (triton_lif.py:782-817, repair >= T/C) for few neurons and long T; the prediction is the
  * hard-reset analogue of the reference's ALIF warm predictor (triton_alif.py:75-92, :276-285).
  * Requires T % C == 0, C >= 1, W >= 0.  Workspace lsh_lif_scan_warm_workspace(T, N, C) bytes,
