@@ -96,6 +96,17 @@ void check_layer(const Tensor& I, const Tensor& u0) {
                     "u0 must be a float32 [N] tensor on I's device");
 }
 
+// A saved tensor as the kernels read it.  A saved-tensor hook may hand back another one than it was
+// given (off the GPU, in half precision, with other strides), so what the forward's checks showed is
+// checked again before its address is used.
+Tensor unpacked(const Tensor& t, torch::IntArrayRef sizes, const Tensor& like) {
+  TORCH_CHECK_VALUE(t.defined() && t.is_cuda() && t.device() == like.device() &&
+                        t.scalar_type() == torch::kFloat32 && t.sizes() == sizes,
+                    "a saved tensor was unpacked to something else than the float32 ", sizes,
+                    " tensor on ", like.device(), " that was saved");
+  return t.contiguous();
+}
+
 // The scaled column sums of the partials (undefined: none) and dL/du0 = beta * Lam[0], in one launch.
 struct Small {
   Tensor sums, du0;
@@ -162,34 +173,36 @@ struct LIFLayer : public torch::autograd::Function<LIFLayer> {
     const auto saved = ctx->get_saved_variables();
     const auto c = ctx->saved_data["c"].toDoubleVector();
     const auto n = ctx->saved_data["n"].toIntVector();
-    const Tensor& I = saved[0];
-    const c10::DeviceGuard guard(I.device());
-    const Tensor gS = grads[0].contiguous();
-    const int64_t T = I.size(0), N = I.size(1);
+    const c10::DeviceGuard guard(grads[0].device());
+    const Tensor gS = grads[0].contiguous();  // of the spikes' shape and device (the engine's check)
+    const int64_t T = gS.size(0), N = gS.size(1);
+    const Tensor I = unpacked(saved[0], gS.sizes(), gS);
     const float beta = (float)c[0], theta = (float)c[1], u_r = (float)c[2], alpha = (float)c[3];
     auto Lam = torch::empty_like(I);
     const bool sums = n[1] || n[2] || n[3];
     Tensor parts;
     if (saved.size() == 4) {
+      const Tensor u0 = unpacked(saved[1], {N}, gS), U = unpacked(saved[2], gS.sizes(), gS),
+                   S = unpacked(saved[3], gS.sizes(), gS);
       const size_t nb = g.lsh_lif_scan_lookback_any_bwd_workspace(T, N);
       const Tensor ws = workspace(nb, I);
       if (sums) {
         parts = partials(g.lsh_lif_param_partials(T, N, 4, 16), 3, I);
-        check(g.lsh_lif_param_bwd(fp(I), fp(saved[1]), fp(saved[2]), fp(saved[3]), fp(gS), fp(Lam),
-                                  dp(parts), T, N, beta, theta, u_r, alpha, 4, 16, raw(ws), nb,
-                                  stream_of(I)),
+        check(g.lsh_lif_param_bwd(fp(I), fp(u0), fp(U), fp(S), fp(gS), fp(Lam), dp(parts), T, N, beta,
+                                  theta, u_r, alpha, 4, 16, raw(ws), nb, stream_of(I)),
               "lsh_lif_param_bwd");
       } else {
-        check(g.lsh_lif_scan_lookback_any_bwd(fp(I), fp(saved[1]), fp(saved[2]), fp(saved[3]), fp(gS),
-                                              nullptr, fp(Lam), T, N, beta, theta, u_r, alpha, 1, 16,
-                                              raw(ws), nb, stream_of(I)),
+        check(g.lsh_lif_scan_lookback_any_bwd(fp(I), fp(u0), fp(U), fp(S), fp(gS), nullptr, fp(Lam), T,
+                                              N, beta, theta, u_r, alpha, 1, 16, raw(ws), nb,
+                                              stream_of(I)),
               "lsh_lif_scan_lookback_any_bwd");
       }
     } else {
+      const Tensor ST = unpacked(saved[1], {(T + 31) / 32, N}, gS);
       const size_t nb = g.lsh_lif_layer_bwd_workspace(T, N);
       const Tensor ws = workspace(nb, I);
       if (sums) parts = partials(g.lsh_lif_layer_partials(T, N), 3, I);
-      check(g.lsh_lif_layer_bwd(fp(I), fp(saved[1]), fp(gS), fp(Lam), dp(parts), T, N, beta, theta, u_r,
+      check(g.lsh_lif_layer_bwd(fp(I), fp(ST), fp(gS), fp(Lam), dp(parts), T, N, beta, theta, u_r,
                                 alpha, raw(ws), nb, stream_of(I)),
             "lsh_lif_layer_bwd");
     }
@@ -254,10 +267,11 @@ struct AffLayer : public torch::autograd::Function<AffLayer> {
     const auto saved = ctx->get_saved_variables();
     const auto c = ctx->saved_data["c"].toDoubleVector();
     const auto n = ctx->saved_data["n"].toIntVector();
-    const Tensor &I = saved[0], &u0 = saved[1], &U = saved[2];
-    const c10::DeviceGuard guard(I.device());
-    const Tensor gS = grads[0].contiguous();
-    const int64_t T = I.size(0), N = I.size(1);
+    const c10::DeviceGuard guard(grads[0].device());
+    const Tensor gS = grads[0].contiguous();  // of the spikes' shape and device (the engine's check)
+    const int64_t T = gS.size(0), N = gS.size(1);
+    const Tensor I = unpacked(saved[0], gS.sizes(), gS), u0 = unpacked(saved[1], {N}, gS),
+                 U = unpacked(saved[2], gS.sizes(), gS);
     const double beta = c[0], theta = c[1], gamma = c[2], alpha = c[4];
     const int code = (int)n[4], Cb = (int)n[5];
     auto Lam = torch::empty_like(I);
@@ -272,10 +286,11 @@ struct AffLayer : public torch::autograd::Function<AffLayer> {
       const Small s = finish(parts, 1.0, 0.0, 0.0, Lam, beta, n[0] != 0);
       return grads_of(s, Lam, {n[1], 0, 0}, 12);
     }
+    const Tensor S = unpacked(saved[3], gS.sizes(), gS);
     const size_t nb = code >= 3 ? g.lsh_lif_scan_lookback_any_bwd_workspace(T, N) : 0;
     const Tensor ws = workspace(nb, I);
     parts = partials(g.lsh_lif_param_partials(T, N, code, Cb), 3, I);
-    check(g.lsh_aff_bwd(fp(I), fp(u0), fp(U), fp(saved[3]), fp(gS), fp(Lam), dp(parts), T, N, (float)beta,
+    check(g.lsh_aff_bwd(fp(I), fp(u0), fp(U), fp(S), fp(gS), fp(Lam), dp(parts), T, N, (float)beta,
                         (float)theta, (float)gamma, (float)alpha, code, Cb, raw(ws), nb, stream_of(I)),
           "lsh_aff_bwd");
     const bool sums = n[1] || n[2] || n[3];

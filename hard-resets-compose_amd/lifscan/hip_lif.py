@@ -961,6 +961,10 @@ def _layer_backward(I, STATES, GS, beta, theta, u_r, alpha=4.0, want_sums=False)
     I = _input(I)
     T, N = I.shape
     GS = _same(GS, I, "GS")
+    if (STATES.shape != ((T + 31) // 32, N) or STATES.device != I.device
+            or STATES.dtype != torch.float32):
+        raise ValueError(f"STATES must be float32 [{(T + 31) // 32}, {N}] on {I.device}")
+    STATES = STATES.contiguous()
     Lam = torch.empty_like(I)
     if T == 0 or N == 0:
         return Lam, torch.zeros(3, device=I.device, dtype=torch.float64) if want_sums else None
