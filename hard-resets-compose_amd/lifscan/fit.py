@@ -110,6 +110,7 @@ def lif_param(I, u0, beta, theta, u_r, alpha=4.0, mode="auto", K=16):
     T, N = I.shape
     choose = mode == "auto"
     if choose:
+        L._check_auto_args(T, N, K, 0)
         fwd, bwd = L.auto_modes(N, T)
         fwd, bwd = L._auto_fwd(fwd, N, T), L._auto_bwd(bwd, N, T)
         u0v = L._cpp_u0(I, u0, alpha) if L._layer_ok(N) else None

@@ -313,7 +313,7 @@ def _converged_fast(I, beta, theta, u_r, u0, C, K, repair, stats):
         plan = warm_plan(T, N, beta)
         if plan is not None:
             return _scan_warm_run(I, beta, theta, u_r, u0, *plan)
-        plan = warm_any_plan(T, N, beta)
+        plan = warm_any_plan(T, N, beta) if int(K) >= 1 else None
         if plan is not None:
             return _warm_any(I, beta, theta, u_r, u0, *plan)
     if _fused_fwd_ok(T, C, K, repair, stats):
@@ -931,7 +931,7 @@ def _converged_layer(T, N, beta, K, repair):
     """True when a converged scan layer (lif_tuned) takes the layer pair: scan_forward_auto would
     give the serial recurrence's bits and neither warm-started nor long chunks are faster."""
     C = _chunk_or_none(T, 16)
-    return (C is not None and T > 0 and _layer_ok(N) and int(K) <= 16 and int(repair) >= T // C
+    return (C is not None and T > 0 and _layer_ok(N) and 1 <= int(K) <= 16 and int(repair) >= T // C
             and warm_plan(T, N, beta) is None and warm_any_plan(T, N, beta) is None
             and not long_sequence_C(T, N))
 
@@ -1169,6 +1169,16 @@ def _auto_fwd(fwd, N, T):
     """auto_modes' forward mode, or "auto" where warm-started chunks may apply: the layer's forward
     then decides from beta (_auto_forward)."""
     return "auto" if 1 <= N <= WARM_FEW_MAX_N and T >= 4 * 256 else fwd
+
+
+def _check_auto_args(T, N, K, repair):
+    """The map scan's refusals of a capacity or a repair budget, where auto_modes gives lif_auto and
+    lif_param that scan, also when the warm-started chunks run in its place."""
+    if T >= AUTO_FWD_MIN_T and auto_modes(N, T)[0] == "scan" and int(repair) < T // _pick_C(T, D=16):
+        if not 1 <= int(K) <= 64:
+            raise ValueError("map capacity K must be in [1, 64]")
+        if int(repair) < 0:
+            raise ValueError("repair must be >= 0")
 
 
 def _auto_states(T, N, beta):
@@ -1415,6 +1425,7 @@ class LIFAuto(torch.autograd.Function):
 
 def lif_auto(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, K=16, repair=0):
     T, N = I.shape
+    _check_auto_args(T, N, K, repair)
     if _layer_ok(N) and T > 0:
         u0v = _cpp_u0(I, u0, theta, u_r, alpha)
         if u0v is not None:  # the same kernels and bits as LIFAuto's layer pair, from C++

@@ -208,3 +208,23 @@ def test_layers_take_the_pair(dev, call, T, N):
     assert abs(grads[2].item() - (want * up).sum()) <= 1e-4 * abs((want * up).sum()) + 1e-4
     with torch.no_grad():
         assert np.array_equal(host(f(0.95)), So)
+
+
+def test_scan_arguments_are_still_refused(dev):
+    """A map capacity or repair budget that the scans refuse is refused whichever forward runs."""
+    from lifscan import hip_lif as L
+    from lifscan.fit import lif_param
+    I, u0 = torch.zeros(16384, 8, device=dev), torch.zeros(8, device=dev)
+    assert L.warm_any_plan(16384, 8, 0.9) is not None
+    for kw in ({"K": 0}, {"K": 65}, {"repair": -1}):
+        with pytest.raises(ValueError):
+            L.lif_auto(I, u0, 0.9, **kw)
+    for K in (0, 65):
+        with pytest.raises(ValueError):
+            lif_param(I, u0, 0.9, 1.0, 0.0, K=K)
+    with pytest.raises(ValueError):  # the layer pair
+        L.lif_tuned(I[:96], u0, 0.9, K=0, repair=10 ** 6)
+    with pytest.raises(ValueError):  # warm-started chunks of a T without a power-of-two chunk
+        L.scan_forward_v3(I[:2064], 0.9, 1.0, 0.0, u0, C=16, K=0, repair=10 ** 6)
+    assert L.lif_auto(I, u0, 0.9, K=64).shape == I.shape  # what was taken still is
+    assert L.lif_tuned(I[:96], u0, 0.9, K=32, repair=10 ** 6).shape == (96, 8)
