@@ -865,7 +865,9 @@ def _wait_header(device):
     if h is None:
         h = torch.zeros(max(int(_n.lib().lsh_lif_scan_exact_workspace()), 256), dtype=torch.uint8,
                         device=device)
-        _WAIT_HEADERS[device] = h
+        # in a capture the clearing only runs when the graph does: a header of that graph's own
+        if not torch.cuda.is_current_stream_capturing():
+            _WAIT_HEADERS[device] = h
     return h
 
 
