@@ -17,6 +17,7 @@
 #include <array>
 #include <cstdint>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -105,6 +106,27 @@ Tensor unpacked(const Tensor& t, torch::IntArrayRef sizes, const Tensor& like) {
                     "a saved tensor was unpacked to something else than the float32 ", sizes,
                     " tensor on ", like.device(), " that was saved");
   return t.contiguous();
+}
+
+// The workspace of the process's most recent look-back adjoint, whose header counts the bounded waits
+// that gave up (hip_lif.last_lookback_timeouts).  Set from the engine's threads; left to the process
+// at its end, when the device may be gone.
+std::mutex& lookback_lock() {
+  static std::mutex m;
+  return m;
+}
+Param& lookback_ws() {
+  static Param* ws = new Param;
+  return *ws;
+}
+void set_last_lookback(const Tensor& ws) {
+  Param old = ws;  // freed outside the lock
+  const std::lock_guard<std::mutex> lock(lookback_lock());
+  std::swap(lookback_ws(), old);
+}
+Param last_lookback() {
+  const std::lock_guard<std::mutex> lock(lookback_lock());
+  return lookback_ws();
 }
 
 // The scaled column sums of the partials (undefined: none) and dL/du0 = beta * Lam[0], in one launch.
@@ -197,6 +219,7 @@ struct LIFLayer : public torch::autograd::Function<LIFLayer> {
                                               stream_of(I)),
               "lsh_lif_scan_lookback_any_bwd");
       }
+      set_last_lookback(ws);
     } else {
       const Tensor ST = unpacked(saved[1], {(T + 31) / 32, N}, gS);
       const size_t nb = g.lsh_lif_layer_bwd_workspace(T, N);
@@ -205,6 +228,7 @@ struct LIFLayer : public torch::autograd::Function<LIFLayer> {
       check(g.lsh_lif_layer_bwd(fp(I), fp(ST), fp(gS), fp(Lam), dp(parts), T, N, beta, theta, u_r,
                                 alpha, raw(ws), nb, stream_of(I)),
             "lsh_lif_layer_bwd");
+      if (nb) set_last_lookback(ws);
     }
     const Small s = finish(parts, 1.0, -1.0, beta, Lam, beta, n[0] != 0);
     return grads_of(s, Lam, {n[1], n[2], n[3]}, 12);
@@ -293,6 +317,7 @@ struct AffLayer : public torch::autograd::Function<AffLayer> {
     check(g.lsh_aff_bwd(fp(I), fp(u0), fp(U), fp(S), fp(gS), fp(Lam), dp(parts), T, N, (float)beta,
                         (float)theta, (float)gamma, (float)alpha, code, Cb, raw(ws), nb, stream_of(I)),
           "lsh_aff_bwd");
+    if (nb) set_last_lookback(ws);
     const bool sums = n[1] || n[2] || n[3];
     const Small s = finish(sums ? parts : Tensor(), 1.0, beta, beta, Lam, beta, n[0] != 0);
     return grads_of(s, Lam, {n[1], n[2], n[3]}, 12);
@@ -325,5 +350,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("lif_layer", &lif_layer, "hard-reset LIF layer: S");
   m.def("lif_spikes", &lif_spikes, "hard-reset LIF spikes outside autograd");
   m.def("aff_layer", &aff_layer, "affine- or soft-reset LIF layer: S");
+  m.def("set_last_lookback", &set_last_lookback, "workspace of the most recent look-back adjoint");
+  m.def("last_lookback", &last_lookback, "that workspace, or None");
   m.def("read_scalars", &read_scalars, "values of one-element tensors in one copy");
 }

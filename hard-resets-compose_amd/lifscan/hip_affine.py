@@ -168,6 +168,8 @@ def _aff_backward(I, u0, U, S, GS, beta, theta, gamma, alpha, mode="auto", C=Non
             _n.ptr(I), _n.ptr(u0), _n.ptr(U), _n.ptr(S), _n.ptr(GS), _n.ptr(Lam), _n.ptr(parts), T, N,
             _f32(beta), _f32(theta), _gamma(_f32(gamma)), _f32(alpha), code, C, _n.ptr(ws), nbytes,
             _n.stream_of(I)), "lsh_aff_bwd")
+    if code >= 3:
+        L._note_lookback(ws)
     return Lam, parts.sum(0)
 
 

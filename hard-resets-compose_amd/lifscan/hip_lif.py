@@ -496,6 +496,7 @@ def warm_any_plan(T, N, beta):
 
 def _warm_any(I, beta, theta, u_r, u0, C, W):
     """The warm-started forward for every T (its last chunk may be short) -> (U, S)."""
+    global _LAST_RUN
     I = _input(I)
     T, N = I.shape
     u0 = _vec(u0, N, I)
@@ -508,6 +509,7 @@ def _warm_any(I, beta, theta, u_r, u0, C, W):
         _n.check(L.lsh_lif_scan_warm_any_fwd(
             _n.ptr(I), _n.ptr(u0), _n.ptr(U), _n.ptr(S), T, N, _f32(beta), _f32(theta), _f32(u_r),
             C, W, _n.ptr(ws), nbytes, _n.stream_of(I)), "lsh_lif_scan_warm_any_fwd")
+    _LAST_RUN = _WarmRun(C, W)
     return U, S
 
 
@@ -981,6 +983,8 @@ def _layer_backward(I, STATES, GS, beta, theta, u_r, alpha=4.0, want_sums=False)
             _n.ptr(I), _n.ptr(STATES), _n.ptr(GS), _n.ptr(Lam), _n.ptr(parts), T, N, _f32(beta),
             _f32(theta), _f32(u_r), _f32(alpha), _n.ptr(ws), nbytes, _n.stream_of(I)),
             "lsh_lif_layer_bwd")
+    if ws is not None:
+        _note_lookback(ws)
     return Lam, (parts.sum(0) if want_sums else None)
 
 
@@ -1022,7 +1026,7 @@ def chunked_bwd_C(T, N, C=64):
 
 
 LOOKBACK_SEG = 256  # steps per workgroup segment of the look-back adjoint
-_LAST_LOOKBACK = None
+_LAST_LOOKBACK = None  # its most recent workspace, where the C++ module does not keep it
 
 
 def scan_backward_lookback(I, u0, U, S, GS, GU, beta, theta, u_r, alpha=4.0, detach=True, C=16):
@@ -1036,7 +1040,6 @@ def scan_backward_lookback(I, u0, U, S, GS, GU, beta, theta, u_r, alpha=4.0, det
 
 def _lookback(I, u0, U, S, GS, GU, beta, theta, u_r, alpha, detach, C=16):
     """The look-back adjoint for every T (its last segment may be short) -> Lam."""
-    global _LAST_LOOKBACK
     I = _input(I)
     T, N = I.shape
     u0 = _vec(u0, N, I)
@@ -1053,15 +1056,27 @@ def _lookback(I, u0, U, S, GS, GU, beta, theta, u_r, alpha, detach, C=16):
             _n.ptr(I), _n.ptr(u0), _n.ptr(U), _n.ptr(S), _n.ptr(GS), _n.ptr(GU), _n.ptr(Lam), T, N,
             _f32(beta), _f32(theta), _f32(u_r), _f32(alpha), int(bool(detach)), int(C), _n.ptr(ws),
             nbytes, _n.stream_of(I)), "lsh_lif_scan_lookback_any_bwd")
-    _LAST_LOOKBACK = ws
+    _note_lookback(ws)
     return Lam
 
 
+def _note_lookback(ws):
+    """Keep a look-back adjoint's workspace for last_lookback_timeouts, and with CHECK_WAITS raise
+    when one of its waits gave up."""
+    global _LAST_LOOKBACK
+    if _n.ops() is not None:
+        _n.ops().set_last_lookback(ws)
+    else:
+        _LAST_LOOKBACK = ws
+    if CHECK_WAITS and last_lookback_timeouts() != 0:
+        raise RuntimeError("look-back adjoint: a wait gave up; the gradients are not valid")
+
+
 def last_lookback_timeouts():
-    """Bounded waits of the most recent look-back adjoint that gave up (must be 0)."""
-    if _LAST_LOOKBACK is None:
-        return None
-    return int(_n.read_stats(_LAST_LOOKBACK, 1).spin_timeouts)
+    """Bounded waits of the process's most recent look-back adjoint that gave up (must be 0), a
+    layer's among them; None when none ran.  Synchronizes."""
+    ws = _LAST_LOOKBACK if _n.ops() is None else _n.ops().last_lookback()
+    return None if ws is None else int(_n.read_stats(ws, 1).spin_timeouts)
 
 
 def scan_backward_tiled(I, u0, U, S, GS, GU, beta, theta, u_r, alpha=4.0, detach=True, C=64,
