@@ -1282,9 +1282,9 @@ class LIFTuned(torch.autograd.Function):
     None for beta).  The backward reads no GU array (it is identically zero here)."""
 
     @staticmethod
-    def forward(ctx, I, u0, beta, theta, u_r, alpha, mode, K, repair):
+    def forward(ctx, I, u0, beta, theta, u_r, alpha, mode, K, repair, b=None):
         I = I.contiguous()
-        b = _f32(beta)
+        b = _f32(beta) if b is None else b
         ctx.cfg = (b, theta, u_r, alpha, mode)
         T, N = I.shape
         if mode != "serial" and _recompute_ok(T, N, K, repair):
@@ -1317,7 +1317,7 @@ class LIFTuned(torch.autograd.Function):
             Lam, sums = bwd(I, ST, gS, b, theta, u_r, alpha, need_b)
             db = sums[0].float().reshape(()) if need_b else None
             du0 = b * Lam[0] if ctx.needs_input_grad[1] else None
-            return (Lam, du0, db, None, None, None, None, None, None)
+            return (Lam, du0, db, None, None, None, None, None, None, None)
         I, u0, U, S = ctx.saved_tensors
         if mode == "serial":
             Lam = serial_backward_auto(I, u0, U, S, gS, None, b, theta, u_r, alpha)
@@ -1325,7 +1325,7 @@ class LIFTuned(torch.autograd.Function):
             Lam = scan_backward_auto(I, u0, U, S, gS, None, b, theta, u_r, alpha)
         du0 = b * Lam[0] if ctx.needs_input_grad[1] else None
         return (Lam, du0, _beta_grad(Lam, U, u0, ctx.needs_input_grad[2]),
-                None, None, None, None, None, None)
+                None, None, None, None, None, None, None)
 
 
 _FORWARD_AD = torch.autograd.forward_ad
@@ -1372,33 +1372,38 @@ def _grad_param(p):
     return p if type(p) is not float and torch.is_tensor(p) and p.requires_grad else None
 
 
-def _rc_path(I, u0, beta, mode, K, repair, *fixed):
-    """u0 as the [N] vector when lif_tuned takes the C++ layer (_cpp_u0) over the recomputing pair
-    of a converged forward, else None."""
-    if mode == "serial":
-        return None
-    u0v = _cpp_u0(I, u0, *fixed)
-    if u0v is None or not _layer_ok(I.shape[1]):
-        return None
-    T, N = I.shape
-    return u0v if _recompute_ok(T, N, K, repair) or _converged_layer(T, N, beta, K, repair) else None
+def _pair_runs(T, N, b, K, repair):
+    """True when a scan-mode lif_tuned call of these sizes takes a recomputing pair."""
+    return _recompute_ok(T, N, K, repair) or _converged_layer(T, N, b, K, repair)
+
+
+def _rc_path(I, u0, beta, mode, K, repair):
+    """u0 as the [N] vector when lif_tuned takes a recomputing pair from C++, else None."""
+    u0v = None if mode == "serial" else _cpp_u0(I, u0)
+    return u0v if u0v is not None and _layer_ok(I.shape[1]) and _pair_runs(*I.shape, _f32(beta), K,
+                                                                           repair) else None
 
 
 def lif_tuned(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, mode="scan", K=16, repair=0):
-    u0v = _rc_path(I, u0, beta, mode, K, repair, theta, u_r, alpha)
-    if u0v is not None:  # the same kernels and bits as LIFTuned's recomputing pairs, from C++
-        return _n.ops().lif_layer(I, u0v, _grad_param(beta), None, None, *_f32s(beta, theta, u_r),
-                                  _f32(alpha), _wait_header(I.device), 0, 0)
-    return LIFTuned.apply(I, u0, beta, theta, u_r, alpha, mode, K, repair)
+    u0v = None if mode == "serial" else _cpp_u0(I, u0, theta, u_r, alpha)
+    if u0v is None or not _layer_ok(I.shape[1]):
+        return LIFTuned.apply(I, u0, beta, theta, u_r, alpha, mode, K, repair)
+    T, N = I.shape
+    b, th, ur = _f32s(beta, theta, u_r)  # read once, for the plans and the call
+    if _pair_runs(T, N, b, K, repair):
+        # the same kernels and bits as LIFTuned's recomputing pairs, from C++
+        return _n.ops().lif_layer(I, u0v, _grad_param(beta), None, None, b, th, ur, _f32(alpha),
+                                  _wait_header(I.device), 0, 0)
+    return LIFTuned.apply(I, u0, beta, th, ur, alpha, mode, K, repair, b)
 
 
 class LIFAuto(torch.autograd.Function):
     """Serial or scan chosen per pass (triton_lif.py:1003-1026)."""
 
     @staticmethod
-    def forward(ctx, I, u0, beta, theta, u_r, alpha, K, repair, fwd_mode, bwd_mode):
+    def forward(ctx, I, u0, beta, theta, u_r, alpha, K, repair, fwd_mode, bwd_mode, b=None):
         I = I.contiguous()
-        b = _f32(beta)
+        b = _f32(beta) if b is None else b
         ctx.cfg = (b, theta, u_r, alpha, bwd_mode)
         T, N = I.shape
         # the exact forward's bits are the serial one's: U, kept only for the backward, is left out
@@ -1427,7 +1432,7 @@ class LIFAuto(torch.autograd.Function):
             Lam, sums = _layer_backward(I, ST, gS, b, theta, u_r, alpha, need_b)
             db = sums[0].float().reshape(()) if need_b else None
             du0 = b * Lam[0] if ctx.needs_input_grad[1] else None
-            return (Lam, du0, db, None, None, None, None, None, None, None)
+            return (Lam, du0, db, None, None, None, None, None, None, None, None)
         I, u0, U, S = ctx.saved_tensors
         if bwd_mode == "scan":
             Lam = scan_backward_auto(I, u0, U, S, gS, None, b, theta, u_r, alpha)
@@ -1437,12 +1442,13 @@ class LIFAuto(torch.autograd.Function):
             Lam = serial_backward_auto(I, u0, U, S, gS, None, b, theta, u_r, alpha)
         du0 = b * Lam[0] if ctx.needs_input_grad[1] else None
         return (Lam, du0, _beta_grad(Lam, U, u0, ctx.needs_input_grad[2]),
-                None, None, None, None, None, None, None)
+                None, None, None, None, None, None, None, None)
 
 
 def lif_auto(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, K=16, repair=0):
     T, N = I.shape
     _check_auto_args(T, N, K, repair)
+    b = None
     if _layer_ok(N) and T > 0:
         u0v = _cpp_u0(I, u0, theta, u_r, alpha)
         if u0v is not None:  # the same kernels and bits as LIFAuto's layer pair, from C++
@@ -1454,12 +1460,12 @@ def lif_auto(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, K=16, repair=0):
                     return _n.ops().lif_layer(I, u0v, _grad_param(beta), None, None, b, th, ur,
                                               _f32(alpha), hdr, 0, 0)
                 return _n.ops().lif_spikes(I, u0v, b, th, ur, hdr)
-            beta, theta, u_r = (b if _grad_param(beta) is None else beta), th, ur  # read once
+            theta, u_r = th, ur  # read once
     fwd, bwd = auto_modes(N, T)
     fwd, bwd = _auto_fwd(fwd, N, T), _auto_bwd(bwd, N, T)
     if not _layer_ok(N) and fwd == bwd:  # one mode for both passes: lif_tuned's path
         return lif_tuned(I, u0, beta, theta, u_r, alpha, mode=fwd, K=K, repair=repair)
-    return LIFAuto.apply(I, u0, beta, theta, u_r, alpha, K, repair, fwd, bwd)
+    return LIFAuto.apply(I, u0, beta, theta, u_r, alpha, K, repair, fwd, bwd, b)
 
 
 def surrogate_grad(x, alpha):

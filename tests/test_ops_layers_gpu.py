@@ -126,3 +126,23 @@ def test_layer_grads_kernel(dev, P, cols, N):
     tol = 2.0 ** -24 * (s * p.sum(0)).abs() + 2.0 ** -52 * P * p.abs().sum(0)
     assert bool(((sums.double() - s * p.sum(0)).abs() <= tol).all())
     assert torch.equal(du0, 0.95 * lam)
+
+
+@pytest.mark.parametrize("T", [96, 4096, 4128])  # the pair, and plans with and without a power-of-two chunk
+@pytest.mark.parametrize("call", ["tuned", "tuned_scan", "auto"])
+def test_device_beta_is_read_once(dev, monkeypatch, T, call):
+    """A beta on the device is read by one synchronizing copy a call, also where plans depend on it."""
+    from lifscan import hip_lif as L
+    I, gS, u0 = _data(T, 70, dev)
+    I.requires_grad_(True)
+    beta = torch.tensor(0.9, device=dev, requires_grad=True)
+    fn = {"tuned": lambda: L.lif_tuned(I, u0, beta, repair=10 ** 6), "tuned_scan": lambda: L.lif_tuned(I, u0, beta),
+          "auto": lambda: L.lif_auto(I, u0, beta)}[call]
+    want = fn().detach()
+    reads = []
+    item = torch.Tensor.item
+    monkeypatch.setattr(torch.Tensor, "item", lambda self: (reads.append(1), item(self))[1])
+    S = fn()
+    assert len(reads) == 1 and torch.equal(S, want)
+    dI, db = torch.autograd.grad(S, [I, beta], gS)
+    assert len(reads) == 1 and dI.shape == I.shape and db.shape == ()
