@@ -24,7 +24,7 @@
 //                   differs from its predecessor's exit.
 //
 // The result is the serial recurrence bit for bit, the result of scan_forward_v3
-// (triton_lif.py:782-817) with repair >= T/C, in at most about the warm pass and one serial sweep:
+// (triton_lif.py:782-817) with repair >= T/C, in at most about the warm pass and two serial sweeps:
 // under a nearly constant current trajectories of different phase never spike together, and every
 // prediction is wrong.  Traffic: I read over W + C rows per chunk (the warm-up rows are the
 // previous chunk's, read at the same time by that chunk's wave, so mostly from cache), U and S

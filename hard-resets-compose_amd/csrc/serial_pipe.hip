@@ -315,12 +315,12 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
 // noisy inputs leave (each meets its stored trajectory soon); with a nearly constant current no
 // trajectory ever meets another one of a different phase, every round makes one more chunk exact,
 // and rounds alone took M of them, some M^2/2 chunk replays.
-// One workgroup per 64 neurons.  A round of nd replays takes 1 + nd/256 units of the budget: a few
+// One workgroup per 64 neurons.  A round of nd replays takes 1 + nd/128 units of the budget: a few
 // lanes walk a row in some 45 ns (the sweep in 17), all 1024 in 250, for their rows lie apart.
 // Measured, N 64, T 50000, beta 0.93 (C 256; the serial sweep alone 0.86 ms), rounds alone -> this:
-// constant current 104.8 -> 0.95 ms, current steps 12.5 -> 0.93 ms, noise 60 -> 39 us (the first
-// comparison by 16 waves instead of 4); N 4096, T 16001, beta 0.95 (C 2000; sweep 0.30 ms) constant
-// current 1.41 -> 0.62 ms.
+// constant current 104.8 -> 0.94 ms, current steps 12.5 -> 0.93 ms, noise 60 -> 39 us (the first
+// comparison by 16 waves instead of 4); N 1000, T 60001, beta 0.95 (C 1888; sweep 1.20 ms) constant
+// current 5.25 -> 2.24 ms; N 4096, T 16001 (C 2000; 0.30 ms) 1.41 -> 0.75 ms.
 constexpr int kWarmScanAhead = 8;  // chunks a wave compares at once
 template <bool NT>
 __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_warm_finish(
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_warm_finish(
   __syncthreads();
   int rounds = 0, nd = s_nd;
   while (nd > 0) {
-    const int units = 1 + nd / 256;
+    const int units = 1 + nd / 128;
     if (units > budget) break;
     budget -= units;
     ++rounds;
@@ -411,8 +411,9 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_warm_finish(
                                        S + row0 * N, nb0, N, T - (int64_t)row0, step);
 }
 
-// The budget of the rounds: M/16 units, a fifth of the serial sweep's time; below 16 chunks the sweep
-// from a wrong start on takes no longer than a round.
+// The budget of the rounds: M/5 units, half the serial sweep's time.  Noisy inputs need up to 6 rounds
+// with 32 chunks and 16 with 128 (beta 0.98 to 0.995); with M/16 units some were swept although two or
+// three rounds more would have done (N 1024, T 32768, beta 0.995 529 -> 754 us).
 void lif_warm_finish_launch(const float* I, float* U, float* S, float* starts, float* ends, int* list0,
                             int* list1, WsHeader* hdr, int64_t T, int64_t N, int M, int C, float beta,
                             float theta, float u_r, hipStream_t st) {
@@ -420,7 +421,7 @@ void lif_warm_finish_launch(const float* I, float* U, float* S, float* starts, f
   with_store_policy(N, [&](auto nt) {
     hipLaunchKernelGGL((k_lif_warm_finish<decltype(nt)::value>), dim3((unsigned)NB),
                        dim3(WAVE * (PIPE_P + 1)), 0, st, I, U, S, starts, ends, list0, list1, hdr, T, N, M,
-                       C, M / 16, LifStep(beta, theta, u_r));
+                       C, M / 5, LifStep(beta, theta, u_r));
   });
 }
 
