@@ -158,7 +158,7 @@ def bench_auto_grid(torch, dev, reps=15):
     a training loop runs them; at the smallest cells a call is ~10 us of GPU work and one call
     between two synchronizations measures the host's latency instead), groups of the three modes
     interleaved so that clock drift favours none, median of 7 groups.  Per cell: the three times,
-    auto's modes, whether the spikes of all three are equal and auto's gradient against serial's;
+    auto_modes' choice and auto's route, whether the spikes of all three are equal and auto's gradient against serial's;
     auto_vs_best = auto's time over the faster of the two modes."""
     from lifscan import hip_lif as L
     rows = []
@@ -207,6 +207,8 @@ def bench_auto_grid(torch, dev, reps=15):
             gs = res["serial"][2]
             best = min(res["serial"][0], res["scan"][0])
             rows.append({"N": N, "T": T, "modes": list(L.auto_modes(N, T)),
+                         "auto_route": {None: "map scan", (0, 0): "layer pair"}.get(
+                             L._auto_route(T, N, 0.9), "warm chunks"),
                          **{k: round(res[k][0], 4) for k in fns},
                          "spikes_equal": all(torch.equal(res[k][1], res["serial"][1]) for k in ("scan", "auto")),
                          "grad_rel_auto": float((res["auto"][2] - gs).norm() / gs.norm()),

@@ -70,19 +70,20 @@ class LIFParamFn(torch.autograd.Function):
     def forward(ctx, I, u0, beta, theta, u_r, alpha, fwd_mode, bwd_mode, K, choose=False):
         b, th, ur = choose if isinstance(choose, tuple) else _f32s(beta, theta, u_r)
         I = I.contiguous()
-        ctx.cfg = (b, th, ur, float(alpha), bwd_mode)
         T, N = I.shape
+        route = L._auto_route(T, N, b) if choose and L._layer_ok(N) and T > 0 else None
+        ctx.cfg = (b, th, ur, float(alpha), "lookback" if route else bwd_mode)
         # lif_param's own choice: the exact forward's bits are the serial one's, so the states before
         # every 32 rows are kept instead of U
-        if choose and L._layer_ok(N) and T > 0 and not L._auto_states(T, N, b):
+        if route == (0, 0):
             S, ST = L._layer_forward(I, b, th, ur, u0)
             ctx.save_for_backward(I, u0, ST)
             ctx.recompute = True
             return S
-        if fwd_mode == "scan":
+        if choose:
+            U, S = L._auto_forward(I, b, th, ur, u0, K, 0, route, fwd_mode)
+        elif fwd_mode == "scan":
             U, S = L.scan_forward_auto(I, b, th, ur, u0, K=K)
-        elif fwd_mode == "auto":
-            U, S = L._auto_forward(I, b, th, ur, u0, K, 0)
         else:
             U, S = L.serial_forward_auto(I, b, th, ur, u0)
         ctx.save_for_backward(I, u0, U, S)
@@ -118,14 +119,10 @@ def lif_param(I, u0, beta, theta, u_r, alpha=4.0, mode="auto", K=16):
         u0v = L._cpp_u0(I, u0, alpha) if L._layer_ok(N) else None
         if u0v is not None:  # the same kernels as LIFParamFn's, from C++
             b, th, ur = choose = _f32s(beta, theta, u_r)
-            plan = L.warm_any_plan(T, N, b)
-            if not L._auto_states(T, N, b):
-                plan = (0, 0)
-            elif plan is None or _param_plan(T, N, bwd)[0] < 3:
-                plan = None
-            if plan is not None:
+            route = L._auto_route(T, N, b)
+            if route is not None:
                 return _n.ops().lif_layer(I, u0v, *map(L._grad_param, (beta, theta, u_r)), b, th, ur,
-                                          float(alpha), L._wait_header(I.device), *plan)
+                                          float(alpha), L._wait_header(I.device), *route)
     else:
         fwd = bwd = mode
     return LIFParamFn.apply(I, u0, beta, theta, u_r, alpha, fwd, bwd, K, choose)

@@ -23,9 +23,11 @@ from . import _native as _n
 
 BN_DEFAULT = 128
 
-# auto dispatch thresholds (serial vs scan per pass), measured on MI355X (beta = 0.95, N from
-# 256 to 65536, T from 1024 to 65536): the scan forward of lif_auto (scan_forward_auto, no
-# repair) beats the serial kernel only with <= 1024 neurons and T >= 16384 (e.g. N = 1024,
+# auto_modes' thresholds (serial vs scan per pass, the reference's choice).  lif_auto and lif_param
+# themselves run the layer pair or warm-started chunks (_auto_route); the forward mode decides only
+# where neither does, the adjoint's only behind such a forward.  Measured on MI355X (beta = 0.95, N
+# from 256 to 65536, T from 1024 to 65536): the map scan (scan_forward_auto, no repair) beats the
+# serial kernel only with <= 1024 neurons and T >= 16384 (e.g. N = 1024,
 # T = 65536: 1.03 vs 1.87 ms; N = 4096, T = 65536: 2.45 vs 2.06 ms).  The scan adjoint, one
 # layer's fwd + bwd through autograd (beta 0.9, x ~ N(0.15, 0.4^2)), serial fwd + serial bwd
 # against serial fwd + scan bwd: below 16384 neurons the serial adjoint wins up to T = 1024
@@ -469,29 +471,60 @@ def _scan_warm_run(I, beta, theta, u_r, u0, C, W):
 
 
 # Warm-started chunks where T has no power-of-two chunk, and for the layers that pick their own
-# forward (lif_auto, lif_param): chunks of T*nb/WARM_TARGET_WAVES steps, the last one short.  From
-# 4W steps up to 1024 neurons and 8W up to 4096 (there the repair of the missed chunks weighs
-# more), against the serial sweep's 18 ns a step.  Measured on MI355X, serial -> warm: beta 0.95
-# (W 512) N = 64, T = 60001 1076 -> 55 us; N = 1000, T = 2001 / 16001 41 -> 27 / 293 -> 70 us;
-# N = 4096, T = 4001 77 -> 49 us; beta 0.99 (W 2560) N = 64 / 1000, T = 16001 290 -> 95 / 293 ->
-# 174 us, but N = 4096, T = 16001 294 -> 420 and T = 60001 1214 -> 972 us.  From 8192 neurons the
-# sweep fills the chip: T = 2001 / 4001 42 / 79 us against 47 / 76.
+# forward: chunks of T*nb/WARM_TARGET_WAVES steps, the last one short.  Forward against the layer
+# pair's (the serial sweep, spikes alone, 17.6 ns a step from T = 1024): from 4W steps up to 1024
+# neurons (up to 512 where W > 1280: more predictions miss), else from 8W.  Measured
+# on MI355X, serial -> warm: beta 0.95 (W 512) N = 64, T = 2048 45 -> 35 us; N = 1024, T = 2048 / 16384
+# 46 -> 35 / 294 -> 61; N = 4096, T = 4096 81 -> 58; beta 0.98 (W 1280) N = 1024, T = 5001 / 8192 97 ->
+# 90 / 152 -> 158; beta 0.99 (W 2560) N = 256, T = 8192 / 12288 152 -> 202 / 222 -> 146; N = 1024, T =
+# 12288 / 24576 224 -> 340 / 438 -> 237; N = 4096, T = 16384 296 -> 306 us.  A decay so near 1 that the
+# longest warm-up is too short (W beyond 8192) has no plan: most predictions would miss.
 WARM_ANY_WIDE_N = 1024
+
+
+def _warm_up(beta):
+    """The warm-up steps that a decay needs, or None where that is more than 8192."""
+    b = abs(_f32(beta))
+    W = max(256, 256 * math.ceil(WARM_K / (1.0 - b) / 256.0)) if b < 1.0 else 8193
+    return W if W <= 8192 else None
 
 
 def warm_any_plan(T, N, beta):
     """(C, W) of the warm-started forward for any T, or None where the serial sweep is as fast."""
-    if N > WARM_FEW_MAX_N or N < 1 or T < 4 * 256:
+    W = _warm_up(beta) if 1 <= N <= WARM_FEW_MAX_N and T >= 4 * 256 else None
+    if W is None:
         return None
-    b = abs(_f32(beta))
-    if not b < 1.0:
-        return None
-    W = int(min(8192, max(256, 256 * math.ceil(WARM_K / (1.0 - b) / 256.0))))
-    if T < (4 if N <= WARM_ANY_WIDE_N else 8) * W:
+    if T < (4 if N <= (WARM_ANY_WIDE_N if W <= 1280 else WARM_ANY_WIDE_N // 2) else 8) * W:
         return None
     target = WARM_TARGET_WAVES_LARGE if T * N >= WARM_LARGE_WORK else WARM_TARGET_WAVES
     C = T * ((N + 63) // 64) // target
     return max(WARM_MIN_C, (C + 15) // 16 * 16), W
+
+
+# Whole layers, forward and adjoint: warm-started chunks store U and S, which the look-back adjoint
+# reads, where the layer pair stores the spikes and a state every 32 rows and replays them; and their
+# host calls are some 12 us longer.  So a layer with gradients takes them from 3072 steps on, and from
+# 4W steps up to 512 neurons, 8W up to 2048, 24W up to 4096; spikes alone from 2048.  Measured on
+# MI355X, kernels of the pair -> warm, us: beta 0.9 (W 256) N = 64, T = 2048 / 4096 57 -> 43 / 94 -> 45
+# (the calls: 56 -> 66, 90 -> 66); N = 1024, T = 3072 81 -> 52; N = 2048, T = 3072 91 -> 81; N = 4096, T =
+# 6000 / 8192 185 -> 185 / 240 -> 227; beta 0.95 (W 512) N = 1024, T = 4096 102 -> 65; N = 2048, T = 4096
+# 113 -> 105; N = 4096, T = 8192 / 12288 241 -> 238 / 343 -> 323; beta 0.98 (W 1280) N = 512, T = 5001 /
+# 8192 115 -> 102 / 172 -> 115; N = 1024, T = 8192 / 12288 187 -> 226 / 274 -> 208; N = 4096, T = 16384
+# 446 -> 490; beta 0.99 (W 2560) N = 256, T = 8192 / 12288 170 -> 222 / 242 -> 186; N = 1024, T = 16384 /
+# 24576 358 -> 397 / 523 -> 389; N = 2048, T = 16384 / 24576 391 -> 451 / 573 -> 545.
+LAYER_WARM_MIN_T = 3072
+LAYER_WARM_SPIKES_MIN_T = 2048
+
+
+def layer_warm_plan(T, N, beta, grad=True):
+    """(C, W) where a layer's forward (and with grad its adjoint behind it) is faster by warm-started
+    chunks than as the layer pair, else None."""
+    plan = warm_any_plan(T, N, beta)
+    if plan is None or T < (LAYER_WARM_MIN_T if grad else LAYER_WARM_SPIKES_MIN_T):
+        return None
+    if grad and T < (4 if N <= 512 else 8 if N <= 2048 else 24) * plan[1]:
+        return None
+    return plan
 
 
 def _warm_any(I, beta, theta, u_r, u0, C, W):
@@ -931,13 +964,20 @@ def _layer_ok(N):
     return RECOMPUTE_BWD and 1 <= N < 1 << 25
 
 
-def _converged_layer(T, N, beta, K, repair):
-    """True when a converged scan layer (lif_tuned) takes the layer pair: scan_forward_auto would
-    give the serial recurrence's bits and neither warm-started nor long chunks are faster."""
+def _tuned_route(T, N, beta, K, repair):
+    """What a scan-mode lif_tuned call takes instead of scan_forward_auto, with the same spikes: (0, 0)
+    the layer pair, (C, W) warm-started chunks, None neither.  The call has to ask for the converged
+    result (the serial recurrence) with arguments that scan_forward_auto takes."""
+    if _recompute_ok(T, N, K, repair):
+        return 0, 0
     C = _chunk_or_none(T, 16)
-    return (C is not None and T > 0 and _layer_ok(N) and 1 <= int(K) <= 16 and int(repair) >= T // C
-            and warm_plan(T, N, beta) is None and warm_any_plan(T, N, beta) is None
-            and not long_sequence_C(T, N))
+    if C is None or T == 0 or not _layer_ok(N) or not 1 <= int(K) <= 16 or int(repair) < T // C:
+        return None
+    plan = layer_warm_plan(T, N, beta)
+    if plan is None and (long_sequence_C(T, N) or (warm_plan(T, N, beta) is not None and (
+            N > WARM_FEW_MAX_N or _warm_up(beta) is None))):
+        return None  # long chunks, or warm_plan's where layer_warm_plan does not look
+    return plan or (0, 0)
 
 
 def _layer_forward(I, beta, theta, u_r, u0, want_states=True):
@@ -1183,43 +1223,45 @@ def auto_modes(N, T):
 
 
 def _auto_fwd(fwd, N, T):
-    """auto_modes' forward mode, or "auto" where warm-started chunks may apply: the layer's forward
-    then decides from beta (_auto_forward)."""
+    """auto_modes' forward mode, or "auto" where warm-started chunks may apply: the layer then decides
+    from beta (_auto_route)."""
     return "auto" if 1 <= N <= WARM_FEW_MAX_N and T >= 4 * 256 else fwd
 
 
 def _check_auto_args(T, N, K, repair):
     """The map scan's refusals of a capacity or a repair budget, where auto_modes gives lif_auto and
     lif_param that scan, also when the warm-started chunks run in its place."""
-    if T >= AUTO_FWD_MIN_T and auto_modes(N, T)[0] == "scan" and int(repair) < T // _pick_C(T, D=16):
+    if auto_modes(N, T)[0] == "scan" and int(repair) < T // _pick_C(T, D=16):
         if not 1 <= int(K) <= 64:
             raise ValueError("map capacity K must be in [1, 64]")
         if int(repair) < 0:
             raise ValueError("repair must be >= 0")
 
 
-def _auto_states(T, N, beta):
-    """True when a layer that chooses keeps U and S for its adjoint (warm-started chunks, or the map
-    scan where they do not apply) instead of the layer pair's states."""
-    return warm_any_plan(T, N, beta) is not None or (
-        T >= AUTO_FWD_MIN_T and auto_modes(N, T)[0] == "scan")
+def _auto_route(T, N, beta, grad=True):
+    """What lif_auto and lif_param run: (0, 0) the layer pair, (C, W) warm-started chunks, None the map
+    scan (auto_modes' forward where neither is faster: N = 64, T = 16384, beta 0.998)."""
+    if T < LAYER_WARM_SPIKES_MIN_T:
+        return 0, 0
+    plan = layer_warm_plan(T, N, beta, grad)
+    if plan is None and T >= AUTO_FWD_MIN_T and auto_modes(N, T)[0] == "scan":
+        return None
+    return plan or (0, 0)
 
 
-def _auto_forward(I, beta, theta, u_r, u0, K, repair):
-    """(U, S) of a layer's own choice: warm-started chunks (the serial recurrence's bits, faster than
-    the serial sweep and than the map scan: N = 64, T = 50000 0.91 ms of map scan -> 0.06 ms), else
-    auto_modes' forward."""
+def _auto_forward(I, beta, theta, u_r, u0, K, repair, plan, fwd_mode):
+    """(U, S) of a layer that keeps them: warm-started chunks where a plan is given, else the map scan
+    where auto_modes has it (and the mode is not "serial"), else the serial sweep."""
     T, N = I.shape
-    plan = warm_any_plan(T, N, beta)
-    if plan is not None:
+    if plan:
         return _warm_any(I, beta, theta, u_r, u0, *plan)
-    if auto_modes(N, T)[0] == "scan":
+    if fwd_mode != "serial" and auto_modes(N, T)[0] == "scan":
         return scan_forward_auto(I, beta, theta, u_r, u0, K=K, repair=repair)
     return serial_forward_auto(I, beta, theta, u_r, u0)
 
 
-# Up to this many neurons lif_auto's adjoint of a long T that has no chunk (auto_modes: serial) is
-# the look-back pass, serial -> look-back: N = 64, T = 4001 94 -> 19 us; N = 1024, T = 2001 50 -> 19
+# Up to this many neurons the adjoint of stored states of a long T that has no chunk (auto_modes:
+# serial) is the look-back pass, serial -> look-back: N = 64, T = 4001 94 -> 19 us; N = 1024, T = 2001 50 -> 19
 # us; N = 8192, T = 4001 166 -> 119 us.  Above, the serial sweep fills the chip as well (N = 14083,
 # T = 2001: 130 against 151 us; rows of odd N are not aligned, which costs both).
 AUTO_LOOKBACK_MAX_N = 8192
@@ -1293,12 +1335,15 @@ class LIFTuned(torch.autograd.Function):
             ctx.save_for_backward(I, u0, ST)
             ctx.recompute = "single"
             return S
-        if mode != "serial" and _converged_layer(T, N, b, K, repair):
+        route = None if mode == "serial" else _tuned_route(T, N, b, K, repair)
+        if route == (0, 0):
             S, ST = _layer_forward(I, b, theta, u_r, u0)
             ctx.save_for_backward(I, u0, ST)
             ctx.recompute = "layer"
             return S
-        if mode == "serial":
+        if route:
+            U, S = _warm_any(I, b, theta, u_r, u0, *route)
+        elif mode == "serial":
             U, S = serial_forward_auto(I, b, theta, u_r, u0)
         else:
             U, S = scan_forward_auto(I, b, theta, u_r, u0, K=K, repair=repair)
@@ -1372,29 +1417,25 @@ def _grad_param(p):
     return p if type(p) is not float and torch.is_tensor(p) and p.requires_grad else None
 
 
-def _pair_runs(T, N, b, K, repair):
-    """True when a scan-mode lif_tuned call of these sizes takes a recomputing pair."""
-    return _recompute_ok(T, N, K, repair) or _converged_layer(T, N, b, K, repair)
-
-
 def _rc_path(I, u0, beta, mode, K, repair):
-    """u0 as the [N] vector when lif_tuned takes a recomputing pair from C++, else None."""
+    """u0 as the [N] vector when lif_tuned runs from C++, else None."""
     u0v = None if mode == "serial" else _cpp_u0(I, u0)
-    return u0v if u0v is not None and _layer_ok(I.shape[1]) and _pair_runs(*I.shape, _f32(beta), K,
-                                                                           repair) else None
+    if u0v is None or not _layer_ok(I.shape[1]):
+        return None
+    return u0v if _tuned_route(*I.shape, _f32(beta), K, repair) is not None else None
 
 
 def lif_tuned(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, mode="scan", K=16, repair=0):
     u0v = None if mode == "serial" else _cpp_u0(I, u0, theta, u_r, alpha)
     if u0v is None or not _layer_ok(I.shape[1]):
         return LIFTuned.apply(I, u0, beta, theta, u_r, alpha, mode, K, repair)
-    T, N = I.shape
     b, th, ur = _f32s(beta, theta, u_r)  # read once, for the plans and the call
-    if _pair_runs(T, N, b, K, repair):
-        # the same kernels and bits as LIFTuned's recomputing pairs, from C++
-        return _n.ops().lif_layer(I, u0v, _grad_param(beta), None, None, b, th, ur, _f32(alpha),
-                                  _wait_header(I.device), 0, 0)
-    return LIFTuned.apply(I, u0, beta, th, ur, alpha, mode, K, repair, b)
+    route = _tuned_route(*I.shape, b, K, repair)
+    if route is None:
+        return LIFTuned.apply(I, u0, beta, th, ur, alpha, mode, K, repair, b)
+    # the same kernels and bits as LIFTuned's, from C++
+    return _n.ops().lif_layer(I, u0v, _grad_param(beta), None, None, b, th, ur, _f32(alpha),
+                              _wait_header(I.device), *route)
 
 
 class LIFAuto(torch.autograd.Function):
@@ -1404,20 +1445,16 @@ class LIFAuto(torch.autograd.Function):
     def forward(ctx, I, u0, beta, theta, u_r, alpha, K, repair, fwd_mode, bwd_mode, b=None):
         I = I.contiguous()
         b = _f32(beta) if b is None else b
-        ctx.cfg = (b, theta, u_r, alpha, bwd_mode)
         T, N = I.shape
+        route = _auto_route(T, N, b) if _layer_ok(N) and T > 0 else None
+        ctx.cfg = (b, theta, u_r, alpha, "lookback" if route else bwd_mode)
         # the exact forward's bits are the serial one's: U, kept only for the backward, is left out
-        if fwd_mode in ("serial", "auto") and _layer_ok(N) and T > 0 and not _auto_states(T, N, b):
+        if route == (0, 0):
             S, ST = _layer_forward(I, b, theta, u_r, u0)
             ctx.save_for_backward(I, u0, ST)
             ctx.recompute = True
             return S
-        if fwd_mode == "scan":
-            U, S = scan_forward_auto(I, b, theta, u_r, u0, K=K, repair=repair)
-        elif fwd_mode == "auto":
-            U, S = _auto_forward(I, b, theta, u_r, u0, K, repair)
-        else:
-            U, S = serial_forward_auto(I, b, theta, u_r, u0)
+        U, S = _auto_forward(I, b, theta, u_r, u0, K, repair, route, fwd_mode)
         ctx.save_for_backward(I, u0, U, S)
         ctx.recompute = False
         return S
@@ -1447,19 +1484,23 @@ class LIFAuto(torch.autograd.Function):
 
 def lif_auto(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, K=16, repair=0):
     T, N = I.shape
-    _check_auto_args(T, N, K, repair)
+    if T >= AUTO_FWD_MIN_T:
+        _check_auto_args(T, N, K, repair)
     b = None
     if _layer_ok(N) and T > 0:
         u0v = _cpp_u0(I, u0, theta, u_r, alpha)
-        if u0v is not None:  # the same kernels and bits as LIFAuto's layer pair, from C++
+        if u0v is not None:  # the same kernels and bits as LIFAuto's, from C++
             b, th, ur = _f32s(beta, theta, u_r)
-            if not _auto_states(T, N, b):
-                hdr = _wait_header(I.device)
-                if torch.is_grad_enabled() and (I.requires_grad or u0v.requires_grad
-                                                or _grad_param(beta) is not None):
+            grad = torch.is_grad_enabled() and (I.requires_grad or u0v.requires_grad
+                                                or _grad_param(beta) is not None)
+            route = _auto_route(T, N, b, grad)
+            if route is not None:
+                if grad:
                     return _n.ops().lif_layer(I, u0v, _grad_param(beta), None, None, b, th, ur,
-                                              _f32(alpha), hdr, 0, 0)
-                return _n.ops().lif_spikes(I, u0v, b, th, ur, hdr)
+                                              _f32(alpha), _wait_header(I.device), *route)
+                if route == (0, 0):
+                    return _n.ops().lif_spikes(I, u0v, b, th, ur, _wait_header(I.device))
+                return _warm_any(I, b, th, ur, u0v, *route)[1]
             theta, u_r = th, ur  # read once
     fwd, bwd = auto_modes(N, T)
     fwd, bwd = _auto_fwd(fwd, N, T), _auto_bwd(bwd, N, T)

@@ -96,3 +96,24 @@ def test_warm_plan():
     assert L.warm_plan(1000, 64, 0.9) is None                  # no power-of-two chunk
     assert L.warm_plan(2 ** 20, 64, 1.0)[1] == 8192
     assert L.warm_plan(0, 64, 0.9) is None and L.warm_plan(4096, 0, 0.9) is None
+
+
+def test_layer_routes():
+    """Where a layer's steps and spikes leave the pair for warm-started chunks, and where neither runs."""
+    from lifscan import hip_lif as L
+    pair = (0, 0)
+    assert L._auto_route(1024, 1024, 0.9) == pair and L._auto_route(2048, 128, 0.9) == pair
+    assert L._auto_route(3071, 64, 0.9) == pair and L._auto_route(3072, 64, 0.9) == (256, 256)
+    assert L._auto_route(4095, 1024, 0.95) == pair and L._auto_route(4096, 1024, 0.95) == (256, 512)
+    assert L._auto_route(6143, 4096, 0.9) == pair and L._auto_route(6144, 4096, 0.9) == (768, 256)
+    assert L._auto_route(2047, 64, 0.9, False) == pair and L._auto_route(2048, 64, 0.9, False) == (256, 256)
+    assert L._auto_route(2048, 16384, 0.9) == pair and L._auto_route(10239, 64, 0.99) == pair
+    assert L._auto_route(16384, 64, 0.998) is None           # warm-ups too short: the map scan
+    big = 10 ** 6
+    assert L._tuned_route(4096, 1024, 0.95, 16, big) == (256, 512) and L._tuned_route(96, 40, 0.9, 16, big) == pair
+    assert L._tuned_route(4096, 1024, 0.95, 16, 0) is None   # not converged
+    assert L._tuned_route(4096, 1024, 0.95, 0, big) is None and L._tuned_route(1002, 64, 0.9, 16, big) is None
+    assert L._tuned_route(2048, 2048, 0.95, 16, big) == pair  # warm_plan has chunks; the pair is faster
+    assert L._tuned_route(12288, 1024, 0.99, 16, big) == pair
+    assert L._tuned_route(65536, 64, 0.999, 16, big) is None  # warm_plan's own chunks
+    assert L.warm_any_plan(10 ** 6, 64, 0.998) is None

@@ -228,3 +228,27 @@ def test_scan_arguments_are_still_refused(dev):
         L.scan_forward_v3(I[:2064], 0.9, 1.0, 0.0, u0, C=16, K=0, repair=10 ** 6)
     assert L.lif_auto(I, u0, 0.9, K=64).shape == I.shape  # what was taken still is
     assert L.lif_tuned(I[:96], u0, 0.9, K=32, repair=10 ** 6).shape == (96, 8)
+
+
+@pytest.mark.parametrize("call", ["auto", "tuned", "param"])
+@pytest.mark.parametrize("T,N,C", [(1024, 1024, 0), (4096, 70, 256)])
+def test_few_neuron_layers_run_from_cpp(dev, call, T, N, C):
+    """The few-neuron layers, the warm-started chunks among them, run as C++ functions with a look-back
+    adjoint behind the forward, and without gradients as spikes alone."""
+    from lifscan import hip_lif as L
+    from lifscan.fit import lif_param
+    assert L.layer_warm_plan(T, N, 0.9) == ((C, 256) if C else None)
+    I, GS, u0 = normal(T, N, 0.12, 0.25, 1), normal(T, N, 0.0, 1.0, 2), uniform(N, 0.0, 1.0, 3)
+    Uo, So = O.serial_forward(I, 0.9, 1.0, 0.0, u0)
+    want = O.serial_backward(I, u0, Uo, So, GS, None, 0.9, 1.0, 0.0, 4.0, True, dtype=np.float64)
+    Ig, ug = gpu(I, dev).requires_grad_(True), gpu(u0, dev).requires_grad_(True)
+    f = {"auto": lambda: L.lif_auto(Ig, ug, 0.9), "tuned": lambda: L.lif_tuned(Ig, ug, 0.9, repair=10 ** 6),
+         "param": lambda: lif_param(Ig, ug, 0.9, 1.0, 0.0)}[call]
+    print(f"layers {call} T={T} N={N}", flush=True)
+    S = f()
+    assert "LIFLayer" in S.grad_fn.name()
+    dI, du0 = torch.autograd.grad(S, [Ig, ug], gpu(GS, dev))
+    assert np.array_equal(host(S), So)
+    assert rel(host(dI), want) < 1e-6 and rel(host(du0), 0.9 * want[0]) < 1e-6
+    with torch.no_grad():
+        assert np.array_equal(host(f()), So)
