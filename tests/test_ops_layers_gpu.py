@@ -17,11 +17,13 @@ def _data(T, N, dev, seed=7):
 def _both(fns, T, N, params, dev, u0_grad=True, wide_grad=True):
     I, gS, u0 = _data(T, N, dev)
     outs = []
-    for fn in fns:
+    for fn, cpp in zip(fns, (True, False)):
         Ig = I.clone().requires_grad_(True)
         ug = u0.clone().requires_grad_(u0_grad)
         ps = [torch.tensor(p, device=dev, requires_grad=r) for p, r in params]
         S = fn(Ig, ug, *ps)
+        # each side ran as what it is compared as
+        assert ("LIFLayer" in S.grad_fn.name() or "AffLayer" in S.grad_fn.name()) == cpp, S.grad_fn.name()
         if wide_grad:
             S.backward(gS)
         else:

@@ -162,6 +162,7 @@ def test_layer_pair_many_neurons(dev):
 
 
 def _layer_pair(dev, T, N):
+    from lifscan import _native as n
     from lifscan import hip_lif as L
     I, GS, u0 = normal(T, N, 0.15, 0.4, T), normal(T, N, 0.0, 1.0, T + 1), uniform(N, 0.0, 1.0, 3)
     U, S = O.serial_forward(I, 0.95, 1.0, -0.1, u0)
@@ -176,6 +177,8 @@ def _layer_pair(dev, T, N):
     lam, none = L._layer_backward(pad(I), st, pad(GS), 0.95, 1.0, -0.1)
     lam2, sums = L._layer_backward(pad(I), st, pad(GS), 0.95, 1.0, -0.1, 4.0, True)
     assert none is None and rel(host(lam), want) < 1e-6 and rel(host(lam2), want) < 1e-6
+    if n.lib().lsh_lif_layer_bwd_workspace(T, N):  # the look-back adjoint: no wait gave up
+        assert L.last_lookback_timeouts() == 0
     grads = O.param_grads(I, u0, U, S, GS, want, 0.95, 1.0, -0.1, 4.0)
     for k, g in enumerate((sums[0], -sums[1], 0.95 * sums[2])):
         assert abs(g.item() - grads[2 + k]) <= 1e-4 * abs(grads[2 + k]) + 1e-5, k
