@@ -38,7 +38,8 @@ namespace lsh {
 // while the current one is computed).  32 and 64 rows measured the same from N = 64 to 8192.
 constexpr int WARM_D = 16;
 
-// T need not be a multiple of C: the last chunk is short.
+// T need not be a multiple of C: the last chunk is short (whole chunks lose nothing by that: N 1024, T
+// 2^18, beta 0.99 842 us either way).
 template <bool NT>
 __global__ __launch_bounds__(64) void k_lif_fwd_warm(const float* __restrict__ I,
                                                      const float* __restrict__ u0,

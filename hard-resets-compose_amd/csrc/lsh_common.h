@@ -134,11 +134,14 @@ __device__ __forceinline__ void st_nt(T* p, T v) { __builtin_nontemporal_store(v
 template <typename T>
 __device__ __forceinline__ T ld_nt(const T* p) { return __builtin_nontemporal_load(p); }
 
-// The policy of a streaming output's stores by the rows' alignment.  Rows of whole 64-byte pieces
+// The policy of a streaming output's stores by the rows' alignment, in the kernels that take it as a
+// parameter (NT): the serial and single-pass sweeps, replays, the layers' adjoints, the warm-started
+// and the affine replay.  The others, the soft adjoint, the ALIF serial adjoint and the look-back with
+// GU or an undetached reset among them, store non-temporally at every N.  Rows of whole 64-byte pieces
 // (N % 16 == 0) are written non-temporally; otherwise neighbouring waves share a piece at either
 // end of each row, and a non-temporal store writes its part through by itself where a plain one
-// waits in L2 for the rest.  Measured, non-temporal -> plain: N 14083, T 1000 serial forward 60 ->
-// 45 us; N 51453, T 512 136 -> 94 us, its spikes and entry states 90 -> 58, recomputing adjoint 115
+// waits in L2 for the rest.  Measured (from 14083 neurons on; fewer follow the same rule), non-temporal ->
+// plain: N 14083, T 1000 serial forward 60 -> 45 us; N 51453, T 512 136 -> 94 us, its spikes and entry states 90 -> 58, recomputing adjoint 115
 // -> 85; but N 12800, T 1000 27 -> 32 us, N 65536, T 4096 406 -> 423 us.
 inline bool rows_aligned(int64_t N) { return N % 16 == 0; }
 // f(std::true_type) for non-temporal stores, f(std::false_type) for plain ones
