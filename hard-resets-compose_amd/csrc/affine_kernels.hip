@@ -124,11 +124,11 @@ __global__ __launch_bounds__(64) void k_aff_env_carry(
 }
 
 // ---------------------------------------------------------------------------------------
-// Chunk maps (triton_affine.py:51-111).  A workgroup owns 16 neurons of one chunk; a 16-lane row
-// serves one neuron (4 neurons a wave), lane i holding piece slots i and 16 + i; the second is
-// touched only while some neuron of the wave has more than 16 pieces.  Inputs are staged through
-// LDS in tiles of 32 steps together with ct = (theta - x)/beta, computed once per (neuron, step);
-// the next tile's inputs are loaded while a tile runs.
+// Chunk maps (triton_affine.py:51-111).  L lanes serve one neuron of one chunk: a 16-lane row (4
+// neurons a wave, 16 a workgroup), lane i holding piece slots i and 16 + i, the second touched only
+// while some neuron of the wave has more than 16 pieces; or 32 lanes with one slot each.  Inputs are
+// staged through LDS in tiles of 32 steps together with ct = (theta - x)/beta, computed once per
+// (neuron, step); the next tile's inputs are loaded while a tile runs.
 // Per step every piece [xl, xr) with value a*u + c meets the threshold cut z = (ct - c)/a
 // (u >= z spikes; a == 0: all or nothing); its left part [xl, min(xr, z)) and its spiking
 // right part [z, xr) are kept when they meet [lo, hi].
@@ -140,15 +140,21 @@ __global__ __launch_bounds__(64) void k_aff_env_carry(
 // reference's compaction does).  Compacting on every birth and death ran on two steps of three.
 // The tests are kept as wave masks (a ballot of one compare is the compare's own result); free
 // slots drift with the others and the masks leave them out.
-// Bound by VALU issue (a correctly rounded division per piece and step): most maps hold 3 to 9
-// pieces, so 32 lanes a neuron left most lanes idle.  Measured, C 128, 32 lanes a neuron and
-// compaction -> this: T 8192, N 200 gamma 0.5 82 -> 51 us, N 333 soft reset 121 -> 101 us;
-// T 4096, N 4096 537 -> 284 and 543 -> 300 us (16 lanes with compaction 59, 111, 353, 367; 8 lanes
-// and four slots 98, 177, 416, 492).
+// Where the chunks and neurons fill the chip it is bound by VALU issue (a correctly rounded division
+// per piece and step): most maps hold 3 to 9 pieces, so 32 lanes leave most lanes idle.  Measured, C
+// 128, 32 lanes and compaction -> 16 lanes: T 8192, N 200 gamma 0.5 82 -> 51 us, N 333 soft reset 121
+// -> 101 us; T 4096, N 4096 537 -> 284 and 543 -> 300 us (16 lanes with compaction 59, 111, 353, 367;
+// 8 lanes and four slots 98, 177, 416, 492).  With few it is bound by a step's own latency, which a
+// second slot and the sorts of overflowing maps lengthen: up to kAffWideBlocks workgroups of 16
+// neurons take 32 lanes.  The scan, 32 lanes and compaction / 16 lanes / 32 lanes, us, with many pieces
+// (beta 0.99, gamma 0.9) and few (0.9, 0.5): T 512, N 65, C 128, K 32 (20 workgroups) 71 / 103 / 69 and
+// 62 / 58 / 52; T 2048, N 333, C 128 (336) 108 / 136 / 100 and 88 / 65 / 64; C 64, K 16 (672) 121 / 138 /
+// 112 and 84 / 55 / 60; T 8192, N 200, C 128, K 32 (832) 234 / 238 / 198 and 158 / 95 / 105; T 4096, N
+// 1000 (2016) 252 / 265 / 224 and 210 / 120 / 157.
+constexpr int64_t kAffWideBlocks = 768;
 constexpr int kAffWaves = 4;                 // waves per workgroup
-constexpr int kAffNPW = kAffWaves * 4;       // neurons per workgroup
 constexpr int kAffTS = 32;                   // steps per staged tile
-constexpr int kAffLd = kAffNPW * kAffTS / (kAffWaves * WAVE);  // inputs a lane stages per tile
+constexpr int aff_npw(int L) { return kAffWaves * (WAVE / L); }  // neurons per workgroup, L lanes each
 
 // One piece slot's step: the cut, the masks of the kept left / right parts and the updated fields.
 struct AffStepSlot {
@@ -176,20 +182,25 @@ __device__ __forceinline__ AffStepSlot aff_slot_step(float pxl, float pxr, float
   return r;
 }
 
-__global__ __launch_bounds__(WAVE * kAffWaves) void k_aff_build(
+template <int L>
+__global__ __launch_bounds__(WAVE * kAffWaves, 7) void k_aff_build(  // 72 registers: 7 waves a SIMD
     const float* __restrict__ I, const float* __restrict__ LO, const float* __restrict__ HI,
     float4* __restrict__ PC, int* __restrict__ NP, int* __restrict__ OVF, int64_t N, int NBLK,
     int C, int K, float beta, float theta, float gamma, float delta) {
-  __shared__ float sX[kAffNPW][kAffTS + 1], sCt[kAffNPW][kAffTS + 1];
-  __shared__ float4 sSlot[kAffNPW][33];  // a neuron's slots, off the banks of the next neuron's
-  __shared__ float sKey[kAffNPW][65];    // sort keys: at most 32 pieces, each with a new part
+  static_assert(L == 16 || L == 32, "a row holds 32 pieces in one or two slots a lane");
+  constexpr bool TWO = L == 16;  // a lane's second slot
+  constexpr int NPW = aff_npw(L), LD = NPW * kAffTS / (kAffWaves * WAVE);  // LD: inputs a lane stages
+  __shared__ float sX[NPW][kAffTS + 1], sCt[NPW][kAffTS + 1];
+  __shared__ float4 sSlot[NPW][33];  // a neuron's slots, off the banks of the next neuron's
+  // sort keys: at most 32 pieces, each with a new part, and three past the last one
+  __shared__ __attribute__((aligned(16))) float sKey[NPW][TWO ? 65 : 68];
   const int64_t m = blockIdx.x / NBLK;
   const int blk = (int)(blockIdx.x - m * NBLK);
   const int tid = threadIdx.x;
   const int lane = tid % WAVE;
-  const int i = lane & 15;
-  const int ln = tid / 16;  // neuron of the workgroup
-  const int64_t n0 = (int64_t)blk * kAffNPW;
+  const int i = lane & (L - 1);
+  const int ln = tid / L;  // neuron of the workgroup
+  const int64_t n0 = (int64_t)blk * NPW;
   const int64_t n = n0 + ln;
   const bool valid_n = n < N;
   const size_t o = (size_t)m * N + (valid_n ? n : N - 1);
@@ -204,7 +215,7 @@ __global__ __launch_bounds__(WAVE * kAffWaves) void k_aff_build(
   // the row's bits of a wave mask
   const auto row_of = [&](unsigned long long mask) {
     const unsigned w = lane < 32 ? (unsigned)mask : (unsigned)(mask >> 32);
-    return (w >> (lane & 16)) & 0xffffu;
+    return TWO ? (w >> (lane & 16)) & 0xffffu : w;
   };
   const auto lane_of = [](unsigned long long mask) {
     return __builtin_amdgcn_inverse_ballot_w64(mask);
@@ -222,14 +233,26 @@ __global__ __launch_bounds__(WAVE * kAffWaves) void k_aff_build(
     if (h1) key[o1 + __popc(l1 & below)] = pxl1;
     if (g0) key[o2 + __popc(b0 & below)] = n0.x;
     if (g1) key[o3 + __popc(b1 & below)] = n1.x;
+    if (!TWO && i < 3) key[tot + i] = INFINITY;  // counted by nothing
     __builtin_amdgcn_wave_barrier();
     int k0 = 0, k1 = 0, m0 = 0, m1 = 0;  // ranks
-    for (int j = 0; j < tot; ++j) {
-      const float v = key[j];
-      k0 += v < pxl0 ? 1 : 0;
-      k1 += v < pxl1 ? 1 : 0;
-      m0 += v < n0.x ? 1 : 0;
-      m1 += v < n1.x ? 1 : 0;
+    if constexpr (TWO) {
+      for (int j = 0; j < tot; ++j) {
+        const float v = key[j];
+        k0 += v < pxl0 ? 1 : 0;
+        k1 += v < pxl1 ? 1 : 0;
+        m0 += v < n0.x ? 1 : 0;
+        m1 += v < n1.x ? 1 : 0;
+      }
+    } else {  // a step's latency counts: four keys a load
+      const auto count = [](int& k, const float4& v, float x) {
+        k += (v.x < x ? 1 : 0) + (v.y < x ? 1 : 0) + (v.z < x ? 1 : 0) + (v.w < x ? 1 : 0);
+      };
+      for (int j = 0; j < tot; j += 4) {
+        const float4 v = *reinterpret_cast<const float4*>(key + j);
+        count(k0, v, pxl0);
+        count(m0, v, n0.x);
+      }
     }
     if (h0 && k0 < K) slot[k0] = make_float4(pxl0, pxr0, pa0, pc0);
     if (h1 && k1 < K) slot[k1] = make_float4(pxl1, pxr1, pa1, pc1);
@@ -238,21 +261,24 @@ __global__ __launch_bounds__(WAVE * kAffWaves) void k_aff_build(
     if (tot > K) ovf = 1;
     cnt = min(tot, K);
     __builtin_amdgcn_wave_barrier();
-    const float4 q0 = slot[i], q1 = slot[16 + i];
+    const float4 q0 = slot[i];
     pxl0 = q0.x, pxr0 = q0.y, pa0 = q0.z, pc0 = q0.w;
-    pxl1 = q1.x, pxr1 = q1.y, pa1 = q1.z, pc1 = q1.w;
     live0 = wave_ballot(i < cnt);
-    live1 = wave_ballot(16 + i < cnt);
+    if constexpr (TWO) {
+      const float4 q1 = slot[L + i];
+      pxl1 = q1.x, pxr1 = q1.y, pa1 = q1.z, pc1 = q1.w;
+      live1 = wave_ballot(L + i < cnt);
+    }
     __builtin_amdgcn_wave_barrier();
   };
   const float* __restrict__ Im = I + (size_t)m * C * N;
-  float xr[kAffLd];
+  float xr[LD];
   const auto load = [&](int j0) {  // this lane's inputs of the tile at j0 (rows past C: the last)
 #pragma unroll
-    for (int q = 0; q < kAffLd; ++q) {
+    for (int q = 0; q < LD; ++q) {
       const int e = tid + q * kAffWaves * WAVE;
-      const int64_t ne = n0 + e % kAffNPW;
-      xr[q] = Im[(size_t)min(j0 + e / kAffNPW, C - 1) * N + (ne < N ? ne : N - 1)];
+      const int64_t ne = n0 + e % NPW;
+      xr[q] = Im[(size_t)min(j0 + e / NPW, C - 1) * N + (ne < N ? ne : N - 1)];
     }
   };
   load(0);
@@ -260,15 +286,15 @@ __global__ __launch_bounds__(WAVE * kAffWaves) void k_aff_build(
     const int ts = min(kAffTS, C - j0);
     __syncthreads();  // the previous tile has been read
 #pragma unroll
-    for (int q = 0; q < kAffLd; ++q) {
+    for (int q = 0; q < LD; ++q) {
       const int e = tid + q * kAffWaves * WAVE;
-      sX[e % kAffNPW][e / kAffNPW] = xr[q];
-      sCt[e % kAffNPW][e / kAffNPW] = (theta - xr[q]) / beta;
+      sX[e % NPW][e / NPW] = xr[q];
+      sCt[e % NPW][e / NPW] = (theta - xr[q]) / beta;
     }
     __syncthreads();
     load(j0 + kAffTS);
     // second slots that are no longer needed: back to one slot a lane
-    if (live1 != 0ull &&
+    if (TWO && live1 != 0ull &&
         wave_ballot(__popc(row_of(live0)) + __popc(row_of(live1)) > 16) == 0ull)
       sort_row(0ull, 0ull, make_float4(0, 0, 0, 0), make_float4(0, 0, 0, 0));
     float xs = sX[ln][0], cts = sCt[ln][0];
@@ -291,7 +317,7 @@ __global__ __launch_bounds__(WAVE * kAffWaves) void k_aff_build(
       }
       unsigned long long new1 = 0ull;
       float4 n1 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (live1 != 0ull) {
+      if (TWO && live1 != 0ull) {
         const AffStepSlot r1 = aff_slot_step(pxl1, pxr1, pa1, pc1, live1, x, ct, lo, hi, beta, gb,
                                              gamma, delta);
         new1 = r1.left & r1.right;
@@ -306,7 +332,8 @@ __global__ __launch_bounds__(WAVE * kAffWaves) void k_aff_build(
       }
       if ((new0 | new1) == 0ull) continue;
       const unsigned b0 = row_of(new0), b1 = row_of(new1);
-      const unsigned f0 = ~row_of(live0) & 0xffffu, f1 = ~row_of(live1) & 0xffffu;
+      constexpr unsigned row = TWO ? 0xffffu : 0xffffffffu;
+      const unsigned f0 = ~row_of(live0) & row, f1 = TWO ? ~row_of(live1) & row : 0u;
       const int nb0 = __popc(b0), nb = nb0 + __popc(b1), nf0 = __popc(f0);
       if (wave_ballot(32 - nf0 - __popc(f1) + nb > K) != 0ull) {
         sort_row(new0, new1, n0, n1);
@@ -324,7 +351,7 @@ __global__ __launch_bounds__(WAVE * kAffWaves) void k_aff_build(
       pa0 = take ? q.z : pa0;
       pc0 = take ? q.w : pc0;
       live0 |= wave_ballot(take);
-      if (wave_ballot(nb > nf0) != 0ull) {
+      if (TWO && wave_ballot(nb > nf0) != 0ull) {
         const int j1 = nf0 + __popc(f1 & below);
         const bool take1 = ((f1 >> i) & 1u) != 0u && j1 < nb;
         const float4 q1 = slot[j1];
@@ -342,9 +369,9 @@ __global__ __launch_bounds__(WAVE * kAffWaves) void k_aff_build(
   if (i < K)
     PC[o * K + i] = i < cnt ? make_float4(pxl0, pxr0, pa0, pc0)
                             : make_float4(INFINITY, INFINITY, 1.0f, 0.0f);
-  if (16 + i < K)
-    PC[o * K + 16 + i] = 16 + i < cnt ? make_float4(pxl1, pxr1, pa1, pc1)
-                                      : make_float4(INFINITY, INFINITY, 1.0f, 0.0f);
+  if (TWO && L + i < K)
+    PC[o * K + L + i] = L + i < cnt ? make_float4(pxl1, pxr1, pa1, pc1)
+                                    : make_float4(INFINITY, INFINITY, 1.0f, 0.0f);
   if (i == 0) {
     NP[o] = cnt;
     OVF[o] = ovf;
@@ -575,7 +602,7 @@ static int aff_scan_check(int64_t T, int64_t N, int C, int K) {
   if (C < 1 || K < 1 || K > 32) return LSH_ERR_SHAPE;
   if (T % C != 0) return LSH_ERR_DIVISIBILITY;
   const int64_t M = T / C;
-  if (M * ((N + kAffNPW - 1) / kAffNPW) > ((int64_t)1 << 31) - 1) return LSH_ERR_SHAPE;
+  if (M * ((N + aff_npw(16) - 1) / aff_npw(16)) > ((int64_t)1 << 31) - 1) return LSH_ERR_SHAPE;
   return LSH_OK;
 }
 
@@ -631,7 +658,6 @@ extern "C" int lsh_aff_scan_fwd(const float* I, const float* u0, float* U, float
   }
   const int M = (int)(T / C);
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  const int NBLK = (int)((N + kAffNPW - 1) / kAffNPW);
   auto F = [&](size_t off) { return reinterpret_cast<float*>(w + off); };
   auto Iq = [&](size_t off) { return reinterpret_cast<int*>(w + off); };
   float4* PC = reinterpret_cast<float4*>(w + L.PIECES);
@@ -640,9 +666,17 @@ extern "C" int lsh_aff_scan_fwd(const float* I, const float* u0, float* U, float
                      delta, r_theta);
   hipLaunchKernelGGL(k_aff_env_carry, dim3((unsigned)NB), dim3(WAVE), 0, st, u0, F(L.EC), F(L.EA),
                      F(L.EB), F(L.HC), F(L.HA), F(L.HB), F(L.LO), F(L.HI), N, M);
-  hipLaunchKernelGGL(k_aff_build, dim3((unsigned)((int64_t)M * NBLK)), dim3(WAVE * kAffWaves), 0,
-                     st, I, F(L.LO), F(L.HI), PC, Iq(L.NP), Iq(L.OVF), N, NBLK, C, K, beta, theta,
-                     gamma, delta);
+  const auto build = [&](auto lanes) {
+    constexpr int LN = decltype(lanes)::value;
+    const int NBLK = (int)((N + aff_npw(LN) - 1) / aff_npw(LN));
+    hipLaunchKernelGGL(k_aff_build<LN>, dim3((unsigned)((int64_t)M * NBLK)), dim3(WAVE * kAffWaves), 0, st,
+                       I, F(L.LO), F(L.HI), PC, Iq(L.NP), Iq(L.OVF), N, NBLK, C, K, beta, theta, gamma,
+                       delta);
+  };
+  if (M * ((N + aff_npw(16) - 1) / aff_npw(16)) <= kAffWideBlocks)
+    build(std::integral_constant<int, 32>{});
+  else
+    build(std::integral_constant<int, 16>{});
   hipLaunchKernelGGL(k_aff_carry,
                      dim3((unsigned)((N + 2 * kAffCarryWaves - 1) / (2 * kAffCarryWaves))),
                      dim3(WAVE * kAffCarryWaves), 0, st, I, u0, PC,
