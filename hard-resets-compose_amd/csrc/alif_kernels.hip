@@ -1931,7 +1931,7 @@ extern "C" int lsh_alif_serial_fwd(const float* I, const float* u0, const float*
     hipLaunchKernelGGL((k_alif_fwd_pipe<decltype(nt)::value>), dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0,
                        (hipStream_t)stream, I, u0, w0, U, W, S, N, T, beta, rho, q, theta0, u_r,
                        nullptr, nullptr, nullptr, nullptr, 1);
-  });
+  }, kPlainSweep);
   LSH_CHECK_LAUNCH();
   return LSH_OK;
 }
@@ -1949,7 +1949,7 @@ extern "C" int lsh_alif_serial_fwd_dparams(const float* I, const float* u0, cons
     hipLaunchKernelGGL((k_alif_fwd_pipe<decltype(nt)::value>), dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0,
                        (hipStream_t)stream, I, u0, w0, U, W, S, N, T, 0.0f, 0.0f, 0.0f, 0.0f, u_r,
                        params, nullptr, nullptr, nullptr, 1);
-  });
+  }, kPlainSweep);
   LSH_CHECK_LAUNCH();
   return LSH_OK;
 }
@@ -2056,7 +2056,7 @@ extern "C" int lsh_alif_scan_fwd(const float* I, const float* u0, const float* w
       hipLaunchKernelGGL((k_alif_fwd_pipe<decltype(nt)::value>), dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0, st,
                          I, u0, w0, U, W, S, N, T, beta, rho, q, theta0, u_r, nullptr, Iq(L.MSTAR),
                          F(L.EU), F(L.EW), C);
-    });
+    }, kPlainSweep);
   } else if (repair > 0 && M > 1) {
     const int64_t rounds = repair < (int64_t)M ? repair : (int64_t)M;
     hipLaunchKernelGGL(k_alif_repair, dim3((unsigned)NB), dim3(256), 0, st, I, U, W, S, F(L.SU),

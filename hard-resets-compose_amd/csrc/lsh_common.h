@@ -134,20 +134,32 @@ __device__ __forceinline__ void st_nt(T* p, T v) { __builtin_nontemporal_store(v
 template <typename T>
 __device__ __forceinline__ T ld_nt(const T* p) { return __builtin_nontemporal_load(p); }
 
-// The policy of a streaming output's stores by the rows' alignment, in the kernels that take it as a
-// parameter (NT): the serial and single-pass sweeps, replays, the layers' adjoints, the warm-started
-// and the affine replay.  The others, the soft adjoint, the ALIF serial adjoint and the look-back with
-// GU or an undetached reset among them, store non-temporally at every N.  Rows of whole 64-byte pieces
-// (N % 16 == 0) are written non-temporally; otherwise neighbouring waves share a piece at either
-// end of each row, and a non-temporal store writes its part through by itself where a plain one
-// waits in L2 for the rest.  Measured (from 14083 neurons on; fewer follow the same rule), non-temporal ->
-// plain: N 14083, T 1000 serial forward 60 -> 45 us; N 51453, T 512 136 -> 94 us, its spikes and entry states 90 -> 58, recomputing adjoint 115
-// -> 85; but N 12800, T 1000 27 -> 32 us, N 65536, T 4096 406 -> 423 us.
+// The policy of a streaming output's stores, in the kernels that take it as a parameter (NT).  Rows of
+// whole 64-byte pieces (N % 16 == 0) are written non-temporally.  Otherwise neighbouring waves share a
+// piece at either end of each row, and a non-temporal store writes its part through by itself where a
+// plain one waits in L2 for the rest; but plain rows also displace the inputs that L2 and the 256 MB
+// cache hold, which costs the serial sweeps of few neurons more.  So each kernel has a least number of
+// neurons for plain stores.  Measured, non-temporal -> plain, us:
+//   serial sweeps forward, U and S (kPlainSweep)  N 333, T 12576 221 -> 222; N 3333, T 16384 293 -> 420;
+//     N 6001, T 2784 / 11168 56 -> 57 / 205 -> 328; N 10001, T 1664 / 6688 60 -> 44 / 267 -> 249; N
+//     33333, T 480 79 -> 47; the affine and the adaptive sweeps alike (N 6001, T 11168 239 -> 331, 315 ->
+//     417; N 10001, T 1664 60 -> 45, 98 -> 62)
+//   single pass forward, U and S, and adjoints (kPlainSweep)  N 4097, T 4064 106 -> 110 and 108 -> 106; N
+//     10001, T 1664 69 -> 60 and 63 -> 64; N 33333, T 480 89 -> 54 and 66 -> 58
+//   single pass forward, spikes and states (kPlainStarts)  N 10001, T 1664 45 -> 48; N 14083, T 288 11 ->
+//     12; N 20001, T 832 54 -> 46; N 51453, T 1280 229 -> 136
+//   look-back adjoints, replays, warm-started chunks (every N)  N 3333, T 16384 193 -> 168; N 1001, T 4160
+//     131 -> 125; N 3333, T 5024 86 -> 61
+// The sweep's spikes and states and the serial adjoint were never faster with plain stores (N 8191, T
+// 8192 154 -> 178; N 3333, T 5024 140 -> 210) and, like the soft adjoint, the ALIF serial adjoint and the
+// look-back with GU or an undetached reset, store non-temporally at every N.
+// Aligned rows lose with plain stores: N 12800, T 1000 27 -> 32 us, N 65536, T 4096 406 -> 423 us.
+constexpr int64_t kPlainSweep = 8192, kPlainStarts = 16384;
 inline bool rows_aligned(int64_t N) { return N % 16 == 0; }
 // f(std::true_type) for non-temporal stores, f(std::false_type) for plain ones
 template <class F>
-inline void with_store_policy(int64_t N, F&& f) {
-  if (rows_aligned(N))
+inline void with_store_policy(int64_t N, F&& f, int64_t plain_from = 0) {
+  if (rows_aligned(N) || N < plain_from)
     f(std::true_type{});
   else
     f(std::false_type{});

@@ -50,7 +50,7 @@ __device__ __forceinline__ int pipe_tile_rows(int64_t T, int64_t k) {
 // serial_bwd_kernel, :1088-1135 bwd_tiled_pf_kernel): tiles from the end of time, coefficients
 // as k_lif_bwd's (v = fl(fl(beta*u_{t-1}) + x_t), sg = surrogate'(v - theta), J = 1 - s_t
 // (+ (u_r - v)*sg when the reset is not detached), a = beta*J, b = gs*sg + J*gu).
-template <bool DETACH, bool HAS_GU, bool NT>
+template <bool DETACH, bool HAS_GU>
 __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_bwd_pipe(
     const float* __restrict__ I, const float* __restrict__ u0, const float* __restrict__ U,
     const float* __restrict__ S, const float* __restrict__ GS, const float* __restrict__ GU,
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_bwd_pipe(
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int j = p + r * P;
-        if (j < nr) st_row<NT>(Lam + (size_t)(lo + j) * (size_t)N + (size_t)nb0, sb, sL[buf][j][lane]);
+        if (j < nr) st_row(Lam + (size_t)(lo + j) * (size_t)N + (size_t)nb0, sb, sL[buf][j][lane]);
       }
     }
     __syncthreads();
@@ -322,12 +322,11 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_serial_fwd_pipe(
 // comparison by 16 waves instead of 4); N 1000, T 60001, beta 0.95 (C 1888; sweep 1.20 ms) constant
 // current 5.25 -> 2.24 ms; N 4096, T 16001 (C 2000; 0.30 ms) 1.41 -> 0.75 ms.
 constexpr int kWarmScanAhead = 8;  // chunks a wave compares at once
-template <bool NT>
 __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_warm_finish(
     const float* __restrict__ I, float* __restrict__ U, float* __restrict__ S, float* starts,
     float* ends, int* list0, int* list1, WsHeader* hdr, int64_t T, int64_t N, int M, int C,
     int budget, LifStep step) {
-  constexpr int NW = PIPE_P + 1, NT_ALL = WAVE * NW;
+  constexpr int NW = PIPE_P + 1, NT = WAVE * NW;
   __shared__ FwdTiles sh;
   __shared__ int s_nd, s_nc, s_first;
   const int tid = threadIdx.x, lane = tid % WAVE;
@@ -365,13 +364,13 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_warm_finish(
     if (units > budget) break;
     budget -= units;
     ++rounds;
-    for (int i = tid; i < nd; i += NT_ALL) {
+    for (int i = tid; i < nd; i += NT) {
       const size_t o = (size_t)(dl[i] / WAVE) * N + (size_t)(nb0 + dl[i] % WAVE);
       starts[o] = ends[o - N];
     }
     if (tid == 0) s_nc = 0;
     __syncthreads();
-    for (int i = tid; i < nd; i += NT_ALL) {
+    for (int i = tid; i < nd; i += NT) {
       const int e = dl[i], m = e / WAVE;
       const size_t o = (size_t)m * N + (size_t)(nb0 + e % WAVE);
       const size_t base = (size_t)m * C * N + (size_t)(nb0 + e % WAVE);
@@ -392,7 +391,7 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_warm_finish(
     }
     if (tid == 0) s_nd = 0;
     __syncthreads();
-    for (int i = tid; i < s_nc; i += NT_ALL) {
+    for (int i = tid; i < s_nc; i += NT) {
       const int e = cl[i];
       const size_t o = (size_t)(e / WAVE) * N + (size_t)(nb0 + e % WAVE);
       if (!same_bits(ends[o - N], starts[o])) dl[atomicAdd(&s_nd, 1)] = e;
@@ -402,12 +401,12 @@ __global__ __launch_bounds__(WAVE*(PIPE_P + 1)) void k_lif_warm_finish(
   }
   if (tid == 0) atomicMax(&hdr->repair_iters, (unsigned int)(rounds + (nd > 0 ? 1 : 0)));
   if (nd == 0) return;
-  for (int i = tid; i < nd; i += NT_ALL) atomicMin(&s_first, dl[i] / WAVE);
+  for (int i = tid; i < nd; i += NT) atomicMin(&s_first, dl[i] / WAVE);
   __builtin_amdgcn_s_waitcnt(0);  // the rounds' stores land before the sweep's to the same rows
   __syncthreads();
   const int c0 = s_first;
   const size_t row0 = (size_t)c0 * C;
-  serial_fwd_tiles<LifStep, NT, false>(sh, I + row0 * N, ends + (size_t)(c0 - 1) * N, U + row0 * N,
+  serial_fwd_tiles<LifStep, true, false>(sh, I + row0 * N, ends + (size_t)(c0 - 1) * N, U + row0 * N,
                                        S + row0 * N, nb0, N, T - (int64_t)row0, step);
 }
 
@@ -418,11 +417,8 @@ void lif_warm_finish_launch(const float* I, float* U, float* S, float* starts, f
                             int* list1, WsHeader* hdr, int64_t T, int64_t N, int M, int C, float beta,
                             float theta, float u_r, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  with_store_policy(N, [&](auto nt) {
-    hipLaunchKernelGGL((k_lif_warm_finish<decltype(nt)::value>), dim3((unsigned)NB),
-                       dim3(WAVE * (PIPE_P + 1)), 0, st, I, U, S, starts, ends, list0, list1, hdr, T, N, M,
-                       C, M / 5, LifStep(beta, theta, u_r));
-  });
+  hipLaunchKernelGGL(k_lif_warm_finish, dim3((unsigned)NB), dim3(WAVE * (PIPE_P + 1)), 0, st, I, U, S,
+                     starts, ends, list0, list1, hdr, T, N, M, C, M / 5, LifStep(beta, theta, u_r));
 }
 
 void lif_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, int64_t N, int64_t T,
@@ -431,17 +427,14 @@ void lif_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, in
   with_store_policy(N, [&](auto nt) {
     hipLaunchKernelGGL((k_serial_fwd_pipe<LifStep, decltype(nt)::value>), dim3((unsigned)NB),
                        dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, U, S, N, T, LifStep(beta, theta, u_r));
-  });
+  }, kPlainSweep);
 }
 
 void lif_starts_fwd_pipe(const float* I, const float* u0, float* STARTS, float* S, int64_t N, int64_t T,
                          float beta, float theta, float u_r, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  with_store_policy(N, [&](auto nt) {
-    hipLaunchKernelGGL((k_serial_fwd_pipe<LifStep, decltype(nt)::value, true>), dim3((unsigned)NB),
-                       dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, STARTS, S, N, T,
-                       LifStep(beta, theta, u_r));
-  });
+  hipLaunchKernelGGL((k_serial_fwd_pipe<LifStep, true, true>), dim3((unsigned)NB),
+                     dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, STARTS, S, N, T, LifStep(beta, theta, u_r));
 }
 
 void aff_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, int64_t N, int64_t T,
@@ -451,7 +444,7 @@ void aff_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, in
     hipLaunchKernelGGL((k_serial_fwd_pipe<AffStep, decltype(nt)::value>), dim3((unsigned)NB),
                        dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, U, S, N, T,
                        AffStep{beta, theta, gamma, delta});
-  });
+  }, kPlainSweep);
 }
 
 template <bool DETACH, bool HAS_GU>
@@ -459,11 +452,8 @@ static void launch_lif_bwd_pipe(const float* I, const float* u0, const float* U,
                                 const float* GS, const float* GU, float* Lam, int64_t N, int64_t T,
                                 float beta, float theta, float u_r, float alpha, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  with_store_policy(N, [&](auto nt) {
-    hipLaunchKernelGGL((k_lif_bwd_pipe<DETACH, HAS_GU, decltype(nt)::value>), dim3((unsigned)NB),
-                       dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, U, S, GS, GU, Lam, N, T, beta, theta,
-                       u_r, alpha);
-  });
+  hipLaunchKernelGGL((k_lif_bwd_pipe<DETACH, HAS_GU>), dim3((unsigned)NB), dim3(WAVE * (PIPE_P + 1)),
+                     0, st, I, u0, U, S, GS, GU, Lam, N, T, beta, theta, u_r, alpha);
 }
 
 void lif_serial_bwd_pipe(const float* I, const float* u0, const float* U, const float* S,

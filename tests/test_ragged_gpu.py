@@ -255,3 +255,28 @@ def test_few_neuron_layers_run_from_cpp(dev, call, T, N, C):
     assert rel(host(dI), want) < 1e-6 and rel(host(du0), 0.9 * want[0]) < 1e-6
     with torch.no_grad():
         assert np.array_equal(host(f()), So)
+
+
+@pytest.mark.parametrize("N", [8191, 8193, 16401])
+def test_store_policies_of_many_neurons(dev, N):
+    """Rows that are no multiple of 64 bytes on both sides of the kernels' least numbers of neurons for
+    plain stores."""
+    from lifscan import hip_lif as L
+    from lifscan import triton_affine as AF
+    from oracle import affine_oracle as AO
+    test_row_alignment_store_policies(dev, N)
+    T = 64
+    I, GS, u0 = normal(T, N, 0.15, 0.4, N), normal(T, N, 0.0, 1.0, N + 1), uniform(N, 0.0, 1.0, 3)
+    Ig, Gg, ug = gpu(I, dev), gpu(GS, dev), gpu(u0, dev)
+    Uo, So = O.serial_forward(I, 0.95, 1.0, 0.0, u0)
+    want = O.serial_backward(I, u0, Uo, So, GS, None, 0.95, 1.0, 0.0, 4.0, True, dtype=np.float64)
+    U, S = L.scan_forward_exact(Ig, 0.95, 1.0, 0.0, ug, maps=False)
+    assert np.array_equal(host(U), Uo) and np.array_equal(host(S), So)
+    S, ST = L._layer_forward(Ig[:63], 0.95, 1.0, 0.0, ug)
+    assert np.array_equal(host(S), So[:63])
+    assert np.array_equal(host(ST), np.stack([u0, Uo[31]]))
+    lam, sums = L._layer_backward(Ig, L._layer_forward(Ig, 0.95, 1.0, 0.0, ug)[1], Gg, 0.95, 1.0, 0.0, 4.0, True)
+    assert rel(host(lam), want) < 1e-6
+    Ua, Sa = AO.serial_forward(I, 0.95, 1.0, 0.5, -0.25, u0)
+    U, S = AF.aff_serial_forward(Ig, 0.95, 1.0, 0.5, -0.25, ug)
+    assert np.array_equal(host(U), Ua) and np.array_equal(host(S), Sa)
