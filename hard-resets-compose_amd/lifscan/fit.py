@@ -119,7 +119,7 @@ def lif_param(I, u0, beta, theta, u_r, alpha=4.0, mode="auto", K=16):
         u0v = L._cpp_u0(I, u0, alpha) if L._layer_ok(N) else None
         if u0v is not None:  # the same kernels as LIFParamFn's, from C++
             b, th, ur = choose = _f32s(beta, theta, u_r)
-            route = L._auto_route(T, N, b)
+            route = L._auto_route(T, N, b, L._wants_grad(I, u0v, beta, theta, u_r))
             if route is not None:
                 return _n.ops().lif_layer(I, u0v, *map(L._grad_param, (beta, theta, u_r)), b, th, ur,
                                           float(alpha), L._wait_header(I.device), *route)

@@ -964,7 +964,7 @@ def _layer_ok(N):
     return RECOMPUTE_BWD and 1 <= N < 1 << 25
 
 
-def _tuned_route(T, N, beta, K, repair):
+def _tuned_route(T, N, beta, K, repair, grad=True):
     """What a scan-mode lif_tuned call takes instead of scan_forward_auto, with the same spikes: (0, 0)
     the layer pair, (C, W) warm-started chunks, None neither.  The call has to ask for the converged
     result (the serial recurrence) with arguments that scan_forward_auto takes."""
@@ -973,7 +973,7 @@ def _tuned_route(T, N, beta, K, repair):
     C = _chunk_or_none(T, 16)
     if C is None or T == 0 or not _layer_ok(N) or not 1 <= int(K) <= 16 or int(repair) < T // C:
         return None
-    plan = layer_warm_plan(T, N, beta)
+    plan = layer_warm_plan(T, N, beta, grad)
     if plan is None and (long_sequence_C(T, N) or (warm_plan(T, N, beta) is not None and (
             N > WARM_FEW_MAX_N or _warm_up(beta) is None))):
         return None  # long chunks, or warm_plan's where layer_warm_plan does not look
@@ -1417,6 +1417,12 @@ def _grad_param(p):
     return p if type(p) is not float and torch.is_tensor(p) and p.requires_grad else None
 
 
+def _wants_grad(I, u0, *params):
+    """True when a layer call's result will be differentiated."""
+    return torch.is_grad_enabled() and (I.requires_grad or u0.requires_grad
+                                        or any(_grad_param(p) is not None for p in params))
+
+
 def _rc_path(I, u0, beta, mode, K, repair):
     """u0 as the [N] vector when lif_tuned runs from C++, else None."""
     u0v = None if mode == "serial" else _cpp_u0(I, u0)
@@ -1430,7 +1436,7 @@ def lif_tuned(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, mode="scan", K=16,
     if u0v is None or not _layer_ok(I.shape[1]):
         return LIFTuned.apply(I, u0, beta, theta, u_r, alpha, mode, K, repair)
     b, th, ur = _f32s(beta, theta, u_r)  # read once, for the plans and the call
-    route = _tuned_route(*I.shape, b, K, repair)
+    route = _tuned_route(*I.shape, b, K, repair, _wants_grad(I, u0v, beta))
     if route is None:
         return LIFTuned.apply(I, u0, beta, th, ur, alpha, mode, K, repair, b)
     # the same kernels and bits as LIFTuned's, from C++
@@ -1491,8 +1497,7 @@ def lif_auto(I, u0, beta=0.9, theta=1.0, u_r=0.0, alpha=4.0, K=16, repair=0):
         u0v = _cpp_u0(I, u0, theta, u_r, alpha)
         if u0v is not None:  # the same kernels and bits as LIFAuto's, from C++
             b, th, ur = _f32s(beta, theta, u_r)
-            grad = torch.is_grad_enabled() and (I.requires_grad or u0v.requires_grad
-                                                or _grad_param(beta) is not None)
+            grad = _wants_grad(I, u0v, beta)
             route = _auto_route(T, N, b, grad)
             if route is not None:
                 if grad:

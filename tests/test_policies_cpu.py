@@ -111,6 +111,8 @@ def test_layer_routes():
     assert L._auto_route(16384, 64, 0.998) is None           # warm-ups too short: the map scan
     big = 10 ** 6
     assert L._tuned_route(4096, 1024, 0.95, 16, big) == (256, 512) and L._tuned_route(96, 40, 0.9, 16, big) == pair
+    assert L._tuned_route(2048, 64, 0.95, 16, big) == pair   # spikes alone leave the pair sooner
+    assert L._tuned_route(2048, 64, 0.95, 16, big, False) == (256, 512)
     assert L._tuned_route(4096, 1024, 0.95, 16, 0) is None   # not converged
     assert L._tuned_route(4096, 1024, 0.95, 0, big) is None and L._tuned_route(1002, 64, 0.9, 16, big) is None
     assert L._tuned_route(2048, 2048, 0.95, 16, big) == pair  # warm_plan has chunks; the pair is faster
