@@ -600,7 +600,7 @@ __global__ __launch_bounds__(64) void k_lif_carry_wave(
           ovf_o = ovf ? 1 : 0;
         }
         if (ovf)  // rare: serial fallback through this chunk
-          nu = wave_serial_rows(I, N, n, (int64_t)(w * 64 + c) * C, C, u, beta, theta, u_r);
+          nu = wave_serial_rows<RW == 32>(I, N, n, (int64_t)(w * 64 + c) * C, C, u, beta, theta, u_r);
         u = nu;
         ovf_acc += ovf ? 1ull : 0ull;
         pcs_acc += (unsigned long long)ne;

@@ -73,17 +73,29 @@ __device__ __forceinline__ float lif_walk(float& p, float x, float beta, float t
 // holds the same state u): the rows are read 64 at a time, one per lane, the next 64 (index
 // clamped to the last row) while a block is walked, and each step takes its input from its lane.
 // The same values as the replay's.
+// SMALL: for a kernel that holds many copies of the walk, which outgrow the instruction cache when
+// every step is unrolled (k_lif_carry_wave<32>, 32 copies: 154 -> 167 us a pass without fallbacks, N 64,
+// M 512): 16 steps unrolled, carried by u.
+template <bool SMALL = false>
 __device__ __forceinline__ float wave_serial_rows(const float* __restrict__ I, int64_t N,
                                                   int64_t n, int64_t r0, int64_t L, float u,
                                                   float beta, float theta, float u_r) {
   const int lane = threadIdx.x & 63;
   const float* Ip = I + (size_t)r0 * N + n;
   const float kr = __fmul_rn(beta, u_r);
-  float p = __fmul_rn(beta, u), v = 0.0f;
+  float p = SMALL ? u : __fmul_rn(beta, u), v = 0.0f;
   float xv = Ip[(size_t)min<int64_t>(lane, L - 1) * N];
   for (int64_t t0 = 0; t0 < L; t0 += 64) {
     const float xn = Ip[(size_t)min<int64_t>(t0 + 64 + lane, L - 1) * N];
-    if (L - t0 >= 64) {
+    if constexpr (SMALL) {
+      bool s;
+      if (L - t0 >= 64) {
+#pragma unroll 16
+        for (int j = 0; j < 64; ++j) p = lif_step(p, lane_f(xv, j), beta, theta, u_r, s);
+      } else {
+        for (int j = 0; j < (int)(L - t0); ++j) p = lif_step(p, lane_f(xv, j), beta, theta, u_r, s);
+      }
+    } else if (L - t0 >= 64) {
 #pragma unroll
       for (int j = 0; j < 64; ++j) v = lif_walk(p, lane_f(xv, j), beta, theta, kr);
     } else {
@@ -91,6 +103,7 @@ __device__ __forceinline__ float wave_serial_rows(const float* __restrict__ I, i
     }
     xv = xn;
   }
+  if constexpr (SMALL) return p;
   return v >= theta ? u_r : v;
 }
 
