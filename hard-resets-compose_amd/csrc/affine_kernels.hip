@@ -681,7 +681,7 @@ extern "C" int lsh_aff_scan_fwd(const float* I, const float* u0, float* U, float
                      dim3((unsigned)((N + 2 * kAffCarryWaves - 1) / (2 * kAffCarryWaves))),
                      dim3(WAVE * kAffCarryWaves), 0, st, I, u0, PC,
                      Iq(L.NP), Iq(L.OVF), F(L.STARTS), h, N, M, C, K, beta, theta, gamma, delta);
-  with_store_policy(N, [&](auto nt) {
+  with_store_policy(rows_aligned(N), [&](auto nt) {
     hipLaunchKernelGGL((k_aff_fwd<16, decltype(nt)::value>), dim3((unsigned)((int64_t)M * NB)), dim3(WAVE), 0, st, I,
                      F(L.STARTS), U, S, F(L.ENDS), N, (int64_t)C, NB, beta, theta, gamma, delta);
   });

@@ -1909,7 +1909,7 @@ static void launch_alif_fwd(const float* I, const float* su, const float* sw, fl
                             float beta, float rho, float q, float theta0, float u_r, hipStream_t st,
                             const float* dpar = nullptr, const int* mstar = nullptr) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  with_store_policy(N, [&](auto nt) {
+  with_store_policy(rows_aligned(N), [&](auto nt) {
     hipLaunchKernelGGL((k_alif_fwd<D, decltype(nt)::value>), dim3((unsigned)(M * NB)), dim3(WAVE), 0, st,
                        I, su, sw, U, W, S, eu, ew, N, Ls, NB, beta, rho, q, theta0, u_r, dpar, mstar);
   });
@@ -1927,11 +1927,11 @@ extern "C" int lsh_alif_serial_fwd(const float* I, const float* u0, const float*
   if (T < 0 || N < 0 || N > (int64_t)1 << 31) return LSH_ERR_SHAPE;
   if (T == 0 || N == 0) return LSH_OK;
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  with_store_policy(N, [&](auto nt) {
+  with_store_policy(nt_sweep(N), [&](auto nt) {
     hipLaunchKernelGGL((k_alif_fwd_pipe<decltype(nt)::value>), dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0,
                        (hipStream_t)stream, I, u0, w0, U, W, S, N, T, beta, rho, q, theta0, u_r,
                        nullptr, nullptr, nullptr, nullptr, 1);
-  }, kPlainSweep);
+  });
   LSH_CHECK_LAUNCH();
   return LSH_OK;
 }
@@ -1945,11 +1945,11 @@ extern "C" int lsh_alif_serial_fwd_dparams(const float* I, const float* u0, cons
   if (T < 0 || N < 0 || N > (int64_t)1 << 31) return LSH_ERR_SHAPE;
   if (T == 0 || N == 0) return LSH_OK;
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  with_store_policy(N, [&](auto nt) {
+  with_store_policy(nt_sweep(N), [&](auto nt) {
     hipLaunchKernelGGL((k_alif_fwd_pipe<decltype(nt)::value>), dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0,
                        (hipStream_t)stream, I, u0, w0, U, W, S, N, T, 0.0f, 0.0f, 0.0f, 0.0f, u_r,
                        params, nullptr, nullptr, nullptr, 1);
-  }, kPlainSweep);
+  });
   LSH_CHECK_LAUNCH();
   return LSH_OK;
 }
@@ -2052,11 +2052,11 @@ extern "C" int lsh_alif_scan_fwd(const float* I, const float* u0, const float* w
                       u_r, st, nullptr, chain ? Iq(L.MSTAR) : nullptr);
   mark(4);
   if (chain) {
-    with_store_policy(N, [&](auto nt) {
+    with_store_policy(nt_sweep(N), [&](auto nt) {
       hipLaunchKernelGGL((k_alif_fwd_pipe<decltype(nt)::value>), dim3((unsigned)NB), dim3(WAVE * (ALIF_PIPE_P + 1)), 0, st,
                          I, u0, w0, U, W, S, N, T, beta, rho, q, theta0, u_r, nullptr, Iq(L.MSTAR),
                          F(L.EU), F(L.EW), C);
-    }, kPlainSweep);
+    });
   } else if (repair > 0 && M > 1) {
     const int64_t rounds = repair < (int64_t)M ? repair : (int64_t)M;
     hipLaunchKernelGGL(k_alif_repair, dim3((unsigned)NB), dim3(256), 0, st, I, U, W, S, F(L.SU),
@@ -2101,7 +2101,7 @@ static void launch_alif_fused_w(const float* I, const float* u0, const float* w0
                        rho, q, theta0, alpha, u_r, dpar);
   };
   if constexpr (RC && !WLW)  // the layer's adjoint
-    with_store_policy(N, launch);
+    with_store_policy(nt_adjoint((int64_t)M * C, N), launch);
   else
     launch(std::true_type{});
 }
@@ -2166,7 +2166,7 @@ static void alif_lookback_launch(const float* I, const float* U, const float* W,
                      dim3(WAVE * ALIF_LB_W), 0, st, I, u0, w0, U, W, S, GS, LW, LV, DW0, partials,  \
                      agg, flags, hdr, N, NB, NSEG, beta, rho, q, theta0, alpha, u_r, dpar)
 #define LSH_LB(WL, P) LSH_LB_NT(WL, P, true)
-  if (RC && !wlw && !rows_aligned(N)) {  // the layer's adjoint
+  if (RC && !wlw && !nt_adjoint(T, N)) {  // the layer's adjoint
     if (ps)
       LSH_LB_NT(false, true, false);
     else

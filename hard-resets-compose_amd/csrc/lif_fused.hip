@@ -392,7 +392,7 @@ static void launch_fwd_fused(const float* I, const float* u0, float* U, float* S
   if constexpr (SPEC)
     launch(std::true_type{});
   else
-    with_store_policy(N, launch, SO ? kPlainStarts : kPlainSweep);
+    with_store_policy(SO ? nt_starts(N) : nt_sweep(N), launch);
 }
 
 // The starts-only forward of any T with chunks of 32 (STARTS may be NULL).
@@ -402,7 +402,7 @@ static void launch_fwd_starts_any(const float* I, const float* u0, float* STARTS
                                   hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
   const int M = (int)((T + 31) / 32);
-  with_store_policy(N, [&](auto nt) {
+  with_store_policy(nt_starts(N), [&](auto nt) {
     constexpr bool NT = decltype(nt)::value;
     const auto launch = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)NB), dim3(WAVE * W), 0, st, I, u0, STARTS, S, h, T, N, M,
@@ -410,7 +410,7 @@ static void launch_fwd_starts_any(const float* I, const float* u0, float* STARTS
     };
     T % 32 == 0 ? launch(k_lif_fwd_fused<1, 32, W, false, true, NT>)
                 : launch(k_lif_fwd_fused<1, 32, W, false, true, NT, true>);
-  }, kPlainStarts);
+  });
 }
 
 // The chunked-serial exact forward (no maps) writing S and the chunk entry states only.
@@ -489,7 +489,7 @@ static void launch_bwd_fused(const float* I, const float* u0, const float* U, co
                        (int64_t)M * C, N, M, beta, theta, u_r, alpha);
   };
   if constexpr (DETACH && !HAS_GU)
-    with_store_policy(N, launch, kPlainSweep);
+    with_store_policy(nt_sweep(N) || nt_adjoint((int64_t)M * C, N), launch);
   else
     launch(std::true_type{});
 }
@@ -542,7 +542,7 @@ static void launch_bwd_rc(const float* I, const float* STARTS, const float* GS, 
                           float u_r, float alpha, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
   const bool rag = T != (int64_t)M * C;
-  with_store_policy(N, [&](auto nt) {
+  with_store_policy(nt_sweep(N) || nt_adjoint(T, N), [&](auto nt) {
     constexpr bool NT = decltype(nt)::value;
     const auto launch = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)NB), dim3(WAVE * W), 0, st, I, STARTS, STARTS, nullptr,
@@ -557,7 +557,7 @@ static void launch_bwd_rc(const float* I, const float* STARTS, const float* GS, 
     }
     partials ? launch(k_lif_bwd_fused<C, W, true, false, 1, true, NT>)
              : launch(k_lif_bwd_fused<C, W, true, false, 0, true, NT>);
-  }, kPlainSweep);
+  });
 }
 
 template <int C>
@@ -589,7 +589,7 @@ static void launch_param_fused(const float* I, const float* u0, const float* U, 
                                float beta, float theta, float u_r, float alpha, int ps,
                                hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  with_store_policy(N, [&](auto nt) {
+  with_store_policy(nt_sweep(N) || nt_adjoint((int64_t)M * C, N), [&](auto nt) {
     constexpr bool NT = decltype(nt)::value;
     if (ps == 2)
       hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 2, false, NT>), dim3((unsigned)NB),
@@ -599,7 +599,7 @@ static void launch_param_fused(const float* I, const float* u0, const float* U, 
       hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 1, false, NT>), dim3((unsigned)NB),
                          dim3(WAVE * W), 0, st, I, u0, U, S, GS, nullptr, Lam, partials, (int64_t)M * C, N,
                          M, beta, theta, u_r, alpha);
-  }, kPlainSweep);
+  });
 }
 
 template <int C>

@@ -1039,7 +1039,7 @@ static void launch_fwd(const float* I, const float* starts, float* U, float* S, 
                        int64_t N, int64_t Ls, int64_t M, float beta, float theta, float u_r,
                        hipStream_t st, const int* done = nullptr) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  with_store_policy(N, [&](auto nt) {
+  with_store_policy(rows_aligned(N), [&](auto nt) {
     hipLaunchKernelGGL((k_lif_fwd<D, decltype(nt)::value>), dim3((unsigned)(M * NB)), dim3(WAVE), 0, st,
                        I, starts, U, S, ends, N, Ls, NB, beta, theta, u_r, done);
   });

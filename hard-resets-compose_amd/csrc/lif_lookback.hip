@@ -270,7 +270,7 @@ static void launch_lookback(const float* I, const float* u0, const float* U, con
       launch(k_lif_bwd_lookback<C, W, DETACH, HAS_GU, PS, true, NT, RC>);
   };
   if constexpr ((C == 16 && DETACH && !HAS_GU) || RC)
-    with_store_policy(N, by_length);
+    with_store_policy(nt_adjoint(T, N), by_length);
   else
     by_length(std::true_type{});
 }

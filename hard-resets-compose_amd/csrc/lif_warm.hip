@@ -168,7 +168,7 @@ static int warm_run(const float* I, const float* u0, float* U, float* S, int64_t
   const int NB = (int)((N + WAVE - 1) / WAVE);
   float* starts = reinterpret_cast<float*>(w + L.STARTS);
   float* ends = reinterpret_cast<float*>(w + L.ENDS);
-  with_store_policy(N, [&](auto nt) {
+  with_store_policy(nt_warm(N), [&](auto nt) {
     hipLaunchKernelGGL((k_lif_fwd_warm<decltype(nt)::value>), dim3((unsigned)((int64_t)M * NB)), dim3(WAVE), 0, st, I, u0, U, S,
                      starts, ends, T, N, C, W, NB, beta, theta, u_r);
   });

@@ -151,28 +151,36 @@ __device__ __forceinline__ T ld_nt(const T* p) { return __builtin_nontemporal_lo
 // whole 64-byte pieces (N % 16 == 0) are written non-temporally.  Otherwise neighbouring waves share a
 // piece at either end of each row, and a non-temporal store writes its part through by itself where a
 // plain one waits in L2 for the rest; but plain rows also displace the inputs that L2 and the 256 MB
-// cache hold, which costs the serial sweeps of few neurons more.  So each kernel has a least number of
-// neurons for plain stores.  Measured, non-temporal -> plain, us:
-//   serial sweeps forward, U and S (kPlainSweep)  N 333, T 12576 221 -> 222; N 3333, T 16384 293 -> 420;
+// cache hold.  So each kernel has bounds of its own.  Measured, non-temporal -> plain, us:
+//   nt_sweep: serial sweeps forward, U and S  N 333, T 12576 221 -> 222; N 3333, T 16384 293 -> 420;
 //     N 6001, T 2784 / 11168 56 -> 57 / 205 -> 328; N 10001, T 1664 / 6688 60 -> 44 / 267 -> 249; N
 //     33333, T 480 79 -> 47; the affine and the adaptive sweeps alike (N 6001, T 11168 239 -> 331, 315 ->
-//     417; N 10001, T 1664 60 -> 45, 98 -> 62)
-//   single pass forward, U and S, and adjoints (kPlainSweep)  N 4097, T 4064 106 -> 110 and 108 -> 106; N
-//     10001, T 1664 69 -> 60 and 63 -> 64; N 33333, T 480 89 -> 54 and 66 -> 58
-//   single pass forward, spikes and states (kPlainStarts)  N 10001, T 1664 45 -> 48; N 14083, T 288 11 ->
+//     417; N 10001, T 1664 60 -> 45, 98 -> 62); the single pass forward  N 4097, T 4064 106 -> 110; N
+//     10001, T 1664 69 -> 60; N 33333, T 480 / 4000 89 -> 54 / 795 -> 715
+//   nt_starts: single pass forward, spikes and states  N 10001, T 1664 45 -> 48; N 14083, T 288 11 ->
 //     12; N 20001, T 832 54 -> 46; N 51453, T 1280 229 -> 136
-//   look-back adjoints, replays, warm-started chunks (every N)  N 3333, T 16384 193 -> 168; N 1001, T 4160
-//     131 -> 125; N 3333, T 5024 86 -> 61
+//   nt_adjoint: look-back and ALIF adjoints  N 3333, T 12384 / 20128 / 24768 / 40256 157 -> 140 / 240 ->
+//     210 / 288 -> 289 / 450 -> 502, the stored look-back 218 -> 208 / 330 -> 331 / 404 -> 452 / 643 ->
+//     755; ALIF N 33333, T 480 / 1984 / 4000 89 -> 68 / 298 -> 264 / 593 -> 657: up to 2^26 elements, where
+//     an array fits the cache; the single-pass adjoints also from nt_sweep's neurons on  N 4097, T 992
+//     26 -> 28; N 33333, T 1216 / 1984 / 4000 179 -> 139 / 299 -> 226 / 615 -> 655
+//   nt_warm: warm-started chunks  N 3333, T 5024 86 -> 61, N 2001, T 65536 677 -> 532, but with rows of
+//     whole 32 bytes N 5000, T 8256 149 -> 168, N 1000, T 23712 96 -> 107: plain where N % 8 != 0
+//   replays (rows_aligned alone)  N 1001, T 4160 131 -> 125; N 60001, T 2208 1121 -> 977
 // The sweep's spikes and states and the serial adjoint were never faster with plain stores (N 8191, T
 // 8192 154 -> 178; N 3333, T 5024 140 -> 210) and, like the soft adjoint, the ALIF serial adjoint and the
 // look-back with GU or an undetached reset, store non-temporally at every N.
 // Aligned rows lose with plain stores: N 12800, T 1000 27 -> 32 us, N 65536, T 4096 406 -> 423 us.
-constexpr int64_t kPlainSweep = 8192, kPlainStarts = 16384;
+constexpr int64_t kPlainSweep = 8192, kPlainStarts = 16384, kPlainElements = (int64_t)1 << 26;
 inline bool rows_aligned(int64_t N) { return N % 16 == 0; }
+inline bool nt_sweep(int64_t N) { return rows_aligned(N) || N < kPlainSweep; }
+inline bool nt_starts(int64_t N) { return rows_aligned(N) || N < kPlainStarts; }
+inline bool nt_adjoint(int64_t T, int64_t N) { return rows_aligned(N) || T * N > kPlainElements; }
+inline bool nt_warm(int64_t N) { return N % 8 == 0; }
 // f(std::true_type) for non-temporal stores, f(std::false_type) for plain ones
 template <class F>
-inline void with_store_policy(int64_t N, F&& f, int64_t plain_from = 0) {
-  if (rows_aligned(N) || N < plain_from)
+inline void with_store_policy(bool nt, F&& f) {
+  if (nt)
     f(std::true_type{});
   else
     f(std::false_type{});

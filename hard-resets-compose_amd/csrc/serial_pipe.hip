@@ -424,10 +424,10 @@ void lif_warm_finish_launch(const float* I, float* U, float* S, float* starts, f
 void lif_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, int64_t N, int64_t T,
                          float beta, float theta, float u_r, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  with_store_policy(N, [&](auto nt) {
+  with_store_policy(nt_sweep(N), [&](auto nt) {
     hipLaunchKernelGGL((k_serial_fwd_pipe<LifStep, decltype(nt)::value>), dim3((unsigned)NB),
                        dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, U, S, N, T, LifStep(beta, theta, u_r));
-  }, kPlainSweep);
+  });
 }
 
 void lif_starts_fwd_pipe(const float* I, const float* u0, float* STARTS, float* S, int64_t N, int64_t T,
@@ -440,11 +440,11 @@ void lif_starts_fwd_pipe(const float* I, const float* u0, float* STARTS, float* 
 void aff_serial_fwd_pipe(const float* I, const float* u0, float* U, float* S, int64_t N, int64_t T,
                          float beta, float theta, float gamma, float delta, hipStream_t st) {
   const int NB = (int)((N + WAVE - 1) / WAVE);
-  with_store_policy(N, [&](auto nt) {
+  with_store_policy(nt_sweep(N), [&](auto nt) {
     hipLaunchKernelGGL((k_serial_fwd_pipe<AffStep, decltype(nt)::value>), dim3((unsigned)NB),
                        dim3(WAVE * (PIPE_P + 1)), 0, st, I, u0, U, S, N, T,
                        AffStep{beta, theta, gamma, delta});
-  }, kPlainSweep);
+  });
 }
 
 template <bool DETACH, bool HAS_GU>
