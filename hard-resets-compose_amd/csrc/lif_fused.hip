@@ -45,8 +45,8 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_fwd_fused(const float* __restri
                                                            const float* __restrict__ u0,
                                                            float* __restrict__ U,
                                                            float* __restrict__ S, WsHeader* hdr,
-                                                           int64_t T, int64_t N, int M, int K,
-                                                           float beta, float theta, float u_r) {
+                                                           int64_t N, int M, int K, float beta,
+                                                           float theta, float u_r, int64_t T) {
   static_assert(!RAG || (SO && !SPEC), "a short last chunk: the starts-only forward");
   constexpr int KL = SPEC ? KMAX : 1;
   __shared__ float sA[W][WAVE], sB[W][WAVE];
@@ -231,8 +231,8 @@ template <int C, int W, bool DETACH, bool HAS_GU, int PS = 0, bool RC = false, b
 __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_fused(
     const float* __restrict__ I, const float* __restrict__ u0, const float* __restrict__ U,
     const float* __restrict__ S, const float* __restrict__ GS, const float* __restrict__ GU,
-    float* __restrict__ Lam, double* __restrict__ partials, int64_t T, int64_t N, int M, float beta,
-    float theta, float u_r, float alpha) {
+    float* __restrict__ Lam, double* __restrict__ partials, int64_t N, int M, float beta,
+    float theta, float u_r, float alpha, int64_t T) {
   static_assert(!RAG || RC, "a short last chunk: the recomputing adjoint");
   static_assert(!PS || (DETACH && !HAS_GU && C <= 64), "parameter sums: detached, no GU");
   static_assert(!RC || (DETACH && !HAS_GU && PS != 2), "recompute: hard reset, detached, no GU");
@@ -387,7 +387,7 @@ static void launch_fwd_fused(const float* I, const float* u0, float* U, float* S
   const int64_t T = (int64_t)M * C;
   const auto launch = [&](auto nt) {
     hipLaunchKernelGGL((k_lif_fwd_fused<KMAX, C, W, SPEC, SO, decltype(nt)::value>), dim3((unsigned)NB),
-                       dim3(WAVE * W), 0, st, I, u0, U, S, h, T, N, M, K, beta, theta, u_r);
+                       dim3(WAVE * W), 0, st, I, u0, U, S, h, N, M, K, beta, theta, u_r, T);
   };
   if constexpr (SPEC)
     launch(std::true_type{});
@@ -405,8 +405,8 @@ static void launch_fwd_starts_any(const float* I, const float* u0, float* STARTS
   with_store_policy(nt_starts(N), [&](auto nt) {
     constexpr bool NT = decltype(nt)::value;
     const auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3((unsigned)NB), dim3(WAVE * W), 0, st, I, u0, STARTS, S, h, T, N, M,
-                         1, beta, theta, u_r);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)NB), dim3(WAVE * W), 0, st, I, u0, STARTS, S, h, N, M, 1,
+                         beta, theta, u_r, T);
     };
     T % 32 == 0 ? launch(k_lif_fwd_fused<1, 32, W, false, true, NT>)
                 : launch(k_lif_fwd_fused<1, 32, W, false, true, NT, true>);
@@ -486,7 +486,7 @@ static void launch_bwd_fused(const float* I, const float* u0, const float* U, co
   const auto launch = [&](auto nt) {
     hipLaunchKernelGGL((k_lif_bwd_fused<C, W, DETACH, HAS_GU, 0, false, decltype(nt)::value>),
                        dim3((unsigned)NB), dim3(WAVE * W), 0, st, I, u0, U, S, GS, GU, Lam, nullptr,
-                       (int64_t)M * C, N, M, beta, theta, u_r, alpha);
+                       N, M, beta, theta, u_r, alpha, (int64_t)M * C);
   };
   if constexpr (DETACH && !HAS_GU)
     with_store_policy(nt_sweep(N) || nt_adjoint((int64_t)M * C, N), launch);
@@ -546,7 +546,7 @@ static void launch_bwd_rc(const float* I, const float* STARTS, const float* GS, 
     constexpr bool NT = decltype(nt)::value;
     const auto launch = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)NB), dim3(WAVE * W), 0, st, I, STARTS, STARTS, nullptr,
-                         GS, nullptr, Lam, partials, T, N, M, beta, theta, u_r, alpha);
+                         GS, nullptr, Lam, partials, N, M, beta, theta, u_r, alpha, T);
     };
     if constexpr (C == 32) {  // the layers' chunk takes every T
       if (rag) {
@@ -593,12 +593,12 @@ static void launch_param_fused(const float* I, const float* u0, const float* U, 
     constexpr bool NT = decltype(nt)::value;
     if (ps == 2)
       hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 2, false, NT>), dim3((unsigned)NB),
-                         dim3(WAVE * W), 0, st, I, u0, U, S, GS, nullptr, Lam, partials, (int64_t)M * C, N,
-                         M, beta, theta, u_r, alpha);
+                         dim3(WAVE * W), 0, st, I, u0, U, S, GS, nullptr, Lam, partials, N, M, beta,
+                         theta, u_r, alpha, (int64_t)M * C);
     else
       hipLaunchKernelGGL((k_lif_bwd_fused<C, W, true, false, 1, false, NT>), dim3((unsigned)NB),
-                         dim3(WAVE * W), 0, st, I, u0, U, S, GS, nullptr, Lam, partials, (int64_t)M * C, N,
-                         M, beta, theta, u_r, alpha);
+                         dim3(WAVE * W), 0, st, I, u0, U, S, GS, nullptr, Lam, partials, N, M, beta,
+                         theta, u_r, alpha, (int64_t)M * C);
   });
 }
 

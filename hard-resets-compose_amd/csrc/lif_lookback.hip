@@ -54,7 +54,7 @@ __global__ __launch_bounds__(WAVE* W) void k_lif_bwd_lookback(
     const float* __restrict__ S, const float* __restrict__ GS, const float* __restrict__ GU,
     float* __restrict__ Lam, float* __restrict__ aggP, float* __restrict__ aggQ,
     float* __restrict__ incl, int* __restrict__ flags, WsHeader* hdr, double* __restrict__ partials,
-    int64_t T, int64_t N, int NB, int NSEG, float beta, float theta, float u_r, float alpha) {
+    int64_t N, int NB, int NSEG, float beta, float theta, float u_r, float alpha, int64_t T) {
   static_assert(!PS || (DETACH && !HAS_GU && C <= 64), "parameter sums: detached, no GU");
   static_assert(!RC || (DETACH && !HAS_GU && PS != 2), "recompute: hard reset, detached, no GU");
   constexpr bool AFF = PS == 2;
@@ -259,8 +259,8 @@ static void launch_lookback(const float* I, const float* u0, const float* U, con
                      flags, nflags, 0);
   const auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)nflags), dim3(WAVE * W), 0, st, I, u0, U, S, GS, GU, Lam,
-                       aggP, aggQ, incl, flags, reinterpret_cast<WsHeader*>(ws), partials, T, N, NB,
-                       NSEG, beta, theta, u_r, alpha);
+                       aggP, aggQ, incl, flags, reinterpret_cast<WsHeader*>(ws), partials, N, NB,
+                       NSEG, beta, theta, u_r, alpha, T);
   };
   const auto by_length = [&](auto nt) {
     constexpr bool NT = decltype(nt)::value;
