@@ -108,25 +108,32 @@ Tensor unpacked(const Tensor& t, torch::IntArrayRef sizes, const Tensor& like) {
   return t.contiguous();
 }
 
-// The workspace of the process's most recent look-back adjoint, whose header counts the bounded waits
-// that gave up (hip_lif.last_lookback_timeouts).  Set from the engine's threads; left to the process
-// at its end, when the device may be gone.
-std::mutex& lookback_lock() {
-  static std::mutex m;
-  return m;
+// The workspace of the most recent look-back adjoint run here, whose header counts the bounded waits
+// that gave up (hip_lif.last_lookback_timeouts), and how many have run, by which the Python side
+// tells which of the two ran last.  Set from the engine's threads; left to the process at its end,
+// when the device may be gone.
+struct Lookback {
+  std::mutex lock;
+  Param ws;
+  int64_t runs = 0;
+};
+Lookback& lookback() {
+  static Lookback* l = new Lookback;
+  return *l;
 }
-Param& lookback_ws() {
-  static Param* ws = new Param;
-  return *ws;
-}
-void set_last_lookback(const Tensor& ws) {
+void note_lookback(const Tensor& ws) {
   Param old = ws;  // freed outside the lock
-  const std::lock_guard<std::mutex> lock(lookback_lock());
-  std::swap(lookback_ws(), old);
+  const std::lock_guard<std::mutex> guard(lookback().lock);
+  std::swap(lookback().ws, old);
+  ++lookback().runs;
 }
 Param last_lookback() {
-  const std::lock_guard<std::mutex> lock(lookback_lock());
-  return lookback_ws();
+  const std::lock_guard<std::mutex> guard(lookback().lock);
+  return lookback().ws;
+}
+int64_t lookback_runs() {
+  const std::lock_guard<std::mutex> guard(lookback().lock);
+  return lookback().runs;
 }
 
 // The scaled column sums of the partials (undefined: none) and dL/du0 = beta * Lam[0], in one launch.
@@ -219,7 +226,7 @@ struct LIFLayer : public torch::autograd::Function<LIFLayer> {
                                               stream_of(I)),
               "lsh_lif_scan_lookback_any_bwd");
       }
-      set_last_lookback(ws);
+      note_lookback(ws);
     } else {
       const Tensor ST = unpacked(saved[1], {(T + 31) / 32, N}, gS);
       const size_t nb = g.lsh_lif_layer_bwd_workspace(T, N);
@@ -228,7 +235,7 @@ struct LIFLayer : public torch::autograd::Function<LIFLayer> {
       check(g.lsh_lif_layer_bwd(fp(I), fp(ST), fp(gS), fp(Lam), dp(parts), T, N, beta, theta, u_r,
                                 alpha, raw(ws), nb, stream_of(I)),
             "lsh_lif_layer_bwd");
-      if (nb) set_last_lookback(ws);
+      if (nb) note_lookback(ws);
     }
     const Small s = finish(parts, 1.0, -1.0, beta, Lam, beta, n[0] != 0);
     return grads_of(s, Lam, {n[1], n[2], n[3]}, 12);
@@ -317,7 +324,7 @@ struct AffLayer : public torch::autograd::Function<AffLayer> {
     check(g.lsh_aff_bwd(fp(I), fp(u0), fp(U), fp(S), fp(gS), fp(Lam), dp(parts), T, N, (float)beta,
                         (float)theta, (float)gamma, (float)alpha, code, Cb, raw(ws), nb, stream_of(I)),
           "lsh_aff_bwd");
-    if (nb) set_last_lookback(ws);
+    if (nb) note_lookback(ws);
     const bool sums = n[1] || n[2] || n[3];
     const Small s = finish(sums ? parts : Tensor(), 1.0, beta, beta, Lam, beta, n[0] != 0);
     return grads_of(s, Lam, {n[1], n[2], n[3]}, 12);
@@ -350,7 +357,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("lif_layer", &lif_layer, "hard-reset LIF layer: S");
   m.def("lif_spikes", &lif_spikes, "hard-reset LIF spikes outside autograd");
   m.def("aff_layer", &aff_layer, "affine- or soft-reset LIF layer: S");
-  m.def("set_last_lookback", &set_last_lookback, "workspace of the most recent look-back adjoint");
-  m.def("last_lookback", &last_lookback, "that workspace, or None");
+  m.def("last_lookback", &last_lookback, "workspace of the most recent look-back adjoint here, or None");
+  m.def("lookback_runs", &lookback_runs, "look-back adjoints run here so far");
   m.def("read_scalars", &read_scalars, "values of one-element tensors in one copy");
 }

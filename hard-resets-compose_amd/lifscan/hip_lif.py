@@ -1066,14 +1066,13 @@ def chunked_bwd_C(T, N, C=64):
 
 
 LOOKBACK_SEG = 256  # steps per workgroup segment of the look-back adjoint
-_LAST_LOOKBACK = None  # its most recent workspace, where the C++ module does not keep it
+_LAST_LOOKBACK = (None, -1)  # the Python functions' last workspace, the C++ functions' runs before it
 
 
 def scan_backward_lookback(I, u0, U, S, GS, GU, beta, theta, u_r, alpha=4.0, detach=True, C=16):
     """Single-pass affine-scan adjoint with a decoupled look-back across workgroups -> Lam
     (for few neurons; T % 256 == 0; C in {16, 32} steps per wave)."""
-    I = _input(I)
-    if I.shape[0] % LOOKBACK_SEG:
+    if torch.is_tensor(I) and I.dim() == 2 and I.shape[0] % LOOKBACK_SEG:
         raise ValueError(f"look-back adjoint needs T % {LOOKBACK_SEG} == 0 (T={I.shape[0]})")
     return _lookback(I, u0, U, S, GS, GU, beta, theta, u_r, alpha, detach, C)
 
@@ -1104,18 +1103,23 @@ def _note_lookback(ws):
     """Keep a look-back adjoint's workspace for last_lookback_timeouts, and with CHECK_WAITS raise
     when one of its waits gave up."""
     global _LAST_LOOKBACK
-    if _n.ops() is not None:
-        _n.ops().set_last_lookback(ws)
-    else:
-        _LAST_LOOKBACK = ws
+    ops = _n.ops()
+    _LAST_LOOKBACK = (ws, ops.lookback_runs() if ops is not None else 0)
     if CHECK_WAITS and last_lookback_timeouts() != 0:
         raise RuntimeError("look-back adjoint: a wait gave up; the gradients are not valid")
+
+
+def _last_lookback():
+    """The workspace of the process's most recent look-back adjoint, of either side, or None."""
+    ops = _n.ops()
+    ws, runs = _LAST_LOOKBACK
+    return ops.last_lookback() if ops is not None and ops.lookback_runs() > max(runs, 0) else ws
 
 
 def last_lookback_timeouts():
     """Bounded waits of the process's most recent look-back adjoint that gave up (must be 0), a
     layer's among them; None when none ran.  Synchronizes."""
-    ws = _LAST_LOOKBACK if _n.ops() is None else _n.ops().last_lookback()
+    ws = _last_lookback()
     return None if ws is None else int(_n.read_stats(ws, 1).spin_timeouts)
 
 

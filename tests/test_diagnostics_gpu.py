@@ -33,7 +33,6 @@ def _adjoints():
 
 @pytest.mark.parametrize("name", ["pair", "pair_python", "warm", "warm_python", "affine", "affine_python"])
 def test_last_lookback_is_the_layers(dev, name):
-    from lifscan import _native as n
     from lifscan import hip_lif as L
     T, fn = _adjoints()[name]
     other = torch.zeros(256, dtype=torch.uint8, device=dev)
@@ -43,7 +42,7 @@ def test_last_lookback_is_the_layers(dev, name):
     b = torch.tensor(0.9, device=dev, requires_grad=True)
     print(f"look-back {name}", flush=True)
     fn(I.requires_grad_(True), torch.zeros(70, device=dev), b).sum().backward()
-    assert n.ops().last_lookback().data_ptr() != other.data_ptr()
+    assert L._last_lookback().data_ptr() != other.data_ptr()
     assert L.last_lookback_timeouts() == 0
 
 
