@@ -69,3 +69,31 @@ def test_nan_and_infinite_inputs(dev, T, N, C, W):
     Us, Ss = L.serial_forward(Ig, 0.93, 1.0, 0.0, ug)
     assert torch.equal(S, Ss) and torch.equal(torch.nan_to_num(U, nan=7.0), torch.nan_to_num(Us, nan=7.0))
     assert bool(torch.isnan(U[301:, 1]).all()) and not bool(torch.isnan(U[:301]).any())
+
+
+@pytest.mark.parametrize("kind", ["constant", "noise"])
+def test_graph_replays(dev, kind):
+    """A captured layer call on warm-started chunks, the serial sweep behind the rounds among them: every
+    replay, with eager calls between, gives the eager spikes."""
+    from lifscan import hip_lif as L
+    T, N = 4096, 70
+    assert L._auto_route(T, N, 0.93, False) == (256, 512)
+    x = _current("constant", T, N) if kind == "constant" else None
+    if x is None:
+        x = (0.08 + 0.5 * np.random.default_rng(3).standard_normal((T, N))).astype(np.float32)
+    u0 = uniform(N, 0.0, 1.0, 5)
+    Ig, ug = gpu(x, dev), gpu(u0, dev)
+    So = O.serial_forward(x, 0.93, 1.0, 0.0, u0)[1]
+    with torch.no_grad():
+        assert np.array_equal(host(L.lif_auto(Ig, ug, 0.93)), So)
+        print(f"warm graph {kind}", flush=True)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            S = L.lif_auto(Ig, ug, 0.93)
+        for _ in range(3):
+            S.fill_(-1.0)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(host(S), So)
+            assert np.array_equal(host(L.lif_auto(Ig, ug, 0.93)), So)
